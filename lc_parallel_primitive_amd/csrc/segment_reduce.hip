@@ -9,10 +9,11 @@
 // value) pairs over the whole input, then index - begin per segment).
 //
 // MI355X design, one launch, no temp storage, segment-length adaptive:
-//  * A workgroup (4 waves) owns 256 consecutive segments, 64 per wave; lanes
-//    0..63 of a wave load the bounds of its segments with one coalesced load
-//    (or compute them, for fixed-size segments).
-//  * Contiguous flat path: a wave whose 64 segments are sorted and disjoint
+//  * A workgroup (4 waves) owns up to 256 consecutive segments, 64 per wave,
+//    fewer where there are few segments (seg_split); the lanes of a wave load
+//    the bounds of its segments with one coalesced load (or compute them, for
+//    fixed-size segments).
+//  * Contiguous flat path: a wave whose segments are sorted and disjoint
 //    (begin[s + 1] >= end[s]: CSR offsets that tile a range, or ranges with
 //    gaps that hold fewer elements than the segments), none of them long,
 //    streams the range from its first begin to its last end in 4 KiB chunks
@@ -29,8 +30,8 @@
 //    2 GiB or more (one buffer resource covers less) folds one segment at a
 //    time instead.
 //  * Segments longer than kSegLong: their indices are compacted into LDS and
-//    the whole workgroup streams each one (4 loads in flight per thread)
-//    after its waves are done.  Fixed-size segments longer than kSegLong
+//    the whole workgroup streams each one (8 16-byte loads in flight per
+//    thread) after its waves are done.  Fixed-size segments longer than kSegLong
 //    take a workgroup-per-segment launch directly.
 //  * Sum/Min/Max write op(init, fold) (init defaults to the operator's
 //    identity; Min starts from max(), Max from lowest()); an empty segment
@@ -67,8 +68,9 @@ constexpr int kSegWaves = kSegBlock / kWave;
 // scalar walk over the chunk's ends 131 / 135 / 173, with the end bitmap
 // and mbcnt 124 / 124 / 145, with the ordered combine 123 / 125 / 136
 // (gathering the tiling layout: 104; with no segment lookup at all 96).
-constexpr int kSegPerWave = 64;
+constexpr int kSegPerWave = 64;  // at most (seg_split)
 constexpr uint32_t kSegLong = 8192;
+constexpr uint32_t kSegLongAlone = 2048;  // with one segment per workgroup
 constexpr uint32_t kNoIndex = 0xFFFFFFFFu;
 
 enum SegOpKind { kSegSum = 0, kSegMin = 1, kSegMax = 2, kSegArgMin = 3, kSegArgMax = 4 };
@@ -191,8 +193,13 @@ __device__ __forceinline__ void seg_store(typename SegAcc<T, OP>::A acc, uint32_
     }
 }
 
-// The whole workgroup streams segment s (4 loads in flight per thread) and
-// thread 0 stores its result.  Every thread must call it (barriers).
+// The whole workgroup streams segment s and thread 0 stores its result: 16-byte
+// loads from the segment's first aligned element on, kWgLoads of them in
+// flight per thread (32 KiB per workgroup), the ragged ends element by
+// element.  One CU reads a segment, so what bounds it is the bytes in flight:
+// 2^26 f32 in segments of 30000 take 39.7 us (6.8 TB/s; 43.1 with four 4-byte
+// loads in flight).  Every thread must call it (barriers).
+constexpr int kWgLoads = 8;
 template <class T, int OP, bool FIXED>
 __device__ __forceinline__ void wg_reduce_segment(const T *__restrict__ in, T *__restrict__ out,
                                                   uint32_t *__restrict__ index_out, uint64_t s, uint64_t S,
@@ -201,21 +208,52 @@ __device__ __forceinline__ void wg_reduce_segment(const T *__restrict__ in, T *_
 {
     using Acc = SegAcc<T, OP>;
     using A = typename Acc::A;
+    constexpr uint32_t V = 16 / sizeof(T);
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
     uint32_t lb, llen;
     seg_bounds<FIXED>(sb, s, S, lb, llen);
-    const uint64_t le = (uint64_t)lb + llen;
-    A a0 = Acc::identity(), a1 = a0, a2 = a0, a3 = a0;
-    uint64_t i = (uint64_t)lb + tid;
-    for (; i + 3 * kSegBlock < le; i += 4 * kSegBlock) {
-        const T x0 = in[i], x1 = in[i + kSegBlock], x2 = in[i + 2 * kSegBlock], x3 = in[i + 3 * kSegBlock];
-        a0 = Acc::fold(a0, x0, (uint32_t)i);
-        a1 = Acc::fold(a1, x1, (uint32_t)(i + kSegBlock));
-        a2 = Acc::fold(a2, x2, (uint32_t)(i + 2 * kSegBlock));
-        a3 = Acc::fold(a3, x3, (uint32_t)(i + 3 * kSegBlock));
+    const T *p = in + lb;
+    // elements before the first 16-byte boundary (the input pointer itself is
+    // aligned to its type only), whole vectors, the rest
+    const uint32_t ahead = (uint32_t)((16 - (reinterpret_cast<uintptr_t>(p) & 15)) & 15) / (uint32_t)sizeof(T);
+    const uint32_t head = ahead < llen ? ahead : llen;
+    const uint32_t nv = (llen - head) / V;
+    A a0 = Acc::identity(), a1 = a0;
+    if (tid < head) a0 = Acc::fold(a0, p[tid], lb + tid);
+    auto fold_vec = [&](u32x4 w, uint32_t i) {
+        T e[V];
+        unpack16<T>(w, e);
+#pragma unroll
+        for (uint32_t j = 0; j < V; ++j) {
+            A &a = j & 1u ? a1 : a0;
+            a = Acc::fold(a, e[j], lb + head + i * V + j);
+        }
+    };
+    const T *pv = p + head;
+    uint32_t i = tid;
+    for (; i < nv && nv - i > (kWgLoads - 1) * kSegBlock; i += kWgLoads * kSegBlock) {
+        u32x4 w[kWgLoads];
+#pragma unroll
+        for (int q = 0; q < kWgLoads; ++q) w[q] = ld16_nt(pv + (uint64_t)(i + q * kSegBlock) * V);
+#pragma unroll
+        for (int q = 0; q < kWgLoads; ++q) fold_vec(w[q], i + q * kSegBlock);
     }
-    for (; i < le; i += kSegBlock) a0 = Acc::fold(a0, in[i], (uint32_t)i);
-    A a = Acc::combine(Acc::combine(a0, a1), Acc::combine(a2, a3));
+    // the rest, half as many at a time: a load past the end reads the last
+    // vector again and is not folded
+    for (; i < nv; i += kWgLoads / 2 * kSegBlock) {
+        u32x4 w[kWgLoads / 2];
+#pragma unroll
+        for (int q = 0; q < kWgLoads / 2; ++q) {
+            const uint32_t v = i + q * kSegBlock;
+            w[q] = ld16_nt(pv + (uint64_t)(v < nv ? v : nv - 1) * V);
+        }
+#pragma unroll
+        for (int q = 0; q < kWgLoads / 2; ++q)
+            if (i + q * kSegBlock < nv) fold_vec(w[q], i + q * kSegBlock);
+    }
+    const uint32_t t = head + nv * V + tid;  // fewer than V elements are left
+    if (tid < V && t < llen) a1 = Acc::fold(a1, p[t], lb + t);
+    A a = Acc::combine(a0, a1);
     a = Acc::wave_reduce(a);
     if (lane == 0) s_wave[wave] = a;
     __syncthreads();
@@ -312,12 +350,12 @@ __device__ __forceinline__ void flat_range(uint32_t nvalid, uint32_t b, uint32_t
 // none long, gaps holding at most as many elements as the segments plus one
 // chunk, and a range end below kFlatMaxEnd.  Wave-uniform.
 template <class T>
-__device__ __forceinline__ bool flat_eligible(uint32_t nvalid, uint32_t b, uint32_t len)
+__device__ __forceinline__ bool flat_eligible(uint32_t nvalid, uint32_t b, uint32_t len, uint32_t long_len)
 {
     constexpr uint32_t CH = kWave * flat_epl<T>();
     const uint32_t lane = lane_id();
     const uint32_t b_next = (uint32_t)__shfl_down((int)b, 1);
-    const bool breaks = lane < nvalid && (len > kSegLong || (lane + 1 < nvalid && b + len > b_next));
+    const bool breaks = lane < nvalid && (len > long_len || (lane + 1 < nvalid && b + len > b_next));
     if (nvalid == 0 || ballot(breaks) != 0) return false;
     uint32_t B, E;
     flat_range(nvalid, b, len, B, E);
@@ -561,7 +599,7 @@ __device__ __forceinline__ void flat_segments(const T *__restrict__ in, T *__res
 template <class T, int OP>
 __device__ __forceinline__ void wave_segments(const T *__restrict__ in, T *__restrict__ out,
                                               uint32_t *__restrict__ index_out, T init, uint64_t wseg0,
-                                              uint32_t nvalid, uint32_t b, uint32_t len)
+                                              uint32_t nvalid, uint32_t b, uint32_t len, uint32_t long_len)
 {
     using Acc = SegAcc<T, OP>;
     using A = typename Acc::A;
@@ -570,7 +608,7 @@ __device__ __forceinline__ void wave_segments(const T *__restrict__ in, T *__res
     for (uint32_t s = 0; s < nvalid; ++s) {
         const uint32_t bs = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)s);
         const uint32_t ls = (uint32_t)__builtin_amdgcn_readlane((int)len, (int)s);
-        if (ls > kSegLong) continue;
+        if (ls > long_len) continue;
         A acc = Acc::identity();
 #pragma unroll 1
         for (uint32_t i = lane; i < ls; i += kWave) acc = Acc::fold(acc, in[(uint64_t)bs + i], bs + i);
@@ -587,30 +625,33 @@ __device__ __forceinline__ void wave_segments(const T *__restrict__ in, T *__res
 template <class T, int OP, bool FIXED>
 __global__ __launch_bounds__(kSegBlock) __attribute__((amdgpu_waves_per_eu(6))) void segment_reduce_kernel(const T *__restrict__ in, T *__restrict__ out,
                                                                    uint32_t *__restrict__ index_out, uint64_t S,
-                                                                   SegBounds sb, T init, int vec_ok)
+                                                                   SegBounds sb, T init, int vec_ok, uint32_t per_wg,
+                                                                   uint32_t spw, uint32_t long_len)
 {
     using Acc = SegAcc<T, OP>;
     using A = typename Acc::A;
-    constexpr int kBatch = kSegWaves * kSegPerWave;
-    __shared__ uint32_t s_long[kBatch];
+    __shared__ uint32_t s_long[kSegWaves * kSegPerWave];
     __shared__ uint32_t s_nlong;
     __shared__ A s_wave[kSegWaves];
     __shared__ FlatSmem<T> s_flat;
 
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
-    const uint64_t wseg0 = (uint64_t)blockIdx.x * kBatch + (uint64_t)wave * kSegPerWave;
-    // lanes 0..kSegPerWave-1 hold the bounds of the wave's segments (one coalesced load)
+    const uint64_t wg_seg0 = (uint64_t)blockIdx.x * per_wg;
+    const uint64_t wseg0 = wg_seg0 + (uint64_t)wave * spw;
+    // lanes 0..spw-1 hold the bounds of the wave's segments (one coalesced
+    // load); with one segment per workgroup it is wave 0's
+    const bool owner = wave * spw < per_wg;
     uint32_t b = 0, len = 0;
-    if (lane < (uint32_t)kSegPerWave) seg_bounds<FIXED>(sb, wseg0 + lane, S, b, len);
+    if (owner && lane < spw) seg_bounds<FIXED>(sb, wseg0 + lane, S, b, len);
     if (tid == 0) s_nlong = 0;
     __syncthreads();
-    const bool is_long = len > kSegLong;
-    if (is_long) s_long[atomicAdd(&s_nlong, 1u)] = (uint32_t)(wave * kSegPerWave + lane);
+    const bool is_long = len > long_len;
+    if (is_long) s_long[atomicAdd(&s_nlong, 1u)] = wave * spw + lane;
 
     // contiguous flat path when the wave's segments are sorted, disjoint and
     // none is long; else the gather form over the concatenated segments
-    const uint32_t nvalid = wseg0 < S ? (uint32_t)(S - wseg0 < kSegPerWave ? S - wseg0 : kSegPerWave) : 0u;
-    if (vec_ok && flat_eligible<T>(nvalid, b, len)) {
+    const uint32_t nvalid = owner && wseg0 < S ? (uint32_t)(S - wseg0 < spw ? S - wseg0 : spw) : 0u;
+    if (vec_ok && flat_eligible<T>(nvalid, b, len, long_len)) {
         flat_segments<T, OP, false>(in, out, index_out, init, wseg0, nvalid, b, len, true, 0u, 0u, 0u,
                                     s_flat.bnd[wave], s_flat.seg_of[wave], s_flat.bbits[wave], s_flat.ebits[wave],
                                     s_flat.stage[wave], s_flat.gbits[wave], s_flat.gdelta[wave]);
@@ -629,7 +670,7 @@ __global__ __launch_bounds__(kSegBlock) __attribute__((amdgpu_waves_per_eu(6))) 
                                        s_flat.ebits[wave], s_flat.stage[wave], s_flat.gbits[wave],
                                        s_flat.gdelta[wave]);
         } else {
-            wave_segments<T, OP>(in, out, index_out, init, wseg0, nvalid, b, len);
+            wave_segments<T, OP>(in, out, index_out, init, wseg0, nvalid, b, len, long_len);
         }
     }
 
@@ -637,8 +678,7 @@ __global__ __launch_bounds__(kSegBlock) __attribute__((amdgpu_waves_per_eu(6))) 
     __syncthreads();
     const uint32_t nlong = s_nlong;
     for (uint32_t q = 0; q < nlong; ++q)
-        wg_reduce_segment<T, OP, FIXED>(in, out, index_out, (uint64_t)blockIdx.x * kBatch + s_long[q], S, sb, init,
-                                        s_wave);
+        wg_reduce_segment<T, OP, FIXED>(in, out, index_out, wg_seg0 + s_long[q], S, sb, init, s_wave);
 }
 
 // Fixed-size segments longer than kSegLong: one workgroup per segment.
@@ -666,6 +706,35 @@ int resident_blocks(K kernel, DeviceCache &cache)
     });
 }
 
+// How S segments are dealt out: segments per workgroup and per wave, and the
+// length from which the whole workgroup takes a segment.  A wave reads its
+// segments one 4 KiB chunk after the other, so what bounds a call with few
+// segments is how many waves they are spread over, whatever their lengths
+// (64 per wave at every S: 4096 segments of 1000 f32, ArgMax, kept 64 waves
+// busy for 73 us; 1024 segments of mean 16000 took 1340 us, one workgroup
+// reading up to 256 long ones in turn).  Measured, us per call (f32 Sum unless
+// named; lines in S, 256 CUs):
+//  * S < 4096, one segment per workgroup, the workgroup taking those over
+//    2048 elements: mean 16000, S = 1048: 20 (one per wave: 36); size 5000
+//    ArgMax, S = 3355: 17 (one per wave: 24).
+//  * from there one segment per wave for every 8192 segments, up to 8: mean
+//    1024, S = 16384: 15 (4 per wave: 29); size 1000 ArgMax, S = 67108: 45
+//    (64 per wave: 94); skewed, mean 4096, S = 16384: 56 (4 per wave: 90).
+//  * from 131072 on 32, from 262144 on 64: mean 128, S = 131072: 13.2 with
+//    32, 14.6 with 16; mean 37, S = 453438: 12.9 with 64, 14.4 with 32.
+struct SegSplit {
+    uint32_t per_wg, per_wave, long_len;
+};
+SegSplit seg_split(uint64_t S)
+{
+    const uint64_t cus = (uint64_t)device_cus();
+    if (S < 16 * cus) return {1, 1, kSegLongAlone};
+    uint32_t per_wave = 1;
+    while (per_wave < 8 && S >= 2 * per_wave * cus * 32) per_wave *= 2;
+    if (S >= 512 * cus) per_wave = S >= 1024 * cus ? kSegPerWave : kSegPerWave / 2;
+    return {kSegWaves * per_wave, per_wave, kSegLong};
+}
+
 template <class T, int OP, bool FIXED>
 int segment_launch(const void *in_, void *out_, uint32_t *index_out, uint64_t S, SegBounds sb, const void *init_,
                    hipStream_t s)
@@ -676,7 +745,7 @@ int segment_launch(const void *in_, void *out_, uint32_t *index_out, uint64_t S,
     if (!out || (OP >= kSegArgMin && !index_out)) return LCPP_ERR_INVALID_ARG;
     if (!FIXED && (!sb.begin || !sb.end || !in)) return LCPP_ERR_INVALID_ARG;
     if (FIXED && sb.size && !in) return LCPP_ERR_INVALID_ARG;
-    if (S > 0xFFFFFFFFull || ceil_div(S, (uint64_t)kSegWaves * kSegPerWave) > 0x7FFFFFFFull) return LCPP_ERR_INVALID_ARG;
+    if (S > 0xFFFFFFFFull) return LCPP_ERR_INVALID_ARG;
     if (FIXED && (uint64_t)sb.size * S > 0xFFFFFFFFull) return LCPP_ERR_INVALID_ARG;  // 32-bit element offsets
     T init = SegAcc<T, OP >= kSegArgMin ? kSegSum : OP>::identity();
     if constexpr (OP < kSegArgMin) {
@@ -691,11 +760,13 @@ int segment_launch(const void *in_, void *out_, uint32_t *index_out, uint64_t S,
         LCPP_CHECK_LAUNCH();
         return LCPP_OK;
     }
-    const uint64_t blocks = ceil_div(S, (uint64_t)kSegWaves * kSegPerWave);
-    const uint32_t grid = (uint32_t)blocks;
+    const SegSplit split = seg_split(S);
+    const uint32_t grid = (uint32_t)ceil_div(S, (uint64_t)split.per_wg);
     const int vec_ok = (reinterpret_cast<uintptr_t>(in) & 15) == 0;
     LCPP_LAUNCH("segment_reduce", s,
-                (segment_reduce_kernel<T, OP, FIXED><<<grid, kSegBlock, 0, s>>>(in, out, index_out, S, sb, init, vec_ok)));
+                (segment_reduce_kernel<T, OP, FIXED><<<grid, kSegBlock, 0, s>>>(in, out, index_out, S, sb, init, vec_ok,
+                                                                            split.per_wg, split.per_wave,
+                                                                            split.long_len)));
     LCPP_CHECK_LAUNCH();
     return LCPP_OK;
 }

@@ -635,3 +635,33 @@ def test_mixed_layouts_random(gpu, seed):
         v, i = seg_call(method, d, S, (b, e), dtype, arg=True)
         ev, ei = o.segment_reduce_arg(is_max, a, b, e)
         assert same(v, ev) and (i == ei).all(), method
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.float32, np.float64])
+@pytest.mark.parametrize("S", [4095, 4096, 16383, 16384, 32768, 65536, 131071, 131072, 262144])
+def test_segment_counts_where_the_split_changes(gpu, S, dtype):
+    """The segments per wave and per workgroup follow S: layouts around every line of that rule, with empty
+    segments, segments over both long-segment lengths that start at any alignment, and a shuffled order."""
+    import gpu_util as g
+
+    rng = np.random.default_rng(S)
+    L = rng.integers(0, 40, S).astype(np.int64)
+    at = rng.choice(S, 24, replace=False)
+    L[at] = np.array([2047, 2048, 2049, 2050, 2051, 4099, 8191, 8192, 8193, 8195, 9001, 20011] * 2)
+    e = np.cumsum(L)
+    n = int(e[-1])
+    b, e = (e - L).astype(np.uint32), e.astype(np.uint32)
+    order = rng.permutation(S)
+    a = g.random_array(dtype, n, seed=S)
+    for lb, le in ((b, e), (b[order], e[order])):
+        for pad in (0, 1):
+            d = g.to_dev(a, pad)
+            got = seg_call("Sum", d, S, (lb, le), dtype)
+            if np.dtype(dtype).kind == "i":
+                assert same(got, o.segment_reduce(o.OP_SUM, a, lb, le))
+            else:
+                s, ab = o.segment_reduce_f64(a, lb, le)
+                assert (np.abs(got.astype(np.float64) - s) <= RTOL_SEG * ab + 1e-30).all()
+            v, i = seg_call("ArgMax", d, S, (lb, le), dtype, arg=True)
+            ev, ei = o.segment_reduce_arg(True, a, lb, le)
+            assert same(v, ev) and (i == ei).all()
