@@ -76,7 +76,7 @@
 //    values it never uses, device_radix_sort.h:118-122).
 #include <mutex>
 
-#include "common.hpp"
+#include "small_sort.hpp"
 
 namespace lcpp {
 namespace {
@@ -1005,6 +1005,9 @@ int rs_run(void *temp, size_t temp_bytes, const void *kin_, void *kout_, const v
     UK *ktmp = reinterpret_cast<UK *>(t + L.ktmp_off);
     UV *vtmp = reinterpret_cast<UV *>(t + L.vtmp_off);
     const int P = (int)L.passes;
+    if (n <= small_sort_max(sizeof(UK)))
+        return small_sort_launch(sizeof(UK), KIND, DESC, rs_rank_path(s) == kRankMatch, kin, kout,
+                                 PAIRS ? vin : nullptr, vout, sizeof(UV), (uint32_t)n, status, s);
 
     // status header, bins, hot digits, plan and the arrival counter are contiguous
     const uint32_t init_words = (uint32_t)((L.hot_off + (2 * L.passes + 1) * 4) / 4);
