@@ -17,7 +17,12 @@
 //    are gathered once, after the last pass.
 //  * Key types differ in what is XORed in and out, so the kernel takes the
 //    masks as arguments and is compiled per key size only.
-// What bounds it is one CU's LDS: about 26 cycles of it per 64 keys and pass.
+// What bounds it is one CU's LDS and VALU: a full pass of 16384 u32 keys takes
+// about 4 us, with a payload 6 us.  Measured (us per call, onesweep pipeline
+// -> here): SortKeys u32 of 1023 keys 96 -> 8.6, 8192: 88 -> 11.8, 16384: 59 ->
+// 19.2; SortKeys u64 of 8192: 87 -> 25.4; SortPairs u32 -> u32 of 16384: 52 ->
+// 29.5 (31.8 with the key and its source position as two LDS words and a
+// branch around each counter update).
 #include "small_sort.hpp"
 
 namespace lcpp {
@@ -29,8 +34,8 @@ constexpr int kSsRadix = 256;
 
 // Raw key -> sort key and back: in(k) = k ^ (negative ? neg : pos) ^ flip
 // (the twiddles of common/util_type.h:98-175; flip inverts for descending
-// order).  `mz` (the sort key of -0.0) ranks as `pz` (+0.0); both are 0 for
-// keys that are not floating.
+// order).  ZEROS (floating keys): `mz`, the sort key of -0.0, ranks as `pz`,
+// that of +0.0.
 template <class UK>
 struct KeyCode {
     UK neg, pos, flip, mz, pz;
@@ -41,20 +46,21 @@ struct KeyCode {
         const UK u = t ^ flip;
         return u ^ ((u & kHigh) ? pos : neg);
     }
-    __device__ __forceinline__ UK ranked(UK t) const { return t == mz ? pz : t; }
 };
 
+// A 4-byte key travels with its source position in one 8-byte LDS word.
 template <int IPT, class UK, bool PAIRS>
 struct SsSmem {
     static constexpr int N = kSsBlock * IPT;
-    UK keys[N];
-    uint16_t src[PAIRS ? N : 2];
+    static constexpr bool kSplit = PAIRS && sizeof(UK) == 8;
+    std::conditional_t<PAIRS, uint64_t, UK> item[N];
+    uint16_t src[kSplit ? N : 2];
     uint32_t cnt[kSsWaves][kSsRadix];
     uint32_t wsum[kSsRadix / kWave];
     uint32_t diff[kSsWaves][sizeof(UK) / 4];
 };
 
-template <int IPT, class UK, bool PAIRS, bool MATCH>
+template <int IPT, class UK, bool PAIRS, bool ZEROS, bool MATCH>
 __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK *kout, const void *vin, void *vout,
                                                               int val_bytes, uint32_t n, KeyCode<UK> code,
                                                               uint32_t *status)
@@ -65,9 +71,12 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
     const uint32_t p0 = wave * (kWave * IPT) + lane;  // position of item 0; item u: + u * 64
     if (tid == 0) *status = 0;
 
+    auto ranked = [&](UK t) { return ZEROS && t == code.mz ? code.pz : t; };
+    auto digit = [&](UK t, uint32_t sh) { return (uint32_t)(ranked(t) >> sh) & 255u; };
+
     UK tk[IPT];
     uint32_t src[PAIRS ? IPT : 1];
-    const UK first = code.ranked(code.in(kin[0]));
+    const UK first = ranked(code.in(kin[0]));
     UK diff = 0;
 #pragma unroll
     for (int u = 0; u < IPT; ++u) {
@@ -77,7 +86,7 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
     }
 #pragma unroll
     for (int u = 0; u < IPT; ++u)
-        if (p0 + u * kWave < n) diff |= code.ranked(tk[u]) ^ first;
+        if (p0 + u * kWave < n) diff |= ranked(tk[u]) ^ first;
     auto or_op = [](uint32_t a, uint32_t b) { return a | b; };
 #pragma unroll
     for (int h = 0; h < (int)sizeof(UK) / 4; ++h) {
@@ -101,9 +110,9 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
         if (busy) {
 #pragma unroll
             for (int u = 0; u < IPT; ++u) {
+                // (no branch: positions past n add 0 to a counter per lane)
                 const bool ok = p0 + u * kWave < n;
-                const uint32_t d = (uint32_t)(code.ranked(tk[u]) >> shift) & 255u;
-                rank[u] = 0;
+                const uint32_t d = digit(tk[u], shift);
                 if constexpr (MATCH) {
                     const uint64_t peers = match_any8(d) & ballot(ok);
                     const uint32_t below = mask_rank(peers);
@@ -111,7 +120,7 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
                     if (ok && below == 0) b = atomicAdd(&cnt[d], (uint32_t)__builtin_popcountll(peers));
                     rank[u] = (uint32_t)__shfl((int)b, ok ? (int)__builtin_ctzll(peers) : 0) + below;
                 } else {
-                    if (ok) rank[u] = atomicAdd(&cnt[d], 1u);
+                    rank[u] = atomicAdd(&cnt[ok ? d : lane], ok ? 1u : 0u);
                 }
             }
         }
@@ -143,20 +152,28 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
         __syncthreads();
         if (busy) {
 #pragma unroll
-            for (int u = 0; u < IPT; ++u) {
+            for (int u = 0; u < IPT; ++u) rank[u] += cnt[digit(tk[u], shift)];
+#pragma unroll
+            for (int u = 0; u < IPT; ++u)
                 if (p0 + u * kWave < n) {
-                    const uint32_t r = rank[u] + cnt[(uint32_t)(code.ranked(tk[u]) >> shift) & 255u];
-                    sm.keys[r] = tk[u];
-                    if constexpr (PAIRS) sm.src[r] = (uint16_t)src[u];
+                    if constexpr (!PAIRS) sm.item[rank[u]] = tk[u];
+                    else if constexpr (sizeof(UK) == 4) sm.item[rank[u]] = (uint64_t)src[u] << 32 | tk[u];
+                    else {
+                        sm.item[rank[u]] = tk[u];
+                        sm.src[rank[u]] = (uint16_t)src[u];
+                    }
                 }
-            }
         }
         __syncthreads();
         // (reads past n give stale words that nothing uses)
 #pragma unroll
         for (int u = 0; u < IPT; ++u) {
-            tk[u] = sm.keys[p0 + u * kWave];
-            if constexpr (PAIRS) src[u] = sm.src[p0 + u * kWave];
+            const auto w = sm.item[p0 + u * kWave];
+            tk[u] = (UK)w;
+            if constexpr (PAIRS) {
+                if constexpr (sizeof(UK) == 4) src[u] = (uint32_t)(w >> 32);
+                else src[u] = sm.src[p0 + u * kWave];
+            }
         }
         for (uint32_t i = tid; i < (uint32_t)(kSsWaves * kSsRadix); i += kSsBlock) (&sm.cnt[0][0])[i] = 0;
         __syncthreads();
@@ -189,7 +206,7 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
         if (p0 + u * kWave < n) kout[p0 + u * kWave] = code.out(tk[u]);
 }
 
-template <int IPT, class UK, bool PAIRS, bool MATCH>
+template <int IPT, class UK, bool PAIRS, bool ZEROS, bool MATCH>
 int ss_run(const KeyCode<UK> &code, const void *kin, void *kout, const void *vin, void *vout, int val_bytes,
            uint32_t n, uint32_t *status, hipStream_t s)
 {
@@ -198,7 +215,7 @@ int ss_run(const KeyCode<UK> &code, const void *kin, void *kout, const void *vin
     if (lds > 64 * 1024) {
         static DeviceCache lds_set;
         if (device_cached(lds_set, [] {
-                return hipFuncSetAttribute(reinterpret_cast<const void *>(&small_sort_kernel<IPT, UK, PAIRS, MATCH>),
+                return hipFuncSetAttribute(reinterpret_cast<const void *>(&small_sort_kernel<IPT, UK, PAIRS, ZEROS, MATCH>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess
                            ? 1
                            : -1;
@@ -206,20 +223,20 @@ int ss_run(const KeyCode<UK> &code, const void *kin, void *kout, const void *vin
             return LCPP_ERR_HIP;
     }
     LCPP_LAUNCH("rs_small", s,
-                (small_sort_kernel<IPT, UK, PAIRS, MATCH><<<1, kSsBlock, lds, s>>>(
+                (small_sort_kernel<IPT, UK, PAIRS, ZEROS, MATCH><<<1, kSsBlock, lds, s>>>(
                     static_cast<const UK *>(kin), static_cast<UK *>(kout), vin, vout, val_bytes, n, code, status)));
     LCPP_CHECK_LAUNCH();
     return LCPP_OK;
 }
 
-template <class UK, bool PAIRS, bool MATCH>
+template <class UK, bool PAIRS, bool ZEROS, bool MATCH>
 int ss_size(const KeyCode<UK> &code, const void *kin, void *kout, const void *vin, void *vout, int vb, uint32_t n,
             uint32_t *status, hipStream_t s)
 {
     // items per thread: the fewest that hold n
-    if (n <= 2 * kSsBlock) return ss_run<2, UK, PAIRS, MATCH>(code, kin, kout, vin, vout, vb, n, status, s);
-    if (n <= 8 * kSsBlock) return ss_run<8, UK, PAIRS, MATCH>(code, kin, kout, vin, vout, vb, n, status, s);
-    if constexpr (sizeof(UK) == 4) return ss_run<16, UK, PAIRS, MATCH>(code, kin, kout, vin, vout, vb, n, status, s);
+    if (n <= 2 * kSsBlock) return ss_run<2, UK, PAIRS, ZEROS, MATCH>(code, kin, kout, vin, vout, vb, n, status, s);
+    if (n <= 8 * kSsBlock) return ss_run<8, UK, PAIRS, ZEROS, MATCH>(code, kin, kout, vin, vout, vb, n, status, s);
+    if constexpr (sizeof(UK) == 4) return ss_run<16, UK, PAIRS, ZEROS, MATCH>(code, kin, kout, vin, vout, vb, n, status, s);
     return LCPP_ERR_INVALID_ARG;
 }
 
@@ -236,11 +253,14 @@ int ss_key(int kind, bool desc, bool match, const void *kin, void *kout, const v
         c.mz = UK(~high) ^ c.flip;
         c.pz = high ^ c.flip;
     }
-    if (vin)
-        return match ? ss_size<UK, true, true>(c, kin, kout, vin, vout, vb, n, status, s)
-                     : ss_size<UK, true, false>(c, kin, kout, vin, vout, vb, n, status, s);
-    return match ? ss_size<UK, false, true>(c, kin, kout, vin, vout, vb, n, status, s)
-                 : ss_size<UK, false, false>(c, kin, kout, vin, vout, vb, n, status, s);
+    auto go = [&](auto pairs, auto zeros) {
+        return match ? ss_size<UK, decltype(pairs)::value, decltype(zeros)::value, true>(c, kin, kout, vin, vout, vb, n,
+                                                                                         status, s)
+                     : ss_size<UK, decltype(pairs)::value, decltype(zeros)::value, false>(c, kin, kout, vin, vout, vb,
+                                                                                          n, status, s);
+    };
+    if (kind == 2) return vin ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
+    return vin ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
 }
 
 }  // namespace
