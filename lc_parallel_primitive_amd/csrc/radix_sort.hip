@@ -74,6 +74,7 @@
 //    does; equal keys keep their input order.
 //  * Keys-only sorts reserve no value scratch (the reference reserves N
 //    values it never uses, device_radix_sort.h:118-122).
+#include <algorithm>
 #include <mutex>
 
 #include "small_sort.hpp"
@@ -93,8 +94,6 @@ constexpr uint32_t kLbGlobal = 0x80000000u;
 constexpr uint32_t kTcPublished = 0x8000u;
 constexpr uint32_t kTcMask = 0x7FFFu;
 constexpr uint64_t kMaxItems = 0xFFFFFFFFull;  // 32-bit positions and counts
-
-enum KeyKind { kUnsigned = 0, kSigned = 1, kFloat = 2 };
 
 // Twiddles of common/util_type.h:98-175 (BaseTraits::TwiddleIn/Out).
 template <class UK, int KIND>
@@ -141,6 +140,17 @@ __device__ __forceinline__ uint32_t digit_of(UK tk, uint32_t shift)
     }
     return (uint32_t)(tk >> shift) & (kRadix - 1);
 }
+
+// How a kernel turns raw keys into sort keys and digits: the key type and
+// order compiled in (StaticCode: the large sorts) or as masks (KeyCode,
+// small_sort.hpp: the others).
+template <class UK_, int KIND, bool DESC>
+struct StaticCode {
+    using UK = UK_;
+    __device__ __forceinline__ UK in(UK raw) const { return sort_key<UK, KIND, DESC>(raw); }
+    __device__ __forceinline__ UK out(UK sk) const { return raw_key<UK, KIND, DESC>(sk); }
+    __device__ __forceinline__ uint32_t digit(UK tk, uint32_t shift) const { return digit_of<UK, KIND, DESC>(tk, shift); }
+};
 
 // Exclusive scan of the values x held by threads 0..255 (one digit each) of
 // the workgroup; other threads pass 0 and get garbage.  Every thread of the
@@ -285,35 +295,40 @@ __device__ void rs_make_plan(const uint32_t *bins, uint32_t passes, uint64_t n, 
 //    byte): SortPairs C4 (six constant key bytes) 1.694 -> 1.677 ms,
 //    full-range keys 5.816 -> 5.825 ms.
 // A column counts at most 1/COLS of the keys a workgroup has seen since its
-// last flush, so the table is flushed every kHistRoundSteps loop steps
+// last flush, so the table is flushed every hist_round_steps loop steps
 // (4-byte keys: 4,177,920 keys < 64 x 65536; 8-byte: 2,088,960 < 32 x 65536).
 template <class UK>
 constexpr uint32_t hist_cols()
 {
     return sizeof(UK) == 4 ? 64u : 32u;
 }
+// Sorts of smaller tiles: a workgroup counts 4096 keys only, and clearing and
+// summing the full table would cost more than that (100003 u32 keys: 8.0 us;
+// 64 columns and 16384 keys per workgroup: 11.6).
+constexpr uint32_t kHistColsMid = 8;
 // Dynamic LDS: the counter table, then 17 words of planning state for the
 // last workgroup (the kernel has no static LDS).
 template <class UK>
-constexpr size_t hist_table_words()
+constexpr size_t hist_table_words(uint32_t cols)
 {
-    return sizeof(UK) * (kRadix / 2) * hist_cols<UK>();
+    return sizeof(UK) * (kRadix / 2) * cols;
 }
 template <class UK>
-constexpr size_t hist_lds_bytes()
+constexpr size_t hist_lds_bytes(uint32_t cols)
 {
-    return (hist_table_words<UK>() + 17) * 4;
+    return (hist_table_words<UK>(cols) + 17) * 4;
 }
-constexpr uint64_t kHistRoundSteps = 255;  // loop steps between flushes of the lane-column table
+// Loop steps (of `step` keys) between flushes of the table: a column counts
+// its lanes' share of them in 16 bits.
+constexpr uint64_t hist_round_steps(uint64_t step, uint32_t cols) { return 65535ull * cols / step; }
 
-template <class UK, int KIND, bool DESC>
+template <class UK, class Code, uint32_t CO, int kVecs>
 __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
-    const UK *__restrict__ keys, uint64_t n, uint64_t chunk, uint32_t *bins, u32x4 *__restrict__ clear,
+    const UK *__restrict__ keys, uint64_t n, uint64_t chunk, Code code, uint32_t *bins, u32x4 *__restrict__ clear,
     uint64_t clear_vecs, uint32_t *arrivals, uint32_t *__restrict__ hot, uint32_t *__restrict__ plan)
 {
     constexpr int P = sizeof(UK);
-    constexpr uint32_t CO = hist_cols<UK>();
-    constexpr uint32_t W = (uint32_t)hist_table_words<UK>();
+    constexpr uint32_t W = (uint32_t)hist_table_words<UK>(CO);
     extern __shared__ uint32_t s_hist[];  // the counter table, then s_last, s_trivial[16]
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = lane_id();
@@ -336,10 +351,10 @@ __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
     const uint64_t b0 = (uint64_t)blockIdx.x * chunk;
     const uint64_t b1 = b0 + chunk < n ? b0 + chunk : n;
     auto count = [&](UK raw) {
-        const UK tk = sort_key<UK, KIND, DESC>(raw);
+        const UK tk = code.in(raw);
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-            const uint32_t dg = digit_of<UK, KIND, DESC>(tk, p * kRadixBits);
+            const uint32_t dg = code.digit(tk, p * kRadixBits);
             atomicAdd(&s_hist[((uint32_t)p * (kRadix / 2) + (dg & 127u)) * CO + lane % CO], dg & 128u ? 0x10000u : 1u);
         }
     };
@@ -363,11 +378,10 @@ __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
         }
     };
     constexpr uint64_t V = 16 / sizeof(UK);
-    constexpr int kVecs = 4;
     constexpr uint64_t step = (uint64_t)kHistBlock * V * kVecs;
     const bool vec = (reinterpret_cast<uintptr_t>(keys) & 15) == 0;
     // rounds of whole steps (every round but the last is a multiple of the step)
-    const uint64_t round_len = kHistRoundSteps * step;
+    constexpr uint64_t round_len = hist_round_steps(step, CO) * step;
     for (uint64_t r0 = b0; r0 < b1;) {
         const uint64_t r1 = b1 - r0 > round_len ? r0 + round_len : b1;
         uint64_t tail = r0;
@@ -482,10 +496,10 @@ __device__ __forceinline__ uint32_t set_half16(uint32_t w, int hi, uint32_t v)
 
 // MATCH: rank by ballot match (stable by construction) instead of relying on
 // the lane order of same-address LDS atomics (rs_rank_path picks one).
-template <int IPT, class UK, class UV, int KIND, bool PAIRS, bool DESC, bool MATCH>
+template <int IPT, class UK, class UV, class Code, bool PAIRS, bool MATCH>
 __global__ __launch_bounds__(kOsBlock)
 __attribute__((amdgpu_waves_per_eu(os_waves_per_eu<UK, UV, PAIRS, MATCH>(), os_waves_per_eu<UK, UV, PAIRS, MATCH>())))
-void rs_onesweep_kernel(RsBuffers<UK, UV> buf, uint32_t n, uint32_t shift, const uint32_t *__restrict__ bins,
+void rs_onesweep_kernel(RsBuffers<UK, UV> buf, Code code, uint32_t n, uint32_t shift, const uint32_t *__restrict__ bins,
                         LbState regions, uint32_t log_run, const uint32_t *__restrict__ hot_digits,
                         const uint32_t *__restrict__ pass_plan, WaitCtl ctl)
 {
@@ -499,7 +513,7 @@ void rs_onesweep_kernel(RsBuffers<UK, UV> buf, uint32_t n, uint32_t shift, const
     // 8: their walk spans ~8 batch words, and a wave walks until its slowest
     // digit ends (SortPairs u64 -> u32 at 2^27, all 8 passes: 5851 -> 5805
     // us; 6 of 8 passes skipped: 1686 -> 1676 us; a window of 4 gains half).
-    constexpr int kWindow = PAIRS && os_waves_per_eu<UK, UV, PAIRS, MATCH>() == 4 ? 8 : 2;
+    constexpr int kWindow = IPT <= 8 ? 8 : PAIRS && os_waves_per_eu<UK, UV, PAIRS, MATCH>() == 4 ? 8 : 2;
     static_assert(TILE <= 65536, "tile ranks are packed in 16 bits");
     __shared__ OnesweepSmem<IPT, UK, UV> sm;
 
@@ -545,7 +559,7 @@ void rs_onesweep_kernel(RsBuffers<UK, UV> buf, uint32_t n, uint32_t shift, const
     const uint32_t wbase = base + wave * WAVE_ITEMS + lane;
     if (valid == (uint32_t)TILE) {
 #pragma unroll
-        for (int u = 0; u < IPT; ++u) tk[u] = sort_key<UK, KIND, DESC>(__builtin_nontemporal_load(kin + wbase + u * kWave));
+        for (int u = 0; u < IPT; ++u) tk[u] = code.in(__builtin_nontemporal_load(kin + wbase + u * kWave));
         if constexpr (PAIRS) {
 #pragma unroll
             for (int u = 0; u < IPT; ++u) v[u] = __builtin_nontemporal_load(vin + wbase + u * kWave);
@@ -554,7 +568,7 @@ void rs_onesweep_kernel(RsBuffers<UK, UV> buf, uint32_t n, uint32_t shift, const
 #pragma unroll
         for (int u = 0; u < IPT; ++u) {
             const uint32_t idx = wbase + u * kWave;
-            tk[u] = idx < n ? sort_key<UK, KIND, DESC>(kin[idx]) : UK(~UK(0));
+            tk[u] = idx < n ? code.in(kin[idx]) : UK(~UK(0));
             if constexpr (PAIRS) v[u] = idx < n ? vin[idx] : UV(0);
         }
     }
@@ -575,7 +589,8 @@ void rs_onesweep_kernel(RsBuffers<UK, UV> buf, uint32_t n, uint32_t shift, const
     // adds their number; the others rank by position among them.  Every key
     // still takes one lane of one atomic instruction, in lane order.  (A
     // separate loop for passes without a hot digit measured no faster.)
-    const uint32_t hot = hot_digit;
+    // A tile with many pads (all of digit 255) represents those instead.
+    const uint32_t hot = (uint32_t)TILE - valid > (uint32_t)TILE / 16 ? (uint32_t)kRadix - 1 : hot_digit;
     auto rank_of = [&](uint32_t dd) -> uint32_t {
         if constexpr (MATCH) {
             const uint64_t peers = match_any8(dd);
@@ -596,8 +611,8 @@ void rs_onesweep_kernel(RsBuffers<UK, UV> buf, uint32_t n, uint32_t shift, const
     };
 #pragma unroll
     for (int u = 0; u < IPT; u += 2) {
-        const uint32_t r0 = rank_of(digit_of<UK, KIND, DESC>(tk[u], shift));
-        const uint32_t r1 = rank_of(digit_of<UK, KIND, DESC>(tk[u + 1], shift));
+        const uint32_t r0 = rank_of(code.digit(tk[u], shift));
+        const uint32_t r1 = rank_of(code.digit(tk[u + 1], shift));
         rank2[u / 2] = r0 | (r1 << 16);
         // (match path: one pair at a time keeps its ballot masks from spilling)
         if (MATCH || (u & 7) == 6) __builtin_amdgcn_sched_barrier(0);
@@ -653,7 +668,7 @@ void rs_onesweep_kernel(RsBuffers<UK, UV> buf, uint32_t n, uint32_t shift, const
     // measured slower: 2.13 against 2.07 ms per sort.)
 #pragma unroll
     for (int u = 0; u < IPT; ++u) {
-        const uint32_t dd = digit_of<UK, KIND, DESC>(tk[u], shift);
+        const uint32_t dd = code.digit(tk[u], shift);
         const uint32_t r = half16(rank2[u / 2], u & 1) + sm.cnt[wave][dd];
         rank2[u / 2] = set_half16(rank2[u / 2], u & 1, r);
         if (r < (uint32_t)HALF) sm.keys[r] = tk[u];
@@ -769,9 +784,9 @@ void rs_onesweep_kernel(RsBuffers<UK, UV> buf, uint32_t n, uint32_t shift, const
             const uint32_t li = j * kOsBlock + tid;
             const uint32_t i = h * HALF + li;
             const UK k = sm.keys[li];
-            const uint32_t p = i + sm.goff[digit_of<UK, KIND, DESC>(k, shift)];
+            const uint32_t p = i + sm.goff[code.digit(k, shift)];
             if constexpr (PAIRS) pos[j] = p;
-            if (p < n) kout[p] = raw_key<UK, KIND, DESC>(k);
+            if (p < n) kout[p] = code.out(k);
             if ((j & 7) == 7) __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (PAIRS) {
@@ -792,10 +807,38 @@ void rs_onesweep_kernel(RsBuffers<UK, UV> buf, uint32_t n, uint32_t shift, const
 }
 
 // ------------------------------------------------------------------ host side
-// Items per thread: 32 (16384-key tiles) for 4-byte keys alone, 16 (8192-key
-// tiles) for 8-byte keys or when values ride along (a tile's keys, values,
-// ranks and output positions then stay in registers without spilling).
+// Items per thread of the large sorts: 32 (16384-key tiles) for 4-byte keys
+// alone, 16 (8192-key tiles) for 8-byte keys or when values ride along (a
+// tile's keys, values, ranks and output positions then stay in registers
+// without spilling).
 constexpr int os_ipt(int key_bytes, int val_bytes) { return key_bytes == 8 || val_bytes ? 16 : 32; }
+
+// A pass cannot be shorter than one tile's life (20 us for 16384 keys, 7-9 us
+// for 2048), and below some millions of keys the large tiles leave CUs idle
+// besides (62 tiles at 2^20 keys).  So the smaller sorts take smaller tiles, as
+// long as the more tiles' look-back does not cost more.  Measured (us per sort;
+// 2048- / 4096-key tiles / those of os_ipt):
+//  * u32 keys: 2^17 38 / 41 / 61, 2^19 43 / 43 / 66, 10^6 58 / 58 / 104 (81 at
+//    1.5 * 10^6), 4 * 10^6 129 / 94 / 110, 8 * 10^6 231 / 147 / 121
+//  * u32 pairs, 4-byte values: 2^17 41 / 45 / 56, 10^6 70 / 68 / 74, 2 * 10^6
+//    97 / 79 / 81, 3 * 10^6 122 / 93 / 91
+//  * u32 pairs, 8-byte values: 2^19 54 / 57 / 71, 10^6 73 / 73 / 77, 2 * 10^6
+//    105 / 85 / 86
+//  * u64 keys: 2^17 74 / 87 / 95, 2^19 95 / 102 / 105, 10^6 127 / 126 / 125
+//  * u64 pairs, 4-byte values: 2^17 82 / 99 / 109, 2^19 108 / 120 / 127, 10^6
+//    139 / 140 / 143, 1.5 * 10^6 183 / 154 / 154
+constexpr int kIptSmall = 4, kIptMid = 8;
+constexpr uint64_t kSmallTilesMax = 1u << 19;
+constexpr uint64_t mid_tiles_max(int key_bytes, int val_bytes)
+{
+    return key_bytes == 8 ? 0 : val_bytes == 8 ? 3u << 19 : val_bytes == 4 ? 1u << 21 : 1u << 22;
+}
+constexpr int os_ipt_for(uint64_t n, int key_bytes, int val_bytes)
+{
+    return n <= kSmallTilesMax                       ? kIptSmall
+           : n <= mid_tiles_max(key_bytes, val_bytes) ? kIptMid
+                                                      : os_ipt(key_bytes, val_bytes);
+}
 
 // Temp layout: status header | bins[P][256] | hot[P] | plan[P] | arrivals
 // (zeroed together by rs_init) | tile counts x 4 regions | batch words x 4
@@ -810,7 +853,7 @@ RsLayout rs_layout(uint64_t n, int key_bytes, int val_bytes)
 {
     RsLayout L{};
     L.passes = (uint64_t)key_bytes;  // 8-bit digits
-    const uint64_t tile = (uint64_t)kOsBlock * os_ipt(key_bytes, val_bytes);
+    const uint64_t tile = (uint64_t)kOsBlock * os_ipt_for(n, key_bytes, val_bytes);
     L.tiles = n ? ceil_div(n, tile) : 0;
     L.batches = ceil_div(L.tiles, kBatch);
     L.bins_off = kStatusBytes;
@@ -822,6 +865,9 @@ RsLayout rs_layout(uint64_t n, int key_bytes, int val_bytes)
     L.ktmp_off = L.bw_off + kLbRegions * L.bw_region;
     L.vtmp_off = L.ktmp_off + align_up(n * key_bytes, 256);
     L.total = n ? L.vtmp_off + align_up(n * val_bytes, 256) : 0;
+    // never less than what a smaller sort (of more, smaller tiles) asks for
+    for (const uint64_t line : {kSmallTilesMax, mid_tiles_max(key_bytes, val_bytes)})
+        if (n > line && line) L.total = std::max(L.total, rs_layout(line, key_bytes, val_bytes).total);
     return L;
 }
 
@@ -945,14 +991,14 @@ int rs_rank_path(hipStream_t s)
 
 // XCD run length of one onesweep instantiation: 8R <= half the workgroups
 // resident at once.  log2(R) + 1, or -1 when the occupancy query fails.
-template <int IPT, class UK, class UV, int KIND, bool PAIRS, bool DESC, bool MATCH>
+template <int IPT, class UK, class UV, class Code, bool PAIRS, bool MATCH>
 int rs_log_run()
 {
     static DeviceCache run_cache;
     return device_cached(run_cache, [] {
         int per_cu = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, reinterpret_cast<const void *>(&rs_onesweep_kernel<IPT, UK, UV, KIND, PAIRS, DESC, MATCH>),
+                &per_cu, reinterpret_cast<const void *>(&rs_onesweep_kernel<IPT, UK, UV, Code, PAIRS, MATCH>),
                 kOsBlock, 0) != hipSuccess)
             return -1;
         const uint64_t resident = (uint64_t)(per_cu > 0 ? per_cu : 1) * (uint64_t)device_cus();
@@ -963,23 +1009,69 @@ int rs_log_run()
 }
 
 // The P onesweep launches of one sort.
-template <int IPT, class UK, class UV, int KIND, bool PAIRS, bool DESC, bool MATCH>
-int rs_passes(const RsBuffers<UK, UV> &buf, uint64_t n, const RsLayout &L, char *t, const uint32_t *bins,
+template <int IPT, class UK, class UV, class Code, bool PAIRS, bool MATCH>
+int rs_passes(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, const RsLayout &L, char *t, const uint32_t *bins,
               const uint32_t *hot, const uint32_t *plan, const WaitCtl &ctl, hipStream_t s)
 {
-    const int lr1 = rs_log_run<IPT, UK, UV, KIND, PAIRS, DESC, MATCH>();
+    const int lr1 = rs_log_run<IPT, UK, UV, Code, PAIRS, MATCH>();
     if (lr1 < 0) return LCPP_ERR_HIP;
     const uint32_t log_run = (uint32_t)(lr1 - 1);
     for (int p = 0; p < (int)L.passes; ++p) {
         const LbState lb{reinterpret_cast<uint16_t *>(t + L.tc_off), reinterpret_cast<uint64_t *>(t + L.bw_off),
                          L.tc_region / 2, L.bw_region / 8};
         LCPP_LAUNCH("rs_onesweep", s,
-                    (rs_onesweep_kernel<IPT, UK, UV, KIND, PAIRS, DESC, MATCH><<<(uint32_t)L.tiles, kOsBlock, 0, s>>>(
-                        buf, (uint32_t)n, (uint32_t)(p * kRadixBits), bins + p * kRadix, lb, log_run, hot + p,
+                    (rs_onesweep_kernel<IPT, UK, UV, Code, PAIRS, MATCH><<<(uint32_t)L.tiles, kOsBlock, 0, s>>>(
+                        buf, code, (uint32_t)n, (uint32_t)(p * kRadixBits), bins + p * kRadix, lb, log_run, hot + p,
                         plan + p, ctl)));
         LCPP_CHECK_LAUNCH();
     }
     return LCPP_OK;
+}
+
+// Init, histogram and passes of one sort of n keys.  MID: the tile and the
+// histogram of the mid-size sorts.
+template <int IPT, class UK, class UV, class Code, bool PAIRS, bool MID>
+int rs_pipeline(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, const RsLayout &L, char *t, hipStream_t s)
+{
+    uint32_t *status = reinterpret_cast<uint32_t *>(t);
+    uint32_t *bins = reinterpret_cast<uint32_t *>(t + L.bins_off);
+    uint32_t *hot = reinterpret_cast<uint32_t *>(t + L.hot_off);
+    uint32_t *plan = hot + L.passes;
+    const int P = (int)L.passes;
+
+    // status header, bins, hot digits, plan and the arrival counter are contiguous
+    const uint32_t init_words = (uint32_t)((L.hot_off + (2 * L.passes + 1) * 4) / 4);
+    LCPP_LAUNCH("rs_init", s, rs_init_kernel<<<1, 256, 0, s>>>(status, init_words));
+    LCPP_CHECK_LAUNCH();
+    {
+        // one 1024-thread workgroup per CU (128 KB of LDS each)
+        constexpr uint32_t CO = MID ? kHistColsMid : hist_cols<UK>();
+        constexpr int kVecs = MID ? 1 : 4;
+        constexpr size_t lds = hist_lds_bytes<UK>(CO);
+        static DeviceCache lds_set;
+        if (device_cached(lds_set, [] {
+                return hipFuncSetAttribute(reinterpret_cast<const void *>(&rs_histogram_kernel<UK, Code, CO, kVecs>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess
+                           ? 1
+                           : -1;
+            }) < 0)
+            return LCPP_ERR_HIP;
+        const uint64_t htile = (uint64_t)kHistBlock * kVecs * (16 / sizeof(UK));
+        const uint64_t htiles = ceil_div(n, htile);
+        const uint64_t cus = (uint64_t)device_cus();
+        uint64_t grid = htiles < cus ? htiles : cus;
+        const uint64_t chunk = ceil_div(htiles, grid) * htile;
+        grid = ceil_div(n, chunk);
+        LCPP_LAUNCH("rs_histogram", s,
+                    (rs_histogram_kernel<UK, Code, CO, kVecs><<<(uint32_t)grid, kHistBlock, lds, s>>>(
+                        buf.kin, n, chunk, code, bins, reinterpret_cast<u32x4 *>(t + L.tc_off),
+                        (L.ktmp_off - L.tc_off) / 16, plan + P, hot, plan)));
+        LCPP_CHECK_LAUNCH();
+    }
+    const int path = rs_rank_path(s);
+    const WaitCtl ctl = wait_ctl(status);
+    return path == kRankMatch ? rs_passes<IPT, UK, UV, Code, PAIRS, true>(buf, code, n, L, t, bins, hot, plan, ctl, s)
+                              : rs_passes<IPT, UK, UV, Code, PAIRS, false>(buf, code, n, L, t, bins, hot, plan, ctl, s);
 }
 
 template <class UK, class UV, int KIND, bool PAIRS, bool DESC>
@@ -998,50 +1090,22 @@ int rs_run(void *temp, size_t temp_bytes, const void *kin_, void *kout_, const v
     if (temp_bytes < L.total) return LCPP_ERR_TEMP_TOO_SMALL;
     if (!temp || (reinterpret_cast<uintptr_t>(temp) & 255)) return LCPP_ERR_INVALID_ARG;
     char *t = static_cast<char *>(temp);
-    uint32_t *status = reinterpret_cast<uint32_t *>(t);
-    uint32_t *bins = reinterpret_cast<uint32_t *>(t + L.bins_off);
-    uint32_t *hot = reinterpret_cast<uint32_t *>(t + L.hot_off);
-    uint32_t *plan = hot + L.passes;
-    UK *ktmp = reinterpret_cast<UK *>(t + L.ktmp_off);
-    UV *vtmp = reinterpret_cast<UV *>(t + L.vtmp_off);
-    const int P = (int)L.passes;
     if (n <= small_sort_max(sizeof(UK)))
         return small_sort_launch(sizeof(UK), KIND, DESC, rs_rank_path(s) == kRankMatch, kin, kout,
-                                 PAIRS ? vin : nullptr, vout, sizeof(UV), (uint32_t)n, status, s);
-
-    // status header, bins, hot digits, plan and the arrival counter are contiguous
-    const uint32_t init_words = (uint32_t)((L.hot_off + (2 * L.passes + 1) * 4) / 4);
-    LCPP_LAUNCH("rs_init", s, rs_init_kernel<<<1, 256, 0, s>>>(status, init_words));
-    LCPP_CHECK_LAUNCH();
-    {
-        // one 1024-thread workgroup per CU (128 KB of LDS each)
-        constexpr size_t lds = hist_lds_bytes<UK>();
-        static DeviceCache lds_set;
-        if (device_cached(lds_set, [] {
-                return hipFuncSetAttribute(reinterpret_cast<const void *>(&rs_histogram_kernel<UK, KIND, DESC>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess
-                           ? 1
-                           : -1;
-            }) < 0)
-            return LCPP_ERR_HIP;
-        const uint64_t htile = (uint64_t)kHistBlock * 4 * (16 / sizeof(UK));
-        const uint64_t htiles = ceil_div(n, htile);
-        const uint64_t cus = (uint64_t)device_cus();
-        uint64_t grid = htiles < cus ? htiles : cus;
-        const uint64_t chunk = ceil_div(htiles, grid) * htile;
-        grid = ceil_div(n, chunk);
-        LCPP_LAUNCH("rs_histogram", s,
-                    rs_histogram_kernel<UK, KIND, DESC><<<(uint32_t)grid, kHistBlock, lds, s>>>(
-                        kin, n, chunk, bins, reinterpret_cast<u32x4 *>(t + L.tc_off),
-                        (L.ktmp_off - L.tc_off) / 16, plan + P, hot, plan));
-        LCPP_CHECK_LAUNCH();
-    }
-    const int path = rs_rank_path(s);
-    const WaitCtl ctl = wait_ctl(status);
+                                 PAIRS ? vin : nullptr, vout, sizeof(UV), (uint32_t)n, static_cast<uint32_t *>(temp), s);
     // buffers per pass come from the device-side plan
-    const RsBuffers<UK, UV> buf{kin, ktmp, kout, vin, vtmp, vout};
-    return path == kRankMatch ? rs_passes<IPT, UK, UV, KIND, PAIRS, DESC, true>(buf, n, L, t, bins, hot, plan, ctl, s)
-                              : rs_passes<IPT, UK, UV, KIND, PAIRS, DESC, false>(buf, n, L, t, bins, hot, plan, ctl, s);
+    const RsBuffers<UK, UV> buf{kin, reinterpret_cast<UK *>(t + L.ktmp_off), kout,
+                                vin, reinterpret_cast<UV *>(t + L.vtmp_off), vout};
+    constexpr int VB = PAIRS ? (int)sizeof(UV) : 0;
+    const int ipt = os_ipt_for(n, sizeof(UK), VB);
+    using Code = KeyCode<UK, KIND == kFloat>;
+    if (ipt == kIptSmall)
+        return rs_pipeline<kIptSmall, UK, UV, Code, PAIRS, true>(buf, Code::of(KIND, DESC), n, L, t, s);
+    if constexpr (mid_tiles_max(sizeof(UK), VB) != 0) {
+        if (ipt == kIptMid)
+            return rs_pipeline<kIptMid, UK, UV, Code, PAIRS, true>(buf, Code::of(KIND, DESC), n, L, t, s);
+    }
+    return rs_pipeline<IPT, UK, UV, StaticCode<UK, KIND, DESC>, PAIRS, false>(buf, {}, n, L, t, s);
 }
 
 int key_kind(lcpp_dtype k)

@@ -32,22 +32,6 @@ constexpr int kSsBlock = 1024;
 constexpr int kSsWaves = kSsBlock / kWave;
 constexpr int kSsRadix = 256;
 
-// Raw key -> sort key and back: in(k) = k ^ (negative ? neg : pos) ^ flip
-// (the twiddles of common/util_type.h:98-175; flip inverts for descending
-// order).  ZEROS (floating keys): `mz`, the sort key of -0.0, ranks as `pz`,
-// that of +0.0.
-template <class UK>
-struct KeyCode {
-    UK neg, pos, flip, mz, pz;
-    static constexpr UK kHigh = UK(1) << (sizeof(UK) * 8 - 1);
-    __device__ __forceinline__ UK in(UK k) const { return k ^ ((k & kHigh) ? neg : pos) ^ flip; }
-    __device__ __forceinline__ UK out(UK t) const
-    {
-        const UK u = t ^ flip;
-        return u ^ ((u & kHigh) ? pos : neg);
-    }
-};
-
 // A 4-byte key travels with its source position in one 8-byte LDS word.
 template <int IPT, class UK, bool PAIRS>
 struct SsSmem {
@@ -62,7 +46,7 @@ struct SsSmem {
 
 template <int IPT, class UK, bool PAIRS, bool ZEROS, bool MATCH>
 __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK *kout, const void *vin, void *vout,
-                                                              int val_bytes, uint32_t n, KeyCode<UK> code,
+                                                              int val_bytes, uint32_t n, KeyCode<UK, ZEROS> code,
                                                               uint32_t *status)
 {
     extern __shared__ __align__(16) unsigned char s_raw[];
@@ -71,12 +55,9 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
     const uint32_t p0 = wave * (kWave * IPT) + lane;  // position of item 0; item u: + u * 64
     if (tid == 0) *status = 0;
 
-    auto ranked = [&](UK t) { return ZEROS && t == code.mz ? code.pz : t; };
-    auto digit = [&](UK t, uint32_t sh) { return (uint32_t)(ranked(t) >> sh) & 255u; };
-
     UK tk[IPT];
     uint32_t src[PAIRS ? IPT : 1];
-    const UK first = ranked(code.in(kin[0]));
+    const UK first = code.ranked(code.in(kin[0]));
     UK diff = 0;
 #pragma unroll
     for (int u = 0; u < IPT; ++u) {
@@ -86,7 +67,7 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
     }
 #pragma unroll
     for (int u = 0; u < IPT; ++u)
-        if (p0 + u * kWave < n) diff |= ranked(tk[u]) ^ first;
+        if (p0 + u * kWave < n) diff |= code.ranked(tk[u]) ^ first;
     auto or_op = [](uint32_t a, uint32_t b) { return a | b; };
 #pragma unroll
     for (int h = 0; h < (int)sizeof(UK) / 4; ++h) {
@@ -112,7 +93,7 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
             for (int u = 0; u < IPT; ++u) {
                 // (no branch: positions past n add 0 to a counter per lane)
                 const bool ok = p0 + u * kWave < n;
-                const uint32_t d = digit(tk[u], shift);
+                const uint32_t d = code.digit(tk[u], shift);
                 if constexpr (MATCH) {
                     const uint64_t peers = match_any8(d) & ballot(ok);
                     const uint32_t below = mask_rank(peers);
@@ -152,7 +133,7 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
         __syncthreads();
         if (busy) {
 #pragma unroll
-            for (int u = 0; u < IPT; ++u) rank[u] += cnt[digit(tk[u], shift)];
+            for (int u = 0; u < IPT; ++u) rank[u] += cnt[code.digit(tk[u], shift)];
 #pragma unroll
             for (int u = 0; u < IPT; ++u)
                 if (p0 + u * kWave < n) {
@@ -207,7 +188,7 @@ __global__ __launch_bounds__(kSsBlock) void small_sort_kernel(const UK *kin, UK 
 }
 
 template <int IPT, class UK, bool PAIRS, bool ZEROS, bool MATCH>
-int ss_run(const KeyCode<UK> &code, const void *kin, void *kout, const void *vin, void *vout, int val_bytes,
+int ss_run(const KeyCode<UK, ZEROS> &code, const void *kin, void *kout, const void *vin, void *vout, int val_bytes,
            uint32_t n, uint32_t *status, hipStream_t s)
 {
     constexpr size_t lds = sizeof(SsSmem<IPT, UK, PAIRS>);
@@ -230,7 +211,7 @@ int ss_run(const KeyCode<UK> &code, const void *kin, void *kout, const void *vin
 }
 
 template <class UK, bool PAIRS, bool ZEROS, bool MATCH>
-int ss_size(const KeyCode<UK> &code, const void *kin, void *kout, const void *vin, void *vout, int vb, uint32_t n,
+int ss_size(const KeyCode<UK, ZEROS> &code, const void *kin, void *kout, const void *vin, void *vout, int vb, uint32_t n,
             uint32_t *status, hipStream_t s)
 {
     // items per thread: the fewest that hold n
@@ -240,27 +221,16 @@ int ss_size(const KeyCode<UK> &code, const void *kin, void *kout, const void *vi
     return LCPP_ERR_INVALID_ARG;
 }
 
-template <class UK>
+template <class UK, bool ZEROS>
 int ss_key(int kind, bool desc, bool match, const void *kin, void *kout, const void *vin, void *vout, int vb,
            uint32_t n, uint32_t *status, hipStream_t s)
 {
-    constexpr UK high = KeyCode<UK>::kHigh;
-    KeyCode<UK> c{0, 0, desc ? UK(~UK(0)) : UK(0), 0, 0};
-    if (kind == 1) c.neg = c.pos = high;
-    if (kind == 2) {
-        c.neg = UK(~UK(0));
-        c.pos = high;
-        c.mz = UK(~high) ^ c.flip;
-        c.pz = high ^ c.flip;
-    }
-    auto go = [&](auto pairs, auto zeros) {
-        return match ? ss_size<UK, decltype(pairs)::value, decltype(zeros)::value, true>(c, kin, kout, vin, vout, vb, n,
-                                                                                         status, s)
-                     : ss_size<UK, decltype(pairs)::value, decltype(zeros)::value, false>(c, kin, kout, vin, vout, vb,
-                                                                                          n, status, s);
-    };
-    if (kind == 2) return vin ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
-    return vin ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
+    const KeyCode<UK, ZEROS> c = KeyCode<UK, ZEROS>::of(kind, desc);
+    if (vin)
+        return match ? ss_size<UK, true, ZEROS, true>(c, kin, kout, vin, vout, vb, n, status, s)
+                     : ss_size<UK, true, ZEROS, false>(c, kin, kout, vin, vout, vb, n, status, s);
+    return match ? ss_size<UK, false, ZEROS, true>(c, kin, kout, vin, vout, vb, n, status, s)
+                 : ss_size<UK, false, ZEROS, false>(c, kin, kout, vin, vout, vb, n, status, s);
 }
 
 }  // namespace
@@ -269,10 +239,14 @@ int small_sort_launch(int key_bytes, int kind, bool descending, bool match, cons
                       const void *vals_in, void *vals_out, int val_bytes, uint32_t n, uint32_t *status,
                       hipStream_t s)
 {
-    return key_bytes == 4 ? ss_key<uint32_t>(kind, descending, match, keys_in, keys_out, vals_in, vals_out, val_bytes,
-                                             n, status, s)
-                          : ss_key<uint64_t>(kind, descending, match, keys_in, keys_out, vals_in, vals_out, val_bytes,
-                                             n, status, s);
+    auto go = [&](auto uk) {
+        using UK = decltype(uk);
+        return kind == kFloat ? ss_key<UK, true>(kind, descending, match, keys_in, keys_out, vals_in, vals_out,
+                                                 val_bytes, n, status, s)
+                              : ss_key<UK, false>(kind, descending, match, keys_in, keys_out, vals_in, vals_out,
+                                                  val_bytes, n, status, s);
+    };
+    return key_bytes == 4 ? go(uint32_t()) : go(uint64_t());
 }
 
 }  // namespace lcpp

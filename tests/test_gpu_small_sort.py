@@ -62,3 +62,28 @@ def test_outputs_may_alias_inputs(rank_path, n):
     DeviceRadixSort().SortPairs(tmp, dk, dk, dv, dv, n)
     rk, rv = o.radix_sort(k, v)
     assert same_bits(g.to_host(dk), rk) and same_bits(g.to_host(dv), rv)
+
+
+@pytest.mark.parametrize("kdt,vdt", [(np.uint32, None), (np.float32, None), (np.uint64, None), (np.float32, np.uint32),
+                                     (np.int32, np.int64), (np.float64, np.uint32)])
+@pytest.mark.parametrize("n", [(1 << 19) - 1, 1 << 19, (1 << 19) + 1, 3 << 19, (3 << 19) + 4095, 1 << 21,
+                               (1 << 21) + 2, 1 << 22, (1 << 22) + 1])
+def test_tile_sizes_change(rank_path, kdt, vdt, n):
+    """Keys with one frequent value (a hot digit in every pass) on either side of every line at which the
+    tiles change, and temp storage that a smaller sort always fits."""
+    import gpu_util as g
+    from lc_parallel_primitive_amd import DeviceRadixSort
+
+    k = g.random_array(kdt, n, seed=n % 1000)
+    k[::5] = k[0]
+    log(f"sort {np.dtype(kdt).name} {vdt} n={n}")
+    if vdt is None:
+        name = np.dtype(kdt).name
+        sizes = [DeviceRadixSort.GetSortKeysTempStorageBytes(name, m) for m in (n - 4097, n - 1, n)]
+        assert sizes == sorted(sizes)
+        assert same_bits(g.to_host(sort_keys(g.to_dev(k), n, kdt)), o.radix_sort(k, nthreads=8))
+    else:
+        v = g.random_array(vdt, n, seed=1)
+        rk, rv = o.radix_sort(k, v, nthreads=8)
+        ko, vo = sort_pairs(g.to_dev(k), g.to_dev(v), n, kdt, vdt)
+        assert same_bits(g.to_host(ko), rk) and same_bits(g.to_host(vo), rv)
