@@ -7,16 +7,17 @@
 // common/thread_operators.h:19-47 (ArgMaxOp/ArgMinOp).
 //
 // MI355X design: one streaming pass.  A grid of at most 512 workgroups
-// (1024 for ArgMin/ArgMax) partitions the input into equal contiguous chunks
-// whose length is a multiple of the tile (128 KiB; 48 KiB for Arg*), so
-// every workgroup's range is exact (the reference dispatches more blocks
-// than it partitions for N > 10,485,760 and reads past the end).  Each thread
-// streams 16-byte vectors (32 per tile; 12 for Arg*), folds them in
-// registers, the workgroup folds its four wave totals, and one partial per
-// workgroup lands in temp storage.  A
-// one-workgroup kernel folds the partials in a fixed order, so the float
-// result is deterministic for a given N.  N <= one tile needs no temp and
-// one launch.
+// (1024 for ArgMin/ArgMax) partitions the input's 16-byte vectors into equal
+// contiguous chunks, so every workgroup's range is exact (the reference
+// dispatches more blocks than it partitions for N > 10,485,760 and reads past
+// the end); the fewer than 16 bytes before the first 16-byte boundary and
+// after the last one are the first workgroup's.  Each thread streams vectors
+// (up to 32 loads in flight; 12 for Arg*), folds them in registers, the
+// workgroup folds its wave totals, and one partial per workgroup lands in temp
+// storage.  A one-workgroup kernel folds the partials in a fixed order, so the
+// float result is deterministic for a given N and alignment.  Inputs that one
+// workgroup reads sooner than a second launch would start (red_alone) take one
+// launch.
 //
 // ArgMin/ArgMax fold (value, index) pairs in the same kernels (the reference
 // first materialises an N-element pair array in temp storage, then reduces
@@ -46,27 +47,101 @@ constexpr uint32_t red_max_grid()
     return ARG ? 1024 : 512;
 }
 
-template <class T, bool ARG>
-constexpr uint64_t red_tile()
-{
-    return (uint64_t)kRedBlock * red_vecs<ARG>() * (16 / sizeof(T));
-}
-
-struct RedGrid {
+// Where the input's 16-byte vectors lie and how they are dealt out.
+struct RedPlan {
+    uint64_t head;   // elements before the first vector
+    uint64_t nv;     // vectors
+    uint64_t chunk;  // vectors per workgroup
     uint32_t grid;
-    uint64_t chunk;  // elements per workgroup, multiple of the tile
+    bool alone;      // one 1024-thread workgroup, one launch
 };
 
-template <class T, bool ARG>
-RedGrid red_grid(uint64_t n)
+// Most input bytes that one workgroup reduces alone.  It reads about 130 GB/s
+// (f32 Sum of 2^15 / 2^16 / 2^17: 2.4 / 3.3 / 5.0 us, ArgMax of 2^16 / 2^17: 5.4
+// / 8.3 us); the two launches of the split form take 2.4 + 1.5 us (ArgMax 3.3 +
+// 2.0) and a gap of 2 us between them.
+template <bool ARG>
+constexpr uint64_t red_alone_bytes()
 {
-    const uint64_t tile = red_tile<T, ARG>();
-    uint64_t tiles = ceil_div(n, tile);
-    if (tiles == 0) tiles = 1;
-    uint64_t grid = tiles < red_max_grid<ARG>() ? tiles : red_max_grid<ARG>();
-    uint64_t chunk = ceil_div(tiles, grid) * tile;
-    grid = n ? ceil_div(n, chunk) : 1;
-    return {(uint32_t)grid, chunk};
+    return ARG ? 1u << 18 : 1u << 19;
+}
+constexpr int kRedAloneBlock = 1024;
+
+// Workgroups for nv vectors: one for every kRedMinVecs vectors per thread, so
+// that an f32 input of 2^20 already has a workgroup on every CU (2.4 us; one
+// workgroup per 32 vectors per thread would be 32 of them).
+constexpr uint64_t kRedMinVecs = 4;
+template <bool ARG>
+constexpr uint32_t red_grid(uint64_t nv)
+{
+    const uint64_t g = nv / (kRedBlock * kRedMinVecs);
+    return g < 1 ? 1u : g > red_max_grid<ARG>() ? red_max_grid<ARG>() : (uint32_t)g;
+}
+
+template <class T, bool ARG>
+RedPlan red_plan(const T *in, uint64_t n)
+{
+    RedPlan p{};
+    const uint64_t off = reinterpret_cast<uintptr_t>(in) & 15;
+    p.head = off ? (16 - off) / sizeof(T) : 0;
+    if (p.head > n) p.head = n;
+    p.nv = (n - p.head) / (16 / sizeof(T));
+    p.alone = n * sizeof(T) <= red_alone_bytes<ARG>();
+    p.grid = p.alone ? 1 : red_grid<ARG>(p.nv);
+    p.chunk = ceil_div(p.nv, p.grid);
+    if (p.grid > 1) {
+        // one load of every thread, or where a chunk is long whole rounds of
+        // them (ArgMax of 2^28 f32: 157.6 us, 158.8 with shorter last rounds)
+        constexpr uint64_t round = (uint64_t)kRedBlock * red_vecs<ARG>();
+        p.chunk = align_up(p.chunk, p.chunk >= 4 * round ? round : kRedBlock);
+        p.grid = (uint32_t)ceil_div(p.nv, p.chunk);
+    }
+    return p;
+}
+
+// Temp layout: the status header, then one partial of `bytes` per workgroup.
+// Inputs of up to one 128 KiB tile (48 KiB for Arg*) need none.
+template <class T, bool ARG>
+uint64_t red_temp(uint64_t n, uint64_t bytes)
+{
+    const uint64_t tile = (uint64_t)kRedBlock * red_vecs<ARG>() * (16 / sizeof(T));
+    if (n <= tile) return 0;
+    const uint64_t g = n * sizeof(T) <= red_alone_bytes<ARG>() ? 1 : red_grid<ARG>(n / (16 / sizeof(T)));
+    return kStatusBytes + align_up(g * bytes, 256);
+}
+
+// Vectors [v0, v1) of the workgroup: fold(vector, its index), up to VECS loads
+// in flight per thread.
+template <int NT, int VECS, class T, class F>
+__device__ __forceinline__ void red_stream(const T *pv, uint64_t v0, uint64_t v1, F fold)
+{
+    constexpr uint64_t V = 16 / sizeof(T);
+    uint64_t i = v0 + threadIdx.x;
+    auto rounds = [&](auto loads) {
+        constexpr int L = decltype(loads)::value;
+        for (; i + (uint64_t)(L - 1) * NT < v1; i += (uint64_t)L * NT) {
+            u32x4 w[L];
+#pragma unroll
+            for (int q = 0; q < L; ++q) w[q] = ld16_nt(pv + (i + (uint64_t)q * NT) * V);
+#pragma unroll
+            for (int q = 0; q < L; ++q) fold(w[q], i + (uint64_t)q * NT);
+        }
+    };
+    rounds(std::integral_constant<int, VECS>{});
+    if constexpr (VECS > 8) rounds(std::integral_constant<int, 8>{});
+    // the rest, four at a time: a load past the end reads the last vector
+    // again and is not folded
+    for (; i < v1; i += 4 * NT) {
+        u32x4 w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint64_t v = i + (uint64_t)q * NT;
+            w[q] = ld16_nt(pv + (v < v1 ? v : v1 - 1) * V);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i + (uint64_t)q * NT < v1) fold(w[q], i + (uint64_t)q * NT);
+    }
 }
 
 // ---------------------------------------------------------------- transforms
@@ -154,53 +229,42 @@ __device__ __forceinline__ T fold16(T acc, u32x4 v, Op op, Xf xf)
 
 // Workgroup fold: wave butterflies, then thread 0 folds the wave totals in
 // wave order.  Result valid in thread 0.
-template <class T, class Op>
+template <int NT = kRedBlock, class T, class Op>
 __device__ __forceinline__ T block_reduce(T x, Op op)
 {
-    __shared__ T s_wave[kRedBlock / kWave];
+    __shared__ T s_wave[NT / kWave];
     x = wave_allreduce(x, op);
     if (lane_id() == 0) s_wave[threadIdx.x / kWave] = x;
     __syncthreads();
     if (threadIdx.x == 0) {
 #pragma unroll
-        for (int w = 1; w < kRedBlock / kWave; ++w) x = op(x, s_wave[w]);
+        for (int w = 1; w < NT / kWave; ++w) x = op(x, s_wave[w]);
     }
     return x;
 }
 
 // Partials: one per workgroup, or with `direct` (a single workgroup) the
 // result op(init, fold) itself.
-template <class T, class Op, class Xf>
-__global__ __launch_bounds__(kRedBlock) void reduce_partials_kernel(const T *__restrict__ in,
-                                                                    uint64_t n, uint64_t chunk,
-                                                                    T *__restrict__ partials,
-                                                                    T init, int direct, uint32_t *status)
+template <int NT, int VECS, class T, class Op, class Xf>
+__global__ __launch_bounds__(NT) void reduce_partials_kernel(const T *__restrict__ in, uint64_t n, uint64_t head,
+                                                             uint64_t nv, uint64_t chunk, T *__restrict__ partials,
+                                                             T init, int direct, uint32_t *status)
 {
     Op op;
     Xf xf;
     if (status && blockIdx.x == 0 && threadIdx.x == 0) *status = 0;  // nothing here waits
     T acc = Op::template identity<T>();
-    const uint64_t b0 = (uint64_t)blockIdx.x * chunk;
-    const uint64_t b1 = b0 + chunk < n ? b0 + chunk : n;
     const uint32_t tid = threadIdx.x;
     constexpr uint64_t V = 16 / sizeof(T);
-    constexpr uint64_t tile = red_tile<T, false>();
-    constexpr int VECS = red_vecs<false>();
-    uint64_t tail = b0;
-    if ((reinterpret_cast<uintptr_t>(in) & 15) == 0) {
-        const uint64_t full_end = b0 + (b1 - b0) / tile * tile;
-        for (uint64_t t = b0; t < full_end; t += tile) {
-            u32x4 v[VECS];
-#pragma unroll
-            for (int i = 0; i < VECS; ++i)
-                v[i] = ld16_nt((in + t + ((uint64_t)i * kRedBlock + tid) * V));
-#pragma unroll
-            for (int i = 0; i < VECS; ++i) acc = fold16<T>(acc, v[i], op, xf);
-        }
-        tail = full_end;
+    const uint64_t v0 = (uint64_t)blockIdx.x * chunk;
+    const uint64_t v1 = v0 + chunk < nv ? v0 + chunk : nv;
+    red_stream<NT, VECS>(in + head, v0, v1, [&](u32x4 w, uint64_t) { acc = fold16<T>(acc, w, op, xf); });
+    if (blockIdx.x == 0) {
+        if (tid < head) acc = op(acc, xf(in[tid]));
+        const uint64_t t = head + nv * V + tid;  // fewer than V elements are left
+        if (t < n) acc = op(acc, xf(in[t]));
     }
-    for (uint64_t i = tail + tid; i < b1; i += kRedBlock) acc = op(acc, xf(in[i]));
-    acc = block_reduce(acc, op);
+    acc = block_reduce<NT>(acc, op);
     if (tid == 0) partials[blockIdx.x] = direct ? op(init, acc) : acc;
 }
 
@@ -220,8 +284,7 @@ __global__ __launch_bounds__(kRedBlock) void reduce_final_kernel(const T *__rest
 template <class T>
 uint64_t reduce_temp(uint64_t n)
 {
-    RedGrid g = red_grid<T, false>(n);
-    return g.grid > 1 ? kStatusBytes + align_up((uint64_t)g.grid * sizeof(T), 256) : 0;
+    return red_temp<T, false>(n, sizeof(T));
 }
 
 template <class T, class Op, class Xf>
@@ -231,91 +294,79 @@ int reduce_launch(void *temp, size_t temp_bytes, const void *in_, void *out_, ui
     const T *in = static_cast<const T *>(in_);
     T *out = static_cast<T *>(out_);
     if (!out || (n && !in)) return LCPP_ERR_INVALID_ARG;
-    RedGrid g = red_grid<T, false>(n);
-    if (g.grid == 1) {
-        // one workgroup writes op(init, fold) itself; a temp buffer, if one
-        // is passed, only has its status word cleared
-        uint32_t *st = temp && temp_bytes >= kStatusBytes && !(reinterpret_cast<uintptr_t>(temp) & 255)
-                           ? static_cast<uint32_t *>(temp)
-                           : nullptr;
-        if (n == 0) {
-            LCPP_LAUNCH("reduce_final", s,
-                        (reduce_final_kernel<T, Op><<<1, kRedBlock, 0, s>>>(out, 0, out, init, st)));
-        } else {
-            LCPP_LAUNCH("reduce_partials", s,
-                        (reduce_partials_kernel<T, Op, Xf><<<1, kRedBlock, 0, s>>>(in, n, g.chunk, out, init, 1, st)));
-        }
+    const uint64_t need = reduce_temp<T>(n);
+    if (temp_bytes < need) return LCPP_ERR_TEMP_TOO_SMALL;
+    const bool aligned = temp && !(reinterpret_cast<uintptr_t>(temp) & 255);
+    if (need && !aligned) return LCPP_ERR_INVALID_ARG;
+    // a temp buffer passed without need only has its status word cleared
+    uint32_t *st = aligned && temp_bytes >= kStatusBytes ? static_cast<uint32_t *>(temp) : nullptr;
+    if (n == 0) {
+        LCPP_LAUNCH("reduce_final", s, (reduce_final_kernel<T, Op><<<1, kRedBlock, 0, s>>>(out, 0, out, init, st)));
         LCPP_CHECK_LAUNCH();
         return LCPP_OK;
     }
-    if (temp_bytes < reduce_temp<T>(n)) return LCPP_ERR_TEMP_TOO_SMALL;
-    if (!temp || (reinterpret_cast<uintptr_t>(temp) & 255)) return LCPP_ERR_INVALID_ARG;
+    const RedPlan p = red_plan<T, false>(in, n);
+    if (p.alone) {
+        LCPP_LAUNCH("reduce_partials", s,
+                    (reduce_partials_kernel<kRedAloneBlock, 8, T, Op, Xf><<<1, kRedAloneBlock, 0, s>>>(
+                        in, n, p.head, p.nv, p.chunk, out, init, 1, st)));
+        LCPP_CHECK_LAUNCH();
+        return LCPP_OK;
+    }
     T *partials = reinterpret_cast<T *>(static_cast<char *>(temp) + kStatusBytes);
     LCPP_LAUNCH("reduce_partials", s,
-                (reduce_partials_kernel<T, Op, Xf><<<g.grid, kRedBlock, 0, s>>>(
-                    in, n, g.chunk, partials, init, 0, static_cast<uint32_t *>(temp))));
+                (reduce_partials_kernel<kRedBlock, red_vecs<false>(), T, Op, Xf><<<p.grid, kRedBlock, 0, s>>>(
+                    in, n, p.head, p.nv, p.chunk, partials, init, 0, st)));
     LCPP_CHECK_LAUNCH();
     LCPP_LAUNCH("reduce_final", s,
-                (reduce_final_kernel<T, Op><<<1, kRedBlock, 0, s>>>(partials, g.grid, out, init, nullptr)));
+                (reduce_final_kernel<T, Op><<<1, kRedBlock, 0, s>>>(partials, p.grid, out, init, nullptr)));
     LCPP_CHECK_LAUNCH();
     return LCPP_OK;
 }
 
 // ---------------------------------------------------------------- ArgMin / ArgMax
-template <class P, class Op>
+template <int NT = kRedBlock, class P, class Op>
 __device__ __forceinline__ P block_reduce_pair(P x, Op op)
 {
-    __shared__ P s_wave[kRedBlock / kWave];
+    __shared__ P s_wave[NT / kWave];
 #pragma unroll
     for (int m = 1; m < kWave; m <<= 1) x = op(x, shfl_xor_pair(x, m));
     if (lane_id() == 0) s_wave[threadIdx.x / kWave] = x;
     __syncthreads();
     if (threadIdx.x == 0) {
 #pragma unroll
-        for (int w = 1; w < kRedBlock / kWave; ++w) x = op(x, s_wave[w]);
+        for (int w = 1; w < NT / kWave; ++w) x = op(x, s_wave[w]);
     }
     return x;
 }
 
-template <class T, bool IS_MAX>
-__global__ __launch_bounds__(kRedBlock) void arg_partials_kernel(const T *__restrict__ in, uint64_t n,
-                                                                 uint64_t chunk,
-                                                                 IdxVal<T> *__restrict__ partials,
-                                                                 T *__restrict__ out,
-                                                                 uint32_t *__restrict__ out_index,
-                                                                 uint32_t *status)
+template <int NT, int VECS, class T, bool IS_MAX>
+__global__ __launch_bounds__(NT) void arg_partials_kernel(const T *__restrict__ in, uint64_t n, uint64_t head,
+                                                          uint64_t nv, uint64_t chunk,
+                                                          IdxVal<T> *__restrict__ partials, T *__restrict__ out,
+                                                          uint32_t *__restrict__ out_index, uint32_t *status)
 {
     using P = IdxVal<T>;
     ArgOp<IS_MAX> op;
     P acc = ArgOp<IS_MAX>::template identity<T>();
     if (status && blockIdx.x == 0 && threadIdx.x == 0) *status = 0;  // nothing here waits
-    const uint64_t b0 = (uint64_t)blockIdx.x * chunk;
-    const uint64_t b1 = b0 + chunk < n ? b0 + chunk : n;
     const uint32_t tid = threadIdx.x;
     constexpr uint64_t V = 16 / sizeof(T);
-    constexpr uint64_t tile = red_tile<T, true>();
-    constexpr int VECS = red_vecs<true>();
-    uint64_t tail = b0;
-    if ((reinterpret_cast<uintptr_t>(in) & 15) == 0) {
-        const uint64_t full_end = b0 + (b1 - b0) / tile * tile;
-        for (uint64_t t = b0; t < full_end; t += tile) {
-            u32x4 v[VECS];
+    const uint64_t v0 = (uint64_t)blockIdx.x * chunk;
+    const uint64_t v1 = v0 + chunk < nv ? v0 + chunk : nv;
+    red_stream<NT, VECS>(in + head, v0, v1, [&](u32x4 w, uint64_t v) {
+        T e[V];
+        unpack16<T>(w, e);
+        const uint32_t i0 = (uint32_t)(head + v * V);
 #pragma unroll
-            for (int i = 0; i < VECS; ++i)
-                v[i] = ld16_nt((in + t + ((uint64_t)i * kRedBlock + tid) * V));
-#pragma unroll
-            for (int i = 0; i < VECS; ++i) {
-                T e[V];
-                unpack16<T>(v[i], e);
-                const uint32_t i0 = (uint32_t)(t + ((uint64_t)i * kRedBlock + tid) * V);
-#pragma unroll
-                for (int j = 0; j < (int)V; ++j) acc = op(acc, P{e[j], i0 + (uint32_t)j});
-            }
-        }
-        tail = full_end;
+        for (int j = 0; j < (int)V; ++j) acc = op(acc, P{e[j], i0 + (uint32_t)j});
+    });
+    if (blockIdx.x == 0) {
+        if (tid < head) acc = op(acc, P{in[tid], tid});
+        const uint64_t t = head + nv * V + tid;  // fewer than V elements are left
+        if (t < n) acc = op(acc, P{in[t], (uint32_t)t});
     }
-    for (uint64_t i = tail + tid; i < b1; i += kRedBlock) acc = op(acc, P{in[i], (uint32_t)i});
-    acc = block_reduce_pair(acc, op);
+    acc = block_reduce_pair<NT>(acc, op);
     if (tid == 0) {
         if (out) {
             out[0] = acc.value;
@@ -346,8 +397,7 @@ __global__ __launch_bounds__(kRedBlock) void arg_final_kernel(const IdxVal<T> *_
 template <class T>
 uint64_t arg_temp(uint64_t n)
 {
-    RedGrid g = red_grid<T, true>(n);
-    return g.grid > 1 ? kStatusBytes + align_up((uint64_t)g.grid * sizeof(IdxVal<T>), 256) : 0;
+    return red_temp<T, true>(n, sizeof(IdxVal<T>));
 }
 
 template <class T, bool IS_MAX>
@@ -358,31 +408,32 @@ int arg_launch(void *temp, size_t temp_bytes, const void *in_, void *out_, uint3
     T *out = static_cast<T *>(out_);
     if (!out || !out_index || (n && !in)) return LCPP_ERR_INVALID_ARG;
     if (n > 0xFFFFFFFFull) return LCPP_ERR_INVALID_ARG;  // 32-bit indices, as the reference
-    RedGrid g = red_grid<T, true>(n);
-    if (g.grid == 1) {
-        uint32_t *st = temp && temp_bytes >= kStatusBytes && !(reinterpret_cast<uintptr_t>(temp) & 255)
-                           ? static_cast<uint32_t *>(temp)
-                           : nullptr;
-        if (n == 0) {
-            LCPP_LAUNCH("arg_final", s,
-                        (arg_final_kernel<T, IS_MAX><<<1, kRedBlock, 0, s>>>(nullptr, 0, out, out_index, st)));
-        } else {
-            LCPP_LAUNCH("arg_partials", s,
-                        (arg_partials_kernel<T, IS_MAX><<<1, kRedBlock, 0, s>>>(in, n, g.chunk, nullptr, out, out_index,
-                                                                                  st)));
-        }
+    const uint64_t need = arg_temp<T>(n);
+    if (temp_bytes < need) return LCPP_ERR_TEMP_TOO_SMALL;
+    const bool aligned = temp && !(reinterpret_cast<uintptr_t>(temp) & 255);
+    if (need && !aligned) return LCPP_ERR_INVALID_ARG;
+    uint32_t *st = aligned && temp_bytes >= kStatusBytes ? static_cast<uint32_t *>(temp) : nullptr;
+    if (n == 0) {
+        LCPP_LAUNCH("arg_final", s,
+                    (arg_final_kernel<T, IS_MAX><<<1, kRedBlock, 0, s>>>(nullptr, 0, out, out_index, st)));
         LCPP_CHECK_LAUNCH();
         return LCPP_OK;
     }
-    if (temp_bytes < arg_temp<T>(n)) return LCPP_ERR_TEMP_TOO_SMALL;
-    if (!temp || (reinterpret_cast<uintptr_t>(temp) & 255)) return LCPP_ERR_INVALID_ARG;
+    const RedPlan p = red_plan<T, true>(in, n);
+    if (p.alone) {
+        LCPP_LAUNCH("arg_partials", s,
+                    (arg_partials_kernel<kRedAloneBlock, 8, T, IS_MAX><<<1, kRedAloneBlock, 0, s>>>(
+                        in, n, p.head, p.nv, p.chunk, nullptr, out, out_index, st)));
+        LCPP_CHECK_LAUNCH();
+        return LCPP_OK;
+    }
     IdxVal<T> *partials = reinterpret_cast<IdxVal<T> *>(static_cast<char *>(temp) + kStatusBytes);
     LCPP_LAUNCH("arg_partials", s,
-                (arg_partials_kernel<T, IS_MAX><<<g.grid, kRedBlock, 0, s>>>(in, n, g.chunk, partials, nullptr, nullptr,
-                                                                             static_cast<uint32_t *>(temp))));
+                (arg_partials_kernel<kRedBlock, red_vecs<true>(), T, IS_MAX><<<p.grid, kRedBlock, 0, s>>>(
+                    in, n, p.head, p.nv, p.chunk, partials, nullptr, nullptr, st)));
     LCPP_CHECK_LAUNCH();
     LCPP_LAUNCH("arg_final", s,
-                (arg_final_kernel<T, IS_MAX><<<1, kRedBlock, 0, s>>>(partials, g.grid, out, out_index, nullptr)));
+                (arg_final_kernel<T, IS_MAX><<<1, kRedBlock, 0, s>>>(partials, p.grid, out, out_index, nullptr)));
     LCPP_CHECK_LAUNCH();
     return LCPP_OK;
 }

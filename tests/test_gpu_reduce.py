@@ -268,3 +268,33 @@ def test_past_2p32_elements(gpu):
     assert run_arg(False, d, m, np.int32) == (0, m - 1)
     del d
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.float32, np.float64])
+@pytest.mark.parametrize("kib", [48, 128, 256, 512, 516, 4096, 12 * 1024])
+@pytest.mark.parametrize("pad", [0, 1, 3])
+def test_sizes_where_the_split_changes(gpu, dtype, kib, pad):
+    """One element either side of the sizes at which one workgroup, the number of workgroups and the length of
+    their chunks change, at every alignment; the extreme sits in the ragged ends as well."""
+    import gpu_util as g
+    from lc_parallel_primitive_amd import DeviceReduce
+
+    size = np.dtype(dtype).itemsize
+    for n in (kib * 1024 // size - 1, kib * 1024 // size, kib * 1024 // size + 1):
+        a = g.random_array(dtype, n, seed=kib)
+        for at in (0, 1, n - 2, n - 1):
+            a[at] = np.finfo(dtype).max if np.dtype(dtype).kind == "f" else np.iinfo(dtype).max
+            d = g.to_dev(a, pad=pad)
+            tmp = g.temp(DeviceReduce.GetArgTempStorageBytes(np.dtype(dtype).name, n))
+            out, idx = g.empty(1, dtype), g.empty(1, np.uint32)
+            DeviceReduce().ArgMax(tmp, d, out, idx, n)
+            assert g.to_host(out)[0] == a[at] and g.to_host(idx)[0] == at
+            a[at] = 1
+        d = g.to_dev(a, pad=pad)
+        got = run("Sum", d, n, dtype)
+        if np.dtype(dtype).kind == "f":
+            s, ab = o.reduce_f64(a)
+            assert abs(float(got) - s) <= RTOL_SUM * ab + 1e-30
+        else:
+            assert got == o.reduce(o.OP_SUM, a)
+        assert run("Min", d, n, dtype) == o.reduce(o.OP_MIN, a)
