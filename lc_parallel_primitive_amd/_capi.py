@@ -93,6 +93,8 @@ def lib() -> ctypes.CDLL:
     Raises FileNotFoundError when the library has not been built: there is
     no fallback implementation."""
     global _lib
+    if _lib is not None:  # set once, complete: no lock on the calls after the first
+        return _lib
     with _lock:
         if _lib is None:
             if not os.path.exists(lib_path):
@@ -113,12 +115,24 @@ def check(status: int, what: str) -> None:
         raise LcppError(status, what)
 
 
+_codes: dict = {}  # dtype object -> lcpp_dtype, filled as dtypes are seen
+
+
 def dtype_code(dtype) -> int:
     """lcpp_dtype of a torch / numpy dtype or a dtype name."""
+    try:
+        return _codes[dtype]
+    except (KeyError, TypeError):
+        pass
     name = str(dtype).replace("torch.", "").replace("numpy.", "")
     if name not in LCPP_DTYPES:
         raise TypeError(f"unsupported dtype {dtype}")
-    return LCPP_DTYPES[name]
+    code = LCPP_DTYPES[name]
+    try:
+        _codes[dtype] = code
+    except TypeError:  # not hashable
+        pass
+    return code
 
 
 def profile_enable() -> None:
