@@ -297,6 +297,43 @@ __device__ __forceinline__ u32x4 pack16(const T (&in)[16 / sizeof(T)])
     return v;
 }
 
+// Vectors [v0, v1) of the workgroup: fold(vector, its index), up to VECS loads
+// in flight per thread.  CACHED: what is read here is read elsewhere too.
+template <int NT, int VECS, bool CACHED = false, class T, class F>
+__device__ __forceinline__ void stream_vecs(const T *pv, uint64_t v0, uint64_t v1, F fold)
+{
+    constexpr uint64_t V = 16 / sizeof(T);
+    uint64_t i = v0 + threadIdx.x;
+    auto load = [&](uint64_t v) {
+        return CACHED ? *reinterpret_cast<const u32x4 *>(pv + v * V) : ld16_nt(pv + v * V);
+    };
+    auto rounds = [&](auto loads) {
+        constexpr int L = decltype(loads)::value;
+        for (; i + (uint64_t)(L - 1) * NT < v1; i += (uint64_t)L * NT) {
+            u32x4 w[L];
+#pragma unroll
+            for (int q = 0; q < L; ++q) w[q] = load(i + (uint64_t)q * NT);
+#pragma unroll
+            for (int q = 0; q < L; ++q) fold(w[q], i + (uint64_t)q * NT);
+        }
+    };
+    rounds(std::integral_constant<int, VECS>{});
+    if constexpr (VECS > 8) rounds(std::integral_constant<int, 8>{});
+    // the rest, four at a time: a load past the end reads the last vector
+    // again and is not folded
+    for (; i < v1; i += 4 * NT) {
+        u32x4 w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint64_t v = i + (uint64_t)q * NT;
+            w[q] = load(v < v1 ? v : v1 - 1);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i + (uint64_t)q * NT < v1) fold(w[q], i + (uint64_t)q * NT);
+    }
+}
+
 // ---------------------------------------------------------------- raw buffers
 // A raw buffer resource (stride 0) over [p, p + bytes): loads past `bytes`
 // return 0 and stores past it are dropped by the address unit, so a ragged

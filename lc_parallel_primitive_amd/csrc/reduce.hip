@@ -110,40 +110,6 @@ uint64_t red_temp(uint64_t n, uint64_t bytes)
     return kStatusBytes + align_up(g * bytes, 256);
 }
 
-// Vectors [v0, v1) of the workgroup: fold(vector, its index), up to VECS loads
-// in flight per thread.
-template <int NT, int VECS, class T, class F>
-__device__ __forceinline__ void red_stream(const T *pv, uint64_t v0, uint64_t v1, F fold)
-{
-    constexpr uint64_t V = 16 / sizeof(T);
-    uint64_t i = v0 + threadIdx.x;
-    auto rounds = [&](auto loads) {
-        constexpr int L = decltype(loads)::value;
-        for (; i + (uint64_t)(L - 1) * NT < v1; i += (uint64_t)L * NT) {
-            u32x4 w[L];
-#pragma unroll
-            for (int q = 0; q < L; ++q) w[q] = ld16_nt(pv + (i + (uint64_t)q * NT) * V);
-#pragma unroll
-            for (int q = 0; q < L; ++q) fold(w[q], i + (uint64_t)q * NT);
-        }
-    };
-    rounds(std::integral_constant<int, VECS>{});
-    if constexpr (VECS > 8) rounds(std::integral_constant<int, 8>{});
-    // the rest, four at a time: a load past the end reads the last vector
-    // again and is not folded
-    for (; i < v1; i += 4 * NT) {
-        u32x4 w[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint64_t v = i + (uint64_t)q * NT;
-            w[q] = ld16_nt(pv + (v < v1 ? v : v1 - 1) * V);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (i + (uint64_t)q * NT < v1) fold(w[q], i + (uint64_t)q * NT);
-    }
-}
-
 // ---------------------------------------------------------------- transforms
 struct XfIdentity {
     template <class T>
@@ -258,7 +224,7 @@ __global__ __launch_bounds__(NT) void reduce_partials_kernel(const T *__restrict
     constexpr uint64_t V = 16 / sizeof(T);
     const uint64_t v0 = (uint64_t)blockIdx.x * chunk;
     const uint64_t v1 = v0 + chunk < nv ? v0 + chunk : nv;
-    red_stream<NT, VECS>(in + head, v0, v1, [&](u32x4 w, uint64_t) { acc = fold16<T>(acc, w, op, xf); });
+    stream_vecs<NT, VECS>(in + head, v0, v1, [&](u32x4 w, uint64_t) { acc = fold16<T>(acc, w, op, xf); });
     if (blockIdx.x == 0) {
         if (tid < head) acc = op(acc, xf(in[tid]));
         const uint64_t t = head + nv * V + tid;  // fewer than V elements are left
@@ -354,7 +320,7 @@ __global__ __launch_bounds__(NT) void arg_partials_kernel(const T *__restrict__ 
     constexpr uint64_t V = 16 / sizeof(T);
     const uint64_t v0 = (uint64_t)blockIdx.x * chunk;
     const uint64_t v1 = v0 + chunk < nv ? v0 + chunk : nv;
-    red_stream<NT, VECS>(in + head, v0, v1, [&](u32x4 w, uint64_t v) {
+    stream_vecs<NT, VECS>(in + head, v0, v1, [&](u32x4 w, uint64_t v) {
         T e[V];
         unpack16<T>(w, e);
         const uint32_t i0 = (uint32_t)(head + v * V);

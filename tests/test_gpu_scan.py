@@ -252,3 +252,35 @@ def test_scan_op_sum_full_size_exclusive_with_init(gpu):
     h = g.to_host(d)
     inc = np.cumsum(h, dtype=np.uint32) + np.uint32(init)
     assert got[0] == init and (got[1:] == inc[:-1]).all()
+
+
+@pytest.mark.parametrize("dtype", [np.uint32, np.float32, np.int64])
+@pytest.mark.parametrize("kib", [32, 64, 480, 512, 16 * 1024])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_sizes_where_the_path_changes(gpu, dtype, kib, in_place):
+    """Around the tiles and the limit of the one-launch scan and the limit of the smaller look-back tiles, at
+    every alignment; an output over the input takes the look-back path."""
+    import gpu_util as g
+    from lc_parallel_primitive_amd import DeviceScan
+
+    size = np.dtype(dtype).itemsize
+    for n in (kib * 1024 // size - 1, kib * 1024 // size, kib * 1024 // size + 1):
+        a = g.random_array(dtype, n, seed=kib)
+        tmp = g.temp(DeviceScan.GetTempStorageBytes(np.dtype(dtype).name, n))
+        assert tmp.numel() >= DeviceScan.GetTempStorageBytes(np.dtype(dtype).name, n - 1)
+        for pad in (0, 1, 3):
+            for inclusive in (False, True):
+                d = g.to_dev(a, pad=pad)
+                out = d if in_place else g.empty(n, dtype, pad=pad)
+                s = DeviceScan()
+                (s.InclusiveSum if inclusive else s.ExclusiveSum)(tmp, d, out, n)
+                got = g.to_host(out)
+                if np.dtype(dtype).kind == "f":
+                    ref, ab = o.scan_f64(a, inclusive)
+                    assert (np.abs(got.astype(np.float64) - ref) <= 1e-5 * ab + 1e-30).all()
+                else:
+                    assert (got == o.scan(a, inclusive)).all()
+        init = dtype(7)
+        d, out = g.to_dev(a), g.empty(n, dtype)
+        DeviceScan().ExclusiveScan(tmp, d, out, n, "max", init)
+        assert (g.to_host(out) == o.scan_op(a, False, o.OP_MAX, init)).all()
