@@ -18,7 +18,7 @@ BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "liblcpp_amd.so")
 DATAGEN_LIB = os.path.join(PKG, "liblcpp_datagen.so")
 
-LIB_SOURCES = ["runtime.hip", "reduce.hip", "scan.hip", "radix_sort.hip", "small_sort.hip", "segment_reduce.hip",
+LIB_SOURCES = ["runtime.hip", "reduce.hip", "scan.hip", "radix_sort.hip", "small_sort.hip", "tie_repair.hip", "segment_reduce.hip",
                "scan_by_key.hip", "reduce_by_key.hip"]
 DATAGEN_SOURCES = ["datagen.hip"]
 

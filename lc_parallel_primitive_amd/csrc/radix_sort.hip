@@ -69,6 +69,10 @@
 //  * The pass plan is made on the device: a pass whose digit is the same for
 //    every key (from the histogram) is skipped, and the others ping-pong so
 //    that the last one writes the output.
+//  * 8-byte keys: digits that are not needed to tell nearly all keys apart (a
+//    sample says so) get no pass; a last launch orders the keys that tie in the
+//    others (tie_repair.hip).  Small sorts take one workgroup (small_sort.hip),
+//    medium ones smaller tiles (os_ipt_for).
 //  * Descending order sorts the bit-inverted sort keys (one XOR in, one out,
 //    compiled only into the descending kernels), as RadixSortTwiddle<true>
 //    does; equal keys keep their input order.
@@ -78,6 +82,7 @@
 #include <mutex>
 
 #include "small_sort.hpp"
+#include "tie_repair.hpp"
 
 namespace lcpp {
 namespace {
@@ -125,12 +130,12 @@ __device__ __forceinline__ UK raw_key(UK sk)
 {
     return tw_out<UK, KIND>(DESC ? UK(~sk) : sk);
 }
-// Digit of a sort key.  -0.0 and +0.0 are given the same digits
+// What a sort key ranks as: -0.0 and +0.0 are given the same digits
 // (radix_rank_sort_operations.h:33-62, ProcessFloatMinusZero); their two sort
 // keys are adjacent, so folding either onto the other yields the same stable
 // order.
 template <class UK, int KIND, bool DESC>
-__device__ __forceinline__ uint32_t digit_of(UK tk, uint32_t shift)
+__device__ __forceinline__ UK rank_key(UK tk)
 {
     if constexpr (KIND == kFloat) {
         constexpr UK high = UK(1) << (sizeof(UK) * 8 - 1);
@@ -138,7 +143,12 @@ __device__ __forceinline__ uint32_t digit_of(UK tk, uint32_t shift)
         constexpr UK minus_zero = UK(~high) ^ flip;  // sort key of -0.0
         if (tk == minus_zero) tk = high ^ flip;      // sort key of +0.0
     }
-    return (uint32_t)(tk >> shift) & (kRadix - 1);
+    return tk;
+}
+template <class UK, int KIND, bool DESC>
+__device__ __forceinline__ uint32_t digit_of(UK tk, uint32_t shift)
+{
+    return (uint32_t)(rank_key<UK, KIND, DESC>(tk) >> shift) & (kRadix - 1);
 }
 
 // How a kernel turns raw keys into sort keys and digits: the key type and
@@ -149,6 +159,7 @@ struct StaticCode {
     using UK = UK_;
     __device__ __forceinline__ UK in(UK raw) const { return sort_key<UK, KIND, DESC>(raw); }
     __device__ __forceinline__ UK out(UK sk) const { return raw_key<UK, KIND, DESC>(sk); }
+    __device__ __forceinline__ UK ranked(UK tk) const { return rank_key<UK, KIND, DESC>(tk); }
     __device__ __forceinline__ uint32_t digit(UK tk, uint32_t shift) const { return digit_of<UK, KIND, DESC>(tk, shift); }
 };
 
@@ -210,6 +221,15 @@ __device__ __forceinline__ int batch_word_state(uint64_t w, uint32_t &v)
     return st;
 }
 
+// splitmix64's output function (Vigna): places, hashes and the probe's digits
+__device__ __forceinline__ uint64_t probe_mix(uint64_t x)
+{
+    x += 0x9E3779B97F4A7C15ull;
+    x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+    x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
+    return x ^ (x >> 31);
+}
+
 // ------------------------------------------------------------------ init
 __global__ __launch_bounds__(256) void rs_init_kernel(uint32_t *words, uint32_t count)
 {
@@ -237,9 +257,10 @@ constexpr int kLbRegions = 4;
 enum PlanBuf : uint32_t { kBufIn = 0, kBufTmp = 1, kBufOut = 2 };
 // Runs in the histogram's last workgroup (NT threads), after the acquire that
 // pairs with every workgroup's release of its bin adds.
+// The lowest `low` digits get no pass.
 template <int NT>
 __device__ void rs_make_plan(const uint32_t *bins, uint32_t passes, uint64_t n, uint32_t *__restrict__ hot,
-                             uint32_t *__restrict__ plan, uint32_t *s_trivial)
+                             uint32_t *__restrict__ plan, uint32_t *s_trivial, uint32_t low)
 {
     const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
     for (uint32_t p = wave; p < passes; p += NT / kWave) {
@@ -258,7 +279,7 @@ __device__ void rs_make_plan(const uint32_t *bins, uint32_t passes, uint64_t n, 
         }
         if (lane == 0) {
             hot[p] = (best >> 8) * 16 >= n ? 255u - (uint32_t)(best & 255u) : (uint32_t)kRadix;
-            s_trivial[p] = (best >> 8) == n;
+            s_trivial[p] = (best >> 8) == n || p < low;
         }
     }
     __syncthreads();
@@ -322,10 +343,101 @@ constexpr size_t hist_lds_bytes(uint32_t cols)
 // its lanes' share of them in 16 bits.
 constexpr uint64_t hist_round_steps(uint64_t step, uint32_t cols) { return 65535ull * cols / step; }
 
+// How many low digits of 8-byte keys need no pass, because keys that tie in the
+// others are few (tie_repair.hip orders those).  One workgroup puts kSamples
+// keys into a hash table by their upper bits, for 24 upper bits first, and a key
+// that meets another one of equal upper and different lower bits counts.  That
+// many of kSamples^2 / 2 pairs say that a key has count * n / (kSamples^2 / 2)
+// such neighbours on average; a quarter of one is taken: a repair with 0.7 of
+// them moves as many bytes as a pass (12 * 10^6 u64 -> u32 pairs: 75 against 61
+// us; with 0.003: 37).  (At most 64 meetings in any case, so that no single
+// group of tying keys can be large in a small input.)  At least two digits must
+// go, since the repair reads all keys once more.  The keys are taken four at a
+// time, from a pseudo-random place of each of 1024 equal parts of the input (at
+// 4096 places the histogram launch of 10^6 keys waited for it: 25.8 us, now
+// 20.0).  The workgroup runs beside those that count.
+// cut[0] = the number of digits, cut[1] = of bits; both are zeroed before.
+constexpr uint32_t kSamples = 4096, kPlaceKeys = 4, kTable = 8192, kMeetings = 64;
+constexpr uint64_t kMeetingKeys = (uint64_t)kSamples * kSamples / 2 / 4;  // most meetings * n
+template <class UK, class Code>
+__device__ void rs_sample(const UK *__restrict__ keys, uint64_t n, const Code &code, uint32_t *s_mem, uint32_t *s_acc,
+                          uint32_t *cut)
+{
+    UK *s_keys = reinterpret_cast<UK *>(s_mem);
+    uint32_t *s_table = s_mem + kSamples * sizeof(UK) / 4;
+    constexpr uint32_t kEach = kSamples / kHistBlock;
+    const uint32_t tid = threadIdx.x;
+    UK mine[kEach];
+    const uint64_t part = n / (kSamples / kPlaceKeys);  // >= 8: sorts of fewer keys take one workgroup
+#pragma unroll
+    for (uint32_t q = 0; q < kEach; ++q) {
+        const uint64_t j = (tid + q * kHistBlock) / kPlaceKeys;
+        mine[q] = code.ranked(code.in(keys[j * part + probe_mix(j) % (part - kPlaceKeys + 1) + tid % kPlaceKeys]));
+    }
+    const UK first = code.ranked(code.in(keys[0]));
+    for (uint32_t i = tid; i < kTable; i += kHistBlock) s_table[i] = 0;
+    if (tid < 3) s_acc[tid] = 0;
+    __syncthreads();
+    UK diff = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kEach; ++q) {
+        s_keys[tid + q * kHistBlock] = mine[q];
+        diff |= mine[q] ^ first;
+    }
+    auto or_op = [](uint32_t a, uint32_t b) { return a | b; };
+    const uint32_t d0 = wave_allreduce((uint32_t)diff, or_op), d1 = wave_allreduce((uint32_t)(diff >> 32), or_op);
+    if (lane_id() == 0) {
+        atomicOr(&s_acc[0], d0);
+        atomicOr(&s_acc[1], d1);
+    }
+    __syncthreads();
+    diff = (UK)s_acc[1] << 32 | s_acc[0];
+    uint32_t vary = 0;  // digits below `low` in which the sample's keys differ
+    for (uint32_t p = 0; p < 5; ++p) vary += (diff >> (p * kRadixBits) & 255u) != 0;
+    for (uint32_t low = 5; vary >= 2; --low) {
+        const uint32_t sh = low * kRadixBits;
+        if (diff >> sh != 0) {  // else all of them tie
+            uint32_t met = 0;
+#pragma unroll
+            for (uint32_t q = 0; q < kEach; ++q) {
+                const UK up = mine[q] >> sh;
+                uint32_t h = (uint32_t)probe_mix(up) % kTable;
+                for (;;) {  // at most half of the table is full
+                    const uint32_t old = atomicCAS(&s_table[h], 0u, tid + q * kHistBlock + 1);
+                    if (old == 0) break;
+                    const UK other = s_keys[old - 1];
+                    if (other >> sh == up) {
+                        met += other != mine[q] ? 1u : 0u;
+                        break;
+                    }
+                    h = (h + 1) % kTable;
+                }
+            }
+            met = wave_allreduce(met, SumOp());
+            if (lane_id() == 0 && met) atomicAdd(&s_acc[2], met);
+            __syncthreads();
+            const uint32_t total = s_acc[2];
+            if (total <= kMeetings && total * n <= kMeetingKeys) {
+                if (tid == 0) {
+                    cut[0] = low;
+                    cut[1] = sh;
+                }
+                return;
+            }
+            __syncthreads();
+            for (uint32_t i = tid; i < kTable; i += kHistBlock) s_table[i] = 0;
+            if (tid == 0) s_acc[2] = 0;
+            __syncthreads();
+        }
+        vary -= (diff >> ((low - 1) * kRadixBits) & 255u) != 0;
+    }
+}
+
 template <class UK, class Code, uint32_t CO, int kVecs>
 __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
     const UK *__restrict__ keys, uint64_t n, uint64_t chunk, Code code, uint32_t *bins, u32x4 *__restrict__ clear,
-    uint64_t clear_vecs, uint32_t *arrivals, uint32_t *__restrict__ hot, uint32_t *__restrict__ plan)
+    uint64_t clear_vecs, uint32_t *arrivals, uint32_t *__restrict__ hot, uint32_t *__restrict__ plan,
+    uint32_t *cut)
 {
     constexpr int P = sizeof(UK);
     constexpr uint32_t W = (uint32_t)hist_table_words<UK>(CO);
@@ -333,14 +445,21 @@ __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = lane_id();
     uint32_t *s_last = s_hist + W, *s_trivial = s_last + 1;
-    for (uint32_t i = tid; i < W; i += kHistBlock) s_hist[i] = 0;
+    // where low digits may be left out, the last workgroup samples the keys
+    const uint32_t counters = gridDim.x - (cut ? 1u : 0u);
+    const bool counts = blockIdx.x < counters;
+    if constexpr (sizeof(UK) == 8) {
+        if (!counts) rs_sample<UK>(keys, n, code, s_hist, s_trivial, cut);
+    }
+    if (counts)
+        for (uint32_t i = tid; i < W; i += kHistBlock) s_hist[i] = 0;
     __syncthreads();
     // The look-back state of four passes is zeroed here, one 16-byte store per
     // thread per loop step (this workgroup's share of it, front to back), so
     // the stores go out beside the key stream instead of before it (2^28 u32
     // keys: 48 MiB of state).  The arrival's release below covers them.
-    const uint64_t cshare = ceil_div(clear_vecs, (uint64_t)gridDim.x);
-    const uint64_t c0 = (uint64_t)blockIdx.x * cshare;
+    const uint64_t cshare = ceil_div(clear_vecs, (uint64_t)counters);
+    const uint64_t c0 = counts ? (uint64_t)blockIdx.x * cshare : clear_vecs;
     const uint64_t c1 = c0 + cshare < clear_vecs ? c0 + cshare : clear_vecs;
     uint64_t cnext = c0 + tid;
     auto clear_step = [&]() {
@@ -348,7 +467,7 @@ __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
         cnext += kHistBlock;
     };
 
-    const uint64_t b0 = (uint64_t)blockIdx.x * chunk;
+    const uint64_t b0 = counts ? (uint64_t)blockIdx.x * chunk : n;
     const uint64_t b1 = b0 + chunk < n ? b0 + chunk : n;
     auto count = [&](UK raw) {
         const UK tk = code.in(raw);
@@ -407,7 +526,7 @@ __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
         if (r0 < b1) flush(true);
     }
     while (cnext < c1) clear_step();  // what the loop steps did not cover
-    flush(false);
+    if (counts) flush(false);
 
     // The last workgroup to arrive plans the passes (hot digits, skipped
     // passes, buffer routing) from the finished bins: every workgroup's adds
@@ -422,7 +541,7 @@ __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
     __syncthreads();
     if (*s_last) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        rs_make_plan<kHistBlock>(bins, (uint32_t)P, n, hot, plan, s_trivial);
+        rs_make_plan<kHistBlock>(bins, (uint32_t)P, n, hot, plan, s_trivial, cut ? ld_relaxed(cut) : 0u);
     }
 }
 
@@ -858,7 +977,7 @@ RsLayout rs_layout(uint64_t n, int key_bytes, int val_bytes)
     L.batches = ceil_div(L.tiles, kBatch);
     L.bins_off = kStatusBytes;
     L.hot_off = L.bins_off + L.passes * kRadix * 4;  // hot digits, then the pass plan: one word each per pass
-    L.tc_off = align_up(L.hot_off + (2 * L.passes + 1) * 4, 256);  // + the histogram's arrival counter
+    L.tc_off = align_up(L.hot_off + (2 * L.passes + 3) * 4, 256);  // + the histogram's arrival counter, two cut words
     L.tc_region = align_up(L.tiles * kRadix * 2, 256);  // 16-bit tile counts
     L.bw_off = L.tc_off + kLbRegions * L.tc_region;
     L.bw_region = align_up(L.batches * kRadix * 8, 256);  // 64-bit batch words
@@ -881,15 +1000,6 @@ RsLayout rs_layout(uint64_t n, int key_bytes, int val_bytes)
 // Any violation selects the match path, which is stable by construction.
 constexpr int kRankAtomic = 1, kRankMatch = 2;
 constexpr uint32_t kProbeBlocks = 256, kProbeRounds = 32;
-
-// splitmix64's output function (Vigna): the probe's digits
-__device__ __forceinline__ uint64_t probe_mix(uint64_t x)
-{
-    x += 0x9E3779B97F4A7C15ull;
-    x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
-    x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
-    return x ^ (x >> 31);
-}
 
 // Four waves per workgroup, each on its own 256 counters; pattern = block & 3.
 // *violations += lanes whose atomic result differs from the counter's value
@@ -1031,7 +1141,8 @@ int rs_passes(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, const 
 // Init, histogram and passes of one sort of n keys.  MID: the tile and the
 // histogram of the mid-size sorts.
 template <int IPT, class UK, class UV, class Code, bool PAIRS, bool MID>
-int rs_pipeline(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, const RsLayout &L, char *t, hipStream_t s)
+int rs_pipeline(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, const RsLayout &L, char *t, uint32_t *cut,
+                hipStream_t s)
 {
     uint32_t *status = reinterpret_cast<uint32_t *>(t);
     uint32_t *bins = reinterpret_cast<uint32_t *>(t + L.bins_off);
@@ -1040,12 +1151,13 @@ int rs_pipeline(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, cons
     const int P = (int)L.passes;
 
     // status header, bins, hot digits, plan and the arrival counter are contiguous
-    const uint32_t init_words = (uint32_t)((L.hot_off + (2 * L.passes + 1) * 4) / 4);
+    const uint32_t init_words = (uint32_t)((L.hot_off + (2 * L.passes + 3) * 4) / 4);
     LCPP_LAUNCH("rs_init", s, rs_init_kernel<<<1, 256, 0, s>>>(status, init_words));
     LCPP_CHECK_LAUNCH();
     {
         // one 1024-thread workgroup per CU (128 KB of LDS each)
-        constexpr uint32_t CO = MID ? kHistColsMid : hist_cols<UK>();
+        constexpr uint32_t CO = !MID ? hist_cols<UK>() : sizeof(UK) == 4 ? kHistColsMid : 2 * kHistColsMid;
+        static_assert(sizeof(UK) == 4 || hist_table_words<UK>(CO) >= 2 * kSamples + kTable, "the sample's LDS");
         constexpr int kVecs = MID ? 1 : 4;
         constexpr size_t lds = hist_lds_bytes<UK>(CO);
         static DeviceCache lds_set;
@@ -1061,11 +1173,11 @@ int rs_pipeline(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, cons
         const uint64_t cus = (uint64_t)device_cus();
         uint64_t grid = htiles < cus ? htiles : cus;
         const uint64_t chunk = ceil_div(htiles, grid) * htile;
-        grid = ceil_div(n, chunk);
+        grid = ceil_div(n, chunk) + (cut ? 1 : 0);
         LCPP_LAUNCH("rs_histogram", s,
                     (rs_histogram_kernel<UK, Code, CO, kVecs><<<(uint32_t)grid, kHistBlock, lds, s>>>(
                         buf.kin, n, chunk, code, bins, reinterpret_cast<u32x4 *>(t + L.tc_off),
-                        (L.ktmp_off - L.tc_off) / 16, plan + P, hot, plan)));
+                        (L.ktmp_off - L.tc_off) / 16, plan + P, hot, plan, cut)));
         LCPP_CHECK_LAUNCH();
     }
     const int path = rs_rank_path(s);
@@ -1099,13 +1211,27 @@ int rs_run(void *temp, size_t temp_bytes, const void *kin_, void *kout_, const v
     constexpr int VB = PAIRS ? (int)sizeof(UV) : 0;
     const int ipt = os_ipt_for(n, sizeof(UK), VB);
     using Code = KeyCode<UK, KIND == kFloat>;
+    // 8-byte keys: where the sampled cut goes.  With fewer passes the first of
+    // them may read the input and write the output, so outputs over the inputs
+    // sort every digit.
+    auto apart = [](const void *a, const void *b, uint64_t bytes) {
+        const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+        return x + bytes <= y || y + bytes <= x;
+    };
+    uint32_t *cut = nullptr;
+    if (sizeof(UK) == 8 && apart(kin, kout, n * sizeof(UK)) && (!PAIRS || apart(vin, vout, n * sizeof(UV))))
+        cut = reinterpret_cast<uint32_t *>(t + L.hot_off) + 2 * L.passes + 1;
+    int rc;
     if (ipt == kIptSmall)
-        return rs_pipeline<kIptSmall, UK, UV, Code, PAIRS, true>(buf, Code::of(KIND, DESC), n, L, t, s);
-    if constexpr (mid_tiles_max(sizeof(UK), VB) != 0) {
-        if (ipt == kIptMid)
-            return rs_pipeline<kIptMid, UK, UV, Code, PAIRS, true>(buf, Code::of(KIND, DESC), n, L, t, s);
-    }
-    return rs_pipeline<IPT, UK, UV, StaticCode<UK, KIND, DESC>, PAIRS, false>(buf, {}, n, L, t, s);
+        rc = rs_pipeline<kIptSmall, UK, UV, Code, PAIRS, true>(buf, Code::of(KIND, DESC), n, L, t, cut, s);
+    else
+    if (mid_tiles_max(sizeof(UK), VB) != 0 && ipt == kIptMid)
+        rc = rs_pipeline<mid_tiles_max(sizeof(UK), VB) ? kIptMid : kIptSmall, UK, UV, Code, PAIRS, true>(
+            buf, Code::of(KIND, DESC), n, L, t, cut, s);
+    else
+        rc = rs_pipeline<IPT, UK, UV, StaticCode<UK, KIND, DESC>, PAIRS, false>(buf, {}, n, L, t, cut, s);
+    if (rc != LCPP_OK || !cut) return rc;
+    return tie_repair_launch(KIND, DESC, kout, PAIRS ? vout : nullptr, VB, buf.ktmp, buf.vtmp, (uint32_t)n, cut + 1, s);
 }
 
 int key_kind(lcpp_dtype k)
