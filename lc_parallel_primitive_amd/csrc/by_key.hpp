@@ -191,5 +191,140 @@ __device__ __forceinline__ void bk_thread_pair(const V (&x)[VP], uint32_t bits, 
     for (int j = 0; j < VP; ++j) seg_fold(f, s, ((bits >> j) & 1u) != 0, x[j], op);
 }
 
+// ---------------------------------------------------------------- small inputs
+// They take one launch without look-back state: every 1024-thread workgroup (4
+// consecutive elements per thread) looks for the run that enters its tile by
+// itself, back to that run's head, and ReduceByKey counts the heads before its
+// tile as well.  What bounds it is the last workgroup's read of the keys before
+// it, from L2.  Measured (us per call, C calls back to back, int32 keys, f32
+// values, n = 2^15 / 2^16, look-back form 8.8 and 13.3): InclusiveSumByKey, runs of
+// 128: 4.8 / 4.9, all keys equal 7.9 / 11.2; ReduceByKey 6.8 / 9.8 (all equal
+// 7.2 / 10.6).  Without 16-byte loads, at 2^14: 6.8, 9.9; 9.0, 10.0.  The lines
+// lie where every kind of run still gains.
+constexpr int kBkAloneBlock = 1024;
+constexpr int kBkAloneWaves = kBkAloneBlock / kWave;
+constexpr int kBkAloneItems = 4;
+constexpr uint32_t kBkAloneTile = kBkAloneBlock * kBkAloneItems;
+constexpr uint64_t bk_alone_max(bool reduce, bool vec) { return (reduce ? 1u << 16 : 1u << 15) >> (vec ? 0 : 2); }
+
+template <class V>
+struct BkAloneSmem {
+    uint32_t cnt[kBkAloneWaves], last[kBkAloneWaves];
+    V fold[kBkAloneWaves], S[kBkAloneWaves];
+    uint32_t F, C[kBkAloneWaves];  // F bit w: wave w has a head
+};
+
+// A thread's items [i0, i0 + 4) of `p`, those below `end` (the others: `fill`);
+// `vec`: p is 16-byte aligned.
+template <class T>
+__device__ __forceinline__ void bk_alone_load(const T *p, uint32_t i0, uint32_t end, bool vec, T fill,
+                                              T (&x)[kBkAloneItems])
+{
+    if (vec && i0 + kBkAloneItems <= end) {
+        constexpr int V = 16 / (int)sizeof(T);
+#pragma unroll
+        for (int q = 0; q < kBkAloneItems / V; ++q) {
+            T e[V];
+            unpack16<T>(*reinterpret_cast<const u32x4 *>(p + i0 + q * V), e);
+#pragma unroll
+            for (int j = 0; j < V; ++j) x[q * V + j] = e[j];
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < kBkAloneItems; ++j) x[j] = i0 + j < end ? p[i0 + j] : fill;
+    }
+}
+
+// Heads of a thread's items below `end`: bit j for item j.
+template <class K>
+__device__ __forceinline__ uint32_t bk_alone_heads(const K *keys, uint32_t i0, uint32_t end, bool vec,
+                                                   K (&key)[kBkAloneItems], K &prev)
+{
+    uint32_t fl = 0;
+    prev = i0 > 0 && i0 < end ? keys[i0 - 1] : K(0);
+    bk_alone_load(keys, i0, end, vec, K(0), key);
+#pragma unroll
+    for (int j = 0; j < kBkAloneItems; ++j) {
+        const bool h = i0 + j == 0 || key[j] != (j ? key[j - 1] : prev);
+        fl |= (uint32_t)(h && i0 + j < end) << j;
+    }
+    return fl;
+}
+
+// What lies before the tile at `base` (> 0): `fold` over the values from the
+// last head before it on, and (COUNT) the number of heads.  Contains barriers;
+// every thread gets both.
+template <bool COUNT, class K, class V, class Op>
+__device__ __forceinline__ void bk_alone_before(const K *keys, const V *vals, uint32_t base, bool vec, Op op, V &fold,
+                                                uint32_t &heads, BkAloneSmem<V> &sm)
+{
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+    uint32_t head = 0, count = 0;  // head: the last one's position + 1
+    auto look = [&](uint32_t lo, uint32_t hi) {  // both multiples of the tile
+        uint32_t last = 0, c = 0;
+#pragma unroll 4
+        for (uint32_t i0 = lo + tid * kBkAloneItems; i0 < hi; i0 += kBkAloneTile) {
+            K key[kBkAloneItems], prev;
+            const uint32_t fl = bk_alone_heads(keys, i0, hi, vec, key, prev);
+            last = fl ? i0 + (uint32_t)(32 - __builtin_clz(fl)) : last;
+            if constexpr (COUNT) c += (uint32_t)__builtin_popcount(fl);
+        }
+        last = wave_allreduce(last, MaxOp());
+        if constexpr (COUNT) c = wave_allreduce(c, SumOp());
+        __syncthreads();
+        if (lane == 0) {
+            sm.last[wave] = last;
+            sm.cnt[wave] = c;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kBkAloneWaves; ++w) {
+            head = sm.last[w] > head ? sm.last[w] : head;
+            if constexpr (COUNT) count += sm.cnt[w];
+        }
+    };
+    // a run is most often found in the tile before; then all that is left
+    if (!COUNT) look(base - kBkAloneTile, base);
+    if (head == 0) look(0, COUNT ? base : base - kBkAloneTile);
+    V acc = op_identity<Op, V>();
+#pragma unroll 8
+    for (uint32_t i = head - 1 + tid; i < base; i += kBkAloneBlock) acc = op(acc, vals[i]);  // element 0 is a head
+    acc = wave_allreduce(acc, op);
+    if (lane == 0) sm.fold[wave] = acc;
+    __syncthreads();
+    fold = sm.fold[0];
+#pragma unroll
+    for (int w = 1; w < kBkAloneWaves; ++w) fold = op(fold, sm.fold[w]);
+    heads = count;
+}
+
+// The fold since the last head before this thread's first item.  f, s: the
+// thread's (has-head, fold since its last head) pair.  Contains a barrier.
+template <class V, class Op>
+__device__ __forceinline__ V bk_alone_prefix(bool f, V s, V before, Op op, BkAloneSmem<V> &sm)
+{
+    const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
+    wave_seg_scan(f, s, op);
+    const int fu = __shfl_up((int)f, 1);
+    const V su = shfl_up(s, 1);
+    if (lane == kWave - 1) {
+        sm.S[wave] = s;
+        if (f) atomicOr(&sm.F, 1u << wave);
+    }
+    __syncthreads();
+    V p = before;
+#pragma unroll
+    for (int w = 0; w < kBkAloneWaves; ++w)
+        if ((uint32_t)w < wave) p = ((sm.F >> w) & 1u) ? sm.S[w] : op(p, sm.S[w]);
+    return lane == 0 ? p : fu ? su : op(p, su);
+}
+
+// Whether [a, a + an) and [b, b + bn) share bytes.
+inline bool bk_overlap(const void *a, uint64_t an, const void *b, uint64_t bn)
+{
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + bn && y < x + an;
+}
+
 }  // namespace
 }  // namespace lcpp

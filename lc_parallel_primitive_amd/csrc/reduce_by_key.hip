@@ -630,6 +630,63 @@ __global__ __launch_bounds__(kBkBlock) void rbk_emit_kernel(const K *__restrict_
     }
 }
 
+// Small inputs (by_key.hpp): every workgroup counts the heads before its tile,
+// so its runs go straight to their places.
+template <class K, class V, class Op>
+__global__ __launch_bounds__(kBkAloneBlock) void rbk_alone_kernel(const K *__restrict__ keys,
+                                                                  const V *__restrict__ vin, uint32_t n,
+                                                                  K *__restrict__ unique_out, V *__restrict__ agg_out,
+                                                                  uint32_t *__restrict__ num_runs, int vec_ok,
+                                                                  uint32_t *status)
+{
+    __shared__ BkAloneSmem<V> sm;
+    Op op;
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+    const uint32_t base = blockIdx.x * kBkAloneTile, i0 = base + tid * kBkAloneItems;
+    if (tid == 0) {
+        sm.F = 0;
+        if (blockIdx.x == 0) *status = 0;
+    }
+    V x[kBkAloneItems];
+    const bool vec = vec_ok != 0;
+    bk_alone_load(vin, i0, n, vec, op_identity<Op, V>(), x);
+    K key[kBkAloneItems], prev;
+    const uint32_t fl = bk_alone_heads(keys, i0, n, vec, key, prev);
+    const uint32_t mine = (uint32_t)__builtin_popcount(fl);
+    const uint32_t upto = wave_inclusive_scan(mine, SumOp());
+    if (lane == kWave - 1) sm.C[wave] = upto;
+    __syncthreads();
+    V before = op_identity<Op, V>();
+    uint32_t c = 0;  // heads before this thread's first item
+    if (base) bk_alone_before<true>(keys, vin, base, vec, op, before, c, sm);
+    bool f;
+    V s;
+    bk_thread_pair<V>(x, fl, op, f, s);
+    s = bk_alone_prefix(f, s, before, op, sm);
+#pragma unroll
+    for (int w = 0; w < kBkAloneWaves; ++w)
+        if ((uint32_t)w < wave) c += sm.C[w];
+    c += upto - mine;
+#pragma unroll
+    for (int j = 0; j < kBkAloneItems; ++j) {
+        if ((fl >> j) & 1u) {  // closes run c - 1
+            if (c > 0) {
+                unique_out[c - 1] = j ? key[j - 1] : prev;
+                agg_out[c - 1] = s;
+            }
+            ++c;
+            s = x[j];
+        } else {
+            s = op(s, x[j]);
+        }
+        if (i0 + j == n - 1) {  // the last run, open at the last element
+            unique_out[c - 1] = key[j];
+            agg_out[c - 1] = s;
+            *num_runs = c;
+        }
+    }
+}
+
 template <class K, class V, class Op>
 int rbk_launch(void *temp, size_t tb, const void *keys_, const void *in_, void *uk_, void *agg_,
                uint32_t *num_runs, uint64_t n, hipStream_t s)
@@ -649,6 +706,17 @@ int rbk_launch(void *temp, size_t tb, const void *keys_, const void *in_, void *
     const RbkLayout<K, V> L = rbk_layout<K, V>(n);
     if (tb < L.total) return LCPP_ERR_TEMP_TOO_SMALL;
     if (!temp || (reinterpret_cast<uintptr_t>(temp) & 255)) return LCPP_ERR_INVALID_ARG;
+    const uint64_t kb = n * sizeof(K), vb = n * sizeof(V);
+    const int vec_ok = ((reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(in)) & 15) == 0;
+    if (n <= bk_alone_max(true, vec_ok) && !bk_overlap(uk, kb, keys, kb) && !bk_overlap(uk, kb, in, vb) &&
+        !bk_overlap(agg, vb, keys, kb) && !bk_overlap(agg, vb, in, vb) && !bk_overlap(num_runs, 4, keys, kb) &&
+        !bk_overlap(num_runs, 4, in, vb)) {
+        LCPP_LAUNCH("reduce_by_key_alone", s,
+                    (rbk_alone_kernel<K, V, Op><<<(uint32_t)ceil_div(n, kBkAloneTile), kBkAloneBlock, 0, s>>>(
+                        keys, in, (uint32_t)n, uk, agg, num_runs, vec_ok, static_cast<uint32_t *>(temp))));
+        LCPP_CHECK_LAUNCH();
+        return LCPP_OK;
+    }
     char *t = static_cast<char *>(temp);
     uint32_t *tile_count = reinterpret_cast<uint32_t *>(t + L.count_off);
     V *tile_fold = reinterpret_cast<V *>(t + L.fold_off);
@@ -664,7 +732,6 @@ int rbk_launch(void *temp, size_t tb, const void *keys_, const void *in_, void *
     if (lb_init(reinterpret_cast<uint64_t *>(t), L.count_off / 8, s, "reduce_by_key_init") != LCPP_OK)
         return LCPP_ERR_HIP;
     const WaitCtl ctl = wait_ctl(reinterpret_cast<uint32_t *>(t));
-    const int vec_ok = ((reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(in)) & 15) == 0;
     LCPP_LAUNCH("reduce_by_key_tile", s,
                 (rbk_tile_kernel<K, V, Op><<<(uint32_t)L.tiles, kBkBlock, 0, s>>>(
                     keys, in, (uint32_t)n, tile_count, tile_fold, pkeys, pvals, uk, agg, tcwords, tvwords, bwords,

@@ -133,6 +133,49 @@ __global__ __launch_bounds__(kBkBlock) void scan_by_key_kernel(const K *__restri
     }
 }
 
+// Small inputs (by_key.hpp).
+template <class K, class V, class Op, bool INCLUSIVE>
+__global__ __launch_bounds__(kBkAloneBlock) void scan_by_key_alone_kernel(const K *__restrict__ keys,
+                                                                          const V *__restrict__ vin,
+                                                                          V *__restrict__ vout, uint32_t n, V init,
+                                                                          int vec_ok, uint32_t *status)
+{
+    __shared__ BkAloneSmem<V> sm;
+    Op op;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t base = blockIdx.x * kBkAloneTile, i0 = base + tid * kBkAloneItems;
+    if (tid == 0) {
+        sm.F = 0;
+        if (blockIdx.x == 0) *status = 0;
+    }
+    V x[kBkAloneItems];
+    const bool vec = vec_ok != 0;
+    bk_alone_load(vin, i0, n, vec, op_identity<Op, V>(), x);
+    K key[kBkAloneItems], prev;
+    const uint32_t fl = bk_alone_heads(keys, i0, n, vec, key, prev);
+    __syncthreads();
+    V before = op_identity<Op, V>();
+    uint32_t heads;
+    if (base) bk_alone_before<false>(keys, vin, base, vec, op, before, heads, sm);
+    bool f;
+    V s;
+    bk_thread_pair<V>(x, fl, op, f, s);
+    s = bk_alone_prefix(f, s, before, op, sm);
+#pragma unroll
+    for (int j = 0; j < kBkAloneItems; ++j) {
+        const bool h = ((fl >> j) & 1u) != 0;
+        V r;
+        if constexpr (INCLUSIVE) {
+            s = h ? x[j] : op(s, x[j]);
+            r = op(s, init);
+        } else {
+            r = h ? init : op(s, init);
+            s = h ? x[j] : op(s, x[j]);
+        }
+        if (i0 + j < n) vout[i0 + j] = r;
+    }
+}
+
 template <class K, class V, class Op>
 int sbk_launch(bool inclusive, void *temp, size_t tb, const void *keys_, const void *in_, void *out_,
                uint64_t n, const void *init_, hipStream_t s)
@@ -149,13 +192,30 @@ int sbk_launch(bool inclusive, void *temp, size_t tb, const void *keys_, const v
     V init;
     if (init_) memcpy(&init, init_, sizeof(V));
     else init = V(0);
+    const int vec = ((reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(in)) & 15) == 0;
+    if (n <= bk_alone_max(false, vec) && !bk_overlap(out, n * sizeof(V), in, n * sizeof(V)) &&
+        !bk_overlap(out, n * sizeof(V), keys, n * sizeof(K))) {
+        const uint32_t grid = (uint32_t)ceil_div(n, kBkAloneTile);
+        uint32_t *status = static_cast<uint32_t *>(temp);
+        if (inclusive)
+            LCPP_LAUNCH("scan_by_key_inclusive", s,
+                        (scan_by_key_alone_kernel<K, V, Op, true><<<grid, kBkAloneBlock, 0, s>>>(keys, in, out,
+                                                                                                 (uint32_t)n, init,
+                                                                                                 vec, status)));
+        else
+            LCPP_LAUNCH("scan_by_key_exclusive", s,
+                        (scan_by_key_alone_kernel<K, V, Op, false><<<grid, kBkAloneBlock, 0, s>>>(keys, in, out,
+                                                                                                  (uint32_t)n, init,
+                                                                                                  vec, status)));
+        LCPP_CHECK_LAUNCH();
+        return LCPP_OK;
+    }
     uint64_t *head = static_cast<uint64_t *>(temp);  // status header, then the look-back words
     uint64_t *words = head + kStatusBytes / 8;
     if (lb_init(head, kStatusBytes / 8 + tiles * lb_words<V>(), s, "scan_by_key_init") != LCPP_OK)
         return LCPP_ERR_HIP;
     const WaitCtl ctl = wait_ctl(static_cast<uint32_t *>(temp));
-    const int vec_ok = ((reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(in) |
-                         reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+    const int vec_ok = vec && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
     if (inclusive)
         LCPP_LAUNCH("scan_by_key_inclusive", s,
                     (scan_by_key_kernel<K, V, Op, true><<<(uint32_t)tiles, kBkBlock, 0, s>>>(keys, in, out, n, words,
