@@ -22,7 +22,8 @@
 //      elements; entry 0 lacks the part of its run in earlier tiles) is
 //      gathered in LDS and stored contiguously into the tile's slot of a
 //      dense staging area.  Runs of mean 128 give 64 per tile.
-//    - A tile with more heads waits for the run count before it and the
+//    - A tile with more heads, and every tile of an input of at most
+//      kRbkDirectTiles tiles, waits for the run count before it and the
 //      fold entering it (to the nearest tile with a head) and writes its runs
 //      to the outputs directly.  The run count is two-level: every tile adds
 //      its head count to its batch word (8 tiles) as it publishes, so a
@@ -69,6 +70,15 @@ constexpr uint32_t kRbkGlobal = 0x80000000u;
 // (2^28 int32 keys, runs of mean 8: 937 us per call against 558 us padded;
 // runs of mean 128, where no tile waits: 367 against 353 us).
 constexpr uint32_t kRbkBwStride = 16;
+
+// Up to this many tiles every tile waits for its place and there is no emit
+// launch: they are all resident (four workgroups per CU), and a wait costs less
+// than another launch that moves the staged runs.  Measured (us per call, C
+// calls back to back, staged -> direct): int32 keys, f32 values, runs of 128: 2^20
+// 18.5 -> 12.8, 5 * 10^6 23.5 -> 18.4, 2^23 (1024 tiles) 26.9 -> 22.3, 2^24 39.0 ->
+// 40.4; runs of 4: 5 * 10^6 27.5 -> 21.7; int64, f64, runs of 1000: 2^21 19.5 ->
+// 13.9, 5 * 10^6 (1221 tiles) 26.7 -> 25.9, 2^24 55.4 -> 66.7.
+constexpr uint64_t kRbkDirectTiles = 1024;
 
 template <class K, class V>
 struct RbkLayout {
@@ -124,7 +134,8 @@ struct RbkSmem {
     V pw[kBkVecs * kBkWaves];
     uint32_t cw[kBkVecs * kBkWaves];
     uint32_t pf;  // bit l: a head before slice l
-    uint32_t tc;
+    uint32_t tc, tf;
+    V ts;
 };
 
 // Heads before `tile` (tile > 0, one wave): the counts of its batch-mates
@@ -211,9 +222,9 @@ __global__ __launch_bounds__(kBkBlock) void rbk_tile_kernel(const K *__restrict_
                                                             uint32_t n, uint32_t *__restrict__ tile_count,
                                                             V *__restrict__ tile_fold, K *__restrict__ pkeys,
                                                             V *__restrict__ pvals, K *__restrict__ unique_out,
-                                                            V *__restrict__ agg_out, uint64_t *tcwords,
-                                                            uint64_t *tvwords, uint64_t *bwords, int vec_ok,
-                                                            WaitCtl ctl)
+                                                            V *__restrict__ agg_out, uint32_t *num_runs,
+                                                            uint64_t *tcwords, uint64_t *tvwords, uint64_t *bwords,
+                                                            int vec_ok, int all_direct, WaitCtl ctl)
 {
     constexpr int VP = bk_vp<V>();
     constexpr uint32_t TILE = bk_tile<V>();
@@ -312,6 +323,8 @@ __global__ __launch_bounds__(kBkBlock) void rbk_tile_kernel(const K *__restrict_
         if (lane == 0) {
             sm.pf = (uint32_t)(heads_incl << 1);  // a head in slices < l
             sm.tc = tc;
+            sm.tf = tf;
+            sm.ts = ts;
             tile_count[tile] = tc | (tf ? kRbkHeadBit : 0u) | (tc > kRbkSlot ? kRbkDenseBit : 0u);
             tile_fold[tile] = ts;
             lb_publish(tcwords, tile, tc, kStPartial, ctl);
@@ -323,9 +336,9 @@ __global__ __launch_bounds__(kBkBlock) void rbk_tile_kernel(const K *__restrict_
     }
     __syncthreads();
 
-    // more than kRbkSlot heads: wait for the run count before the tile (wave
-    // 0) and the fold entering it (wave 1), then write the runs directly
-    const bool direct = sm.tc > kRbkSlot;
+    // more than kRbkSlot heads, or no emit launch to move staged runs: wait
+    // for the run count before the tile (wave 0) and the fold entering it (wave 1), then write the runs directly
+    const bool direct = all_direct || sm.tc > kRbkSlot;
     if (direct) {
         if (wave == 0) {
             const uint32_t p = tile > 0 ? rbk_count_before(tcwords, bwords, tile, ctl) : 0u;
@@ -475,6 +488,15 @@ __global__ __launch_bounds__(kBkBlock) void rbk_tile_kernel(const K *__restrict_
         else pass2(std::false_type{});
     } else {
         pass2(std::false_type{});
+    }
+    // no emit launch follows: the last run (open at element n - 1) and the count
+    if (all_direct && tile == gridDim.x - 1 && tid == 0) {
+        const uint32_t runs = cpre + sm.tc;
+        if (runs >= 1 && runs <= n) {
+            unique_out[runs - 1] = keys[n - 1];
+            agg_out[runs - 1] = sm.tf ? sm.ts : op(vpre, sm.ts);
+        }
+        *num_runs = runs;
     }
     if (!direct) {
         __syncthreads();
@@ -732,11 +754,13 @@ int rbk_launch(void *temp, size_t tb, const void *keys_, const void *in_, void *
     if (lb_init(reinterpret_cast<uint64_t *>(t), L.count_off / 8, s, "reduce_by_key_init") != LCPP_OK)
         return LCPP_ERR_HIP;
     const WaitCtl ctl = wait_ctl(reinterpret_cast<uint32_t *>(t));
+    const int all_direct = L.tiles <= kRbkDirectTiles;
     LCPP_LAUNCH("reduce_by_key_tile", s,
                 (rbk_tile_kernel<K, V, Op><<<(uint32_t)L.tiles, kBkBlock, 0, s>>>(
-                    keys, in, (uint32_t)n, tile_count, tile_fold, pkeys, pvals, uk, agg, tcwords, tvwords, bwords,
-                    vec_ok, ctl)));
+                    keys, in, (uint32_t)n, tile_count, tile_fold, pkeys, pvals, uk, agg, num_runs, tcwords, tvwords,
+                    bwords, vec_ok, all_direct, ctl)));
     LCPP_CHECK_LAUNCH();
+    if (all_direct) return LCPP_OK;
     LCPP_LAUNCH("reduce_by_key_emit", s,
                 (rbk_emit_kernel<K, V, Op><<<(uint32_t)L.groups, kBkBlock, 0, s>>>(
                     keys, (uint32_t)n, (uint32_t)L.tiles, tile_count, tile_fold, pkeys, pvals, uk, agg, num_runs,

@@ -84,3 +84,22 @@ def test_scan_in_place(gpu):
     DeviceScan().InclusiveSumByKey(tmp, dk, dv, dv, n)
     assert (g.to_host(dv) == o.scan_by_key(k, v, True)).all()
 
+
+@pytest.mark.parametrize("kdt,vdt,tile", [(np.int32, np.int32, 8192), (np.int64, np.uint64, 4096)])
+@pytest.mark.parametrize("run", [3, 128, 30_000])
+@pytest.mark.parametrize("tiles,extra", [(1023, 5), (1024, 0), (1024, 1), (1100, -3)])
+def test_reduce_by_key_where_staging_begins(gpu, kdt, vdt, tile, run, tiles, extra):
+    """Inputs whose tiles all wait for their place, and one tile more: tiles with few runs stage them."""
+    import gpu_util as g
+    from lc_parallel_primitive_amd import DeviceReduce
+
+    n = tiles * tile + extra
+    kn, vn = np.dtype(kdt).name, np.dtype(vdt).name
+    log(f"reduce by key {kn} {vn} n={n} run={run}")
+    k, v = keys_of(kdt, n, run, 7), g.random_array(vdt, n, seed=8)
+    rk, rv = o.reduce_by_key(k, v, o.OP_SUM)
+    tmp = g.temp(DeviceReduce.GetReduceByKeyTempStorageBytes(kn, vn, n))
+    uo, ao, runs = g.empty(n, kdt), g.empty(n, vdt), g.empty(1, np.uint32)
+    DeviceReduce().ReduceByKey(tmp, g.to_dev(k), g.to_dev(v), uo, ao, runs, "sum", n)
+    assert g.to_host(runs)[0] == rk.size
+    assert (g.to_host(uo)[:rk.size] == rk).all() and (g.to_host(ao)[:rk.size] == rv).all()
