@@ -323,9 +323,13 @@ constexpr uint32_t hist_cols()
 {
     return sizeof(UK) == 4 ? 64u : 32u;
 }
-// Sorts of smaller tiles: a workgroup counts 4096 keys only, and clearing and
-// summing the full table would cost more than that (100003 u32 keys: 8.0 us;
-// 64 columns and 16384 keys per workgroup: 11.6).
+// Sorts of smaller tiles: a workgroup counts few keys (8192 of 4 bytes), and
+// clearing and summing the full table would cost more than that (100003 u32
+// keys, the launch: 8.0 us; 64 columns and 16384 keys per workgroup: 11.6).
+// What bounds it then is the workgroups' adds to the same bins, so there are at
+// most half as many of them as CUs (a sort of u32 keys, us, 4096 / 8192 keys per
+// workgroup / 8192 and at most 128 workgroups: 2^16 35.8 / 36.4 / 36.4, 2^19 44.0 /
+// 42.6 / 42.5, 10^6 57.0 / 53.0 / 53.0, 2 * 10^6 69.2 / 69.3 / 66.9).
 constexpr uint32_t kHistColsMid = 8;
 // Dynamic LDS: the counter table, then 17 words of planning state for the
 // last workgroup (the kernel has no static LDS).
@@ -1155,10 +1159,10 @@ int rs_pipeline(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, cons
     LCPP_LAUNCH("rs_init", s, rs_init_kernel<<<1, 256, 0, s>>>(status, init_words));
     LCPP_CHECK_LAUNCH();
     {
-        // one 1024-thread workgroup per CU (128 KB of LDS each)
+        // one 1024-thread workgroup per CU (128 KB of LDS each), or per two
         constexpr uint32_t CO = !MID ? hist_cols<UK>() : sizeof(UK) == 4 ? kHistColsMid : 2 * kHistColsMid;
         static_assert(sizeof(UK) == 4 || hist_table_words<UK>(CO) >= 2 * kSamples + kTable, "the sample's LDS");
-        constexpr int kVecs = MID ? 1 : 4;
+        constexpr int kVecs = MID ? 2 : 4;
         constexpr size_t lds = hist_lds_bytes<UK>(CO);
         static DeviceCache lds_set;
         if (device_cached(lds_set, [] {
@@ -1170,7 +1174,7 @@ int rs_pipeline(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, cons
             return LCPP_ERR_HIP;
         const uint64_t htile = (uint64_t)kHistBlock * kVecs * (16 / sizeof(UK));
         const uint64_t htiles = ceil_div(n, htile);
-        const uint64_t cus = (uint64_t)device_cus();
+        const uint64_t cus = (uint64_t)device_cus() / (MID ? 2 : 1);
         uint64_t grid = htiles < cus ? htiles : cus;
         const uint64_t chunk = ceil_div(htiles, grid) * htile;
         grid = ceil_div(n, chunk) + (cut ? 1 : 0);
