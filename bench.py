@@ -11,7 +11,7 @@ measured live with HIP events recorded by the library on the launch stream;
 `secondary` holds every other BASELINE configuration (reduce 2^24 with the
 256 MB MALL flushed before each timed call and unflushed beside it, reduce
 2^28, both scans, the low-entropy sort, SortPairs as configured and with all
-8 digit passes moving data, the by-key primitives, segment reduce), each with
+a full key range, the by-key primitives, segment reduce), each with
 its dominant kernel's time and, where BASELINE names one, a CPU number;
 `cpu_baseline` and those per-entry CPU numbers time the oracle's C
 restatements of the reference algorithms (oracle/) at each configuration's
@@ -375,8 +375,9 @@ def main():
                         "pairs")
                 if full:
                     add("DeviceRadixSort::SortPairs uint64->uint32 N=2^27, keys over the full 64-bit range "
-                        "(all 8 digit passes move data)", 200 * n, call, 5, "rs_onesweep", items=n,
-                        note="200 B per pair: histogram 8 + 8 passes x (8 + 4 read, 8 + 4 written)")
+                        "(4 of 8 digit passes move data, ties are repaired)", 112 * n, call, 5, "rs_onesweep", items=n,
+                        note="112 B per pair: histogram 8 + 4 passes x (8 + 4 read, 8 + 4 written) + the repair's "
+                             "read of the keys 8; a pass for every digit would move 200")
                 else:
                     # 16 random low bits: passes 2..7 see one digit for every key and are
                     # skipped (identity permutations), so the bytes counted are the
@@ -385,7 +386,7 @@ def main():
                         "2 of 8 digit passes move data)", 56 * n, call, 5, "rs_onesweep", items=n,
                         cpu=lambda: cpu_pairs(n),
                         note="56 B per pair counted: the 6 passes whose digit every key shares are skipped; "
-                             "the full-range entry times 8 moving passes")
+                             "the full-range entry times 4 moving passes and the repair")
                     # on the 8-pass accounting (200 B per pair: histogram 8 + 8 x 24) an 8-pass
                     # onesweep needs 200 n / 8 TB/s at least; skipping the trivial passes beats that
                     e = sec[-1]

@@ -355,7 +355,10 @@ constexpr uint64_t hist_round_steps(uint64_t step, uint32_t cols) { return 65535
 // such neighbours on average; a quarter of one is taken: a repair with 0.7 of
 // them moves as many bytes as a pass (12 * 10^6 u64 -> u32 pairs: 75 against 61
 // us; with 0.003: 37).  (At most 64 meetings in any case, so that no single
-// group of tying keys can be large in a small input.)  At least two digits must
+// group of tying keys can be large in a small input; and no more keys than the
+// upper bits have values, since few meetings say little about a large one.  Above
+// kTieMaxItems keys no meeting still allows runs of 32, and every digit gets its
+// pass.)  At least two digits must
 // go, since the repair reads all keys once more.  The keys are taken four at a
 // time, from a pseudo-random place of each of 1024 equal parts of the input (at
 // 4096 places the histogram launch of 10^6 keys waited for it: 25.8 us, now
@@ -363,6 +366,7 @@ constexpr uint64_t hist_round_steps(uint64_t step, uint32_t cols) { return 65535
 // cut[0] = the number of digits, cut[1] = of bits; both are zeroed before.
 constexpr uint32_t kSamples = 4096, kPlaceKeys = 4, kTable = 8192, kMeetings = 64;
 constexpr uint64_t kMeetingKeys = (uint64_t)kSamples * kSamples / 2 / 4;  // most meetings * n
+constexpr uint64_t kTieMaxItems = 1u << 28;
 template <class UK, class Code>
 __device__ void rs_sample(const UK *__restrict__ keys, uint64_t n, const Code &code, uint32_t *s_mem, uint32_t *s_acc,
                           uint32_t *cut)
@@ -421,7 +425,7 @@ __device__ void rs_sample(const UK *__restrict__ keys, uint64_t n, const Code &c
             if (lane_id() == 0 && met) atomicAdd(&s_acc[2], met);
             __syncthreads();
             const uint32_t total = s_acc[2];
-            if (total <= kMeetings && total * n <= kMeetingKeys) {
+            if (total <= kMeetings && total * n <= kMeetingKeys && n >> (64 - sh) == 0) {
                 if (tid == 0) {
                     cut[0] = low;
                     cut[1] = sh;
@@ -1223,7 +1227,8 @@ int rs_run(void *temp, size_t temp_bytes, const void *kin_, void *kout_, const v
         return x + bytes <= y || y + bytes <= x;
     };
     uint32_t *cut = nullptr;
-    if (sizeof(UK) == 8 && apart(kin, kout, n * sizeof(UK)) && (!PAIRS || apart(vin, vout, n * sizeof(UV))))
+    if (sizeof(UK) == 8 && n <= kTieMaxItems && apart(kin, kout, n * sizeof(UK)) &&
+        (!PAIRS || apart(vin, vout, n * sizeof(UV))))
         cut = reinterpret_cast<uint32_t *>(t + L.hot_off) + 2 * L.passes + 1;
     int rc;
     if (ipt == kIptSmall)
