@@ -251,8 +251,10 @@ __device__ __forceinline__ void wg_reduce_segment(const T *__restrict__ in, T *_
         for (int q = 0; q < kWgLoads / 2; ++q)
             if (i + q * kSegBlock < nv) fold_vec(w[q], i + q * kSegBlock);
     }
-    const uint32_t t = head + nv * V + tid;  // fewer than V elements are left
-    if (tid < V && t < llen) a1 = Acc::fold(a1, p[t], lb + t);
+    // the fewer than V elements left, by their number: a position past them
+    // would wrap in a segment of nearly 2^32
+    const uint32_t rest = llen - head - nv * V;
+    if (tid < rest) a1 = Acc::fold(a1, p[llen - rest + tid], lb + (llen - rest + tid));
     A a = Acc::combine(a0, a1);
     a = Acc::wave_reduce(a);
     if (lane == 0) s_wave[wave] = a;

@@ -665,3 +665,35 @@ def test_segment_counts_where_the_split_changes(gpu, S, dtype):
             v, i = seg_call("ArgMax", d, S, (lb, le), dtype, arg=True)
             ev, ei = o.segment_reduce_arg(True, a, lb, le)
             assert same(v, ev) and (i == ei).all()
+
+
+@pytest.mark.parametrize("dtype", ["int32", "int64"])
+def test_longest_segments_off_a_16_byte_boundary(gpu, dtype):
+    """One segment of nearly 2^32 elements that begins off a 16-byte boundary:
+    the positions of its ragged end lie within a vector of 2^32 and must not
+    wrap to its first elements.  The input is zero but for marks at both ends,
+    so a sum that counts an element twice (or not at all) differs."""
+    import torch
+
+    import gpu_util as g
+    from lc_parallel_primitive_amd import DeviceSegmentReduce
+
+    top = (1 << 32) - 1
+    t = torch.zeros(top + 4, dtype=getattr(torch, dtype), device="cuda")
+    out = torch.empty(1, dtype=t.dtype, device="cuda")
+    r = DeviceSegmentReduce()
+    marks = torch.tensor([1, 10, 100, 1000], dtype=t.dtype, device="cuda")
+    for pad in range(4 if dtype == "int32" else 2):
+        for size in (top - 2, top - 1, top):
+            d = t[pad:pad + size]
+            d[:4], d[-4:] = marks, marks * 10_000
+            log(f"segment {dtype} size={size} pad={pad}")
+            r.Sum(None, d, out, 1, size)
+            assert int(g.to_host(out)[0]) == 11_110_000 + 1111, (pad, size)
+            if pad == 1:  # elements 1 .. size - 1 through offsets
+                b, e = g.to_dev(np.array([1], np.uint32)), g.to_dev(np.array([size], np.uint32))
+                r.Sum(None, t, out, 1, b, e)
+                assert int(g.to_host(out)[0]) == 1111 + 1_110_000, size  # all but the last mark
+            d[:4], d[-4:] = 0, 0
+    del t
+    torch.cuda.empty_cache()
