@@ -197,7 +197,7 @@ __device__ __forceinline__ void seg_store(typename SegAcc<T, OP>::A acc, uint32_
 // loads from the segment's first aligned element on, kWgLoads of them in
 // flight per thread (32 KiB per workgroup), the ragged ends element by
 // element.  One CU reads a segment, so what bounds it is the bytes in flight:
-// 2^26 f32 in segments of 30000 take 39.7 us (6.8 TB/s; 43.1 with four 4-byte
+// 2^26 f32 in segments of 30000 take 40.9 us (6.6 TB/s; 42.9 with four 4-byte
 // loads in flight).  Every thread must call it (barriers).
 constexpr int kWgLoads = 8;
 template <class T, int OP, bool FIXED>
@@ -218,14 +218,17 @@ __device__ __forceinline__ void wg_reduce_segment(const T *__restrict__ in, T *_
     const uint32_t ahead = (uint32_t)((16 - (reinterpret_cast<uintptr_t>(p) & 15)) & 15) / (uint32_t)sizeof(T);
     const uint32_t head = ahead < llen ? ahead : llen;
     const uint32_t nv = (llen - head) / V;
-    A a0 = Acc::identity(), a1 = a0;
-    if (tid < head) a0 = Acc::fold(a0, p[tid], lb + tid);
-    auto fold_vec = [&](u32x4 w, uint32_t i) {
+    // four partial folds per thread: a float sum's error grows with the chain of
+    // additions (two, f32, zero mean: rms error 1.3 times as large at 10^5
+    // elements, 1.5 at 5 * 10^5)
+    A acc[4] = {Acc::identity(), Acc::identity(), Acc::identity(), Acc::identity()};
+    if (tid < head) acc[0] = Acc::fold(acc[0], p[tid], lb + tid);
+    auto fold_vec = [&](u32x4 w, uint32_t i, int q) {  // q: its number among the vectors loaded together
         T e[V];
         unpack16<T>(w, e);
 #pragma unroll
         for (uint32_t j = 0; j < V; ++j) {
-            A &a = j & 1u ? a1 : a0;
+            A &a = acc[((uint32_t)q * V + j) & 3u];
             a = Acc::fold(a, e[j], lb + head + i * V + j);
         }
     };
@@ -236,7 +239,7 @@ __device__ __forceinline__ void wg_reduce_segment(const T *__restrict__ in, T *_
 #pragma unroll
         for (int q = 0; q < kWgLoads; ++q) w[q] = ld16_nt(pv + (uint64_t)(i + q * kSegBlock) * V);
 #pragma unroll
-        for (int q = 0; q < kWgLoads; ++q) fold_vec(w[q], i + q * kSegBlock);
+        for (int q = 0; q < kWgLoads; ++q) fold_vec(w[q], i + q * kSegBlock, q);
     }
     // the rest, half as many at a time: a load past the end reads the last
     // vector again and is not folded
@@ -249,13 +252,13 @@ __device__ __forceinline__ void wg_reduce_segment(const T *__restrict__ in, T *_
         }
 #pragma unroll
         for (int q = 0; q < kWgLoads / 2; ++q)
-            if (i + q * kSegBlock < nv) fold_vec(w[q], i + q * kSegBlock);
+            if (i + q * kSegBlock < nv) fold_vec(w[q], i + q * kSegBlock, q);
     }
     // the fewer than V elements left, by their number: a position past them
     // would wrap in a segment of nearly 2^32
     const uint32_t rest = llen - head - nv * V;
-    if (tid < rest) a1 = Acc::fold(a1, p[llen - rest + tid], lb + (llen - rest + tid));
-    A a = Acc::combine(a0, a1);
+    if (tid < rest) acc[1] = Acc::fold(acc[1], p[llen - rest + tid], lb + (llen - rest + tid));
+    A a = Acc::combine(Acc::combine(acc[0], acc[1]), Acc::combine(acc[2], acc[3]));
     a = Acc::wave_reduce(a);
     if (lane == 0) s_wave[wave] = a;
     __syncthreads();

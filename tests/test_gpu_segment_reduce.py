@@ -697,3 +697,35 @@ def test_longest_segments_off_a_16_byte_boundary(gpu, dtype):
             d[:4], d[-4:] = 0, 0
     del t
     torch.cuda.empty_cache()
+
+
+def _four_chain_sums(rows):
+    """Row sums of float32 `rows` as 256 threads of four float32 partial sums each give them, folded as a tree."""
+    S, L = rows.shape
+    x = np.zeros((S, -(-L // 1024) * 1024), np.float32)
+    x[:, :L] = rows
+    acc = np.zeros((S, 1024), np.float32)
+    for c in x.reshape(S, -1, 1024).swapaxes(0, 1):
+        acc += c
+    while acc.shape[1] > 1:
+        acc = acc[:, ::2] + acc[:, 1::2]
+    return acc[:, 0]
+
+
+@pytest.mark.parametrize("size,S", [(100_000, 512), (200_000, 512)])
+def test_long_segment_sums_keep_four_partial_sums(gpu, size, S):
+    """The error of a long float32 segment's sum grows with the length of a
+    thread's chain of additions: it is that of four partial sums per thread
+    (chains of half that number are 1.3-1.4 times as far off).  The bound is
+    that of the model, with 15 % for the spread of an rms over S sums
+    (1 / sqrt(2 S), 3 %) on either side."""
+    import gpu_util as g
+
+    rng = np.random.default_rng(size)
+    rows = rng.standard_normal((S, size), dtype=np.float32)
+    exact = rows.sum(axis=1, dtype=np.float64)
+    got = seg_call("Sum", g.to_dev(rows.ravel()), S, (size,), np.float32).astype(np.float64)
+    rms = np.sqrt(np.mean((got - exact) ** 2))
+    model = np.sqrt(np.mean((_four_chain_sums(rows).astype(np.float64) - exact) ** 2))
+    log(f"segment long sums size={size}: rms error {rms:.3g}, four chains {model:.3g}")
+    assert rms <= 1.15 * model
