@@ -1220,15 +1220,16 @@ int rs_run(void *temp, size_t temp_bytes, const void *kin_, void *kout_, const v
     const int ipt = os_ipt_for(n, sizeof(UK), VB);
     using Code = KeyCode<UK, KIND == kFloat>;
     // 8-byte keys: where the sampled cut goes.  With fewer passes the first of
-    // them may read the input and write the output, so outputs over the inputs
-    // sort every digit.
-    auto apart = [](const void *a, const void *b, uint64_t bytes) {
+    // them may read the inputs and write the outputs, so any output over any
+    // input sorts every digit.
+    auto apart = [](const void *a, uint64_t a_bytes, const void *b, uint64_t b_bytes) {
         const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
-        return x + bytes <= y || y + bytes <= x;
+        return x + a_bytes <= y || y + b_bytes <= x;
     };
+    const uint64_t kb = n * sizeof(UK), vb = n * sizeof(UV);
     uint32_t *cut = nullptr;
-    if (sizeof(UK) == 8 && n <= kTieMaxItems && apart(kin, kout, n * sizeof(UK)) &&
-        (!PAIRS || apart(vin, vout, n * sizeof(UV))))
+    if (sizeof(UK) == 8 && n <= kTieMaxItems && apart(kin, kb, kout, kb) &&
+        (!PAIRS || (apart(vin, vb, vout, vb) && apart(vin, vb, kout, kb) && apart(kin, kb, vout, vb))))
         cut = reinterpret_cast<uint32_t *>(t + L.hot_off) + 2 * L.passes + 1;
     int rc;
     if (ipt == kIptSmall)

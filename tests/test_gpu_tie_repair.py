@@ -91,6 +91,25 @@ def test_output_over_input(gpu):
     assert same_bits(g.to_host(dk), rk) and same_bits(g.to_host(dv), rv)
 
 
+@pytest.mark.parametrize("keys_over_values", [False, True])
+def test_output_over_the_other_input(gpu, keys_over_values):
+    """keys_out over vals_in, or vals_out over keys_in: uniform keys of this
+    number would take three passes, the first of them from the inputs to the
+    outputs."""
+    import gpu_util as g
+    from lc_parallel_primitive_amd import DeviceRadixSort
+
+    n = 100_003
+    k = np.random.default_rng(3).integers(0, 1 << 64, n, dtype=np.uint64)
+    v = np.arange(n, dtype=np.uint64) * 3
+    dk, dv, other = g.to_dev(k), g.to_dev(v), g.empty(n, np.uint64)
+    ko, vo = (dv, other) if keys_over_values else (other, dk)
+    tmp = g.temp(DeviceRadixSort.GetSortPairsTempStorageBytes("uint64", "uint64", n))
+    DeviceRadixSort().SortPairs(tmp, dk, ko, dv, vo, n)
+    rk, rv = o.radix_sort(k, v)
+    assert same_bits(g.to_host(ko), rk) and same_bits(g.to_host(vo), rv)
+
+
 def test_graph_replays(gpu):
     """A captured sort plans again for the keys of each replay."""
     import gpu_util as g
