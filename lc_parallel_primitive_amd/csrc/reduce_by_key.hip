@@ -23,9 +23,9 @@
 //      gathered in LDS and stored contiguously into the tile's slot of a
 //      dense staging area.  Runs of mean 128 give 64 per tile.
 //    - A tile with more heads, and every tile of an input of at most
-//      kRbkDirectTiles tiles, waits for the run count before it and the
-//      fold entering it (to the nearest tile with a head) and writes its runs
-//      to the outputs directly.  The run count is two-level: every tile adds
+//      kRbkDirectTiles tiles that no output overlaps, waits for the run count
+//      before it and the fold entering it (to the nearest tile with a head)
+//      and writes its runs to the outputs directly.  The run count is two-level: every tile adds
 //      its head count to its batch word (8 tiles) as it publishes, so a
 //      waiting tile sums its batch-mates' counts and walks the batch words
 //      back (whole batches add their totals) to batch 0 or to a batch whose
@@ -730,9 +730,12 @@ int rbk_launch(void *temp, size_t tb, const void *keys_, const void *in_, void *
     if (!temp || (reinterpret_cast<uintptr_t>(temp) & 255)) return LCPP_ERR_INVALID_ARG;
     const uint64_t kb = n * sizeof(K), vb = n * sizeof(V);
     const int vec_ok = ((reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(in)) & 15) == 0;
-    if (n <= bk_alone_max(true, vec_ok) && !bk_overlap(uk, kb, keys, kb) && !bk_overlap(uk, kb, in, vb) &&
-        !bk_overlap(agg, vb, keys, kb) && !bk_overlap(agg, vb, in, vb) && !bk_overlap(num_runs, 4, keys, kb) &&
-        !bk_overlap(num_runs, 4, in, vb)) {
+    // Outputs over an input: runs are staged until every tile has read its part
+    // (as far as they fit their slots).
+    const bool apart = !bk_overlap(uk, kb, keys, kb) && !bk_overlap(uk, kb, in, vb) && !bk_overlap(agg, vb, keys, kb) &&
+                       !bk_overlap(agg, vb, in, vb) && !bk_overlap(num_runs, 4, keys, kb) &&
+                       !bk_overlap(num_runs, 4, in, vb);
+    if (apart && n <= bk_alone_max(true, vec_ok)) {
         LCPP_LAUNCH("reduce_by_key_alone", s,
                     (rbk_alone_kernel<K, V, Op><<<(uint32_t)ceil_div(n, kBkAloneTile), kBkAloneBlock, 0, s>>>(
                         keys, in, (uint32_t)n, uk, agg, num_runs, vec_ok, static_cast<uint32_t *>(temp))));
@@ -754,7 +757,7 @@ int rbk_launch(void *temp, size_t tb, const void *keys_, const void *in_, void *
     if (lb_init(reinterpret_cast<uint64_t *>(t), L.count_off / 8, s, "reduce_by_key_init") != LCPP_OK)
         return LCPP_ERR_HIP;
     const WaitCtl ctl = wait_ctl(reinterpret_cast<uint32_t *>(t));
-    const int all_direct = L.tiles <= kRbkDirectTiles;
+    const int all_direct = apart && L.tiles <= kRbkDirectTiles;
     LCPP_LAUNCH("reduce_by_key_tile", s,
                 (rbk_tile_kernel<K, V, Op><<<(uint32_t)L.tiles, kBkBlock, 0, s>>>(
                     keys, in, (uint32_t)n, tile_count, tile_fold, pkeys, pvals, uk, agg, num_runs, tcwords, tvwords,

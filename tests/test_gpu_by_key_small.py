@@ -103,3 +103,27 @@ def test_reduce_by_key_where_staging_begins(gpu, kdt, vdt, tile, run, tiles, ext
     DeviceReduce().ReduceByKey(tmp, g.to_dev(k), g.to_dev(v), uo, ao, runs, "sum", n)
     assert g.to_host(runs)[0] == rk.size
     assert (g.to_host(uo)[:rk.size] == rk).all() and (g.to_host(ao)[:rk.size] == rv).all()
+
+
+@pytest.mark.parametrize("n", [3000, 40_000, 300_000])
+@pytest.mark.parametrize("ahead", [0, 64, 8192])
+def test_reduce_by_key_outputs_over_the_inputs(gpu, n, ahead):
+    """Outputs that start `ahead` elements into the inputs, long runs: every
+    tile has read its elements before a run is stored."""
+    import gpu_util as g
+    import torch
+    from lc_parallel_primitive_amd import DeviceReduce
+
+    k, v = keys_of(np.int32, n, 600, n), g.random_array(np.int32, n, seed=n)
+    rk, rv = o.reduce_by_key(k, v, o.OP_SUM)
+    assert rk.size <= n // 400  # fits the tiles' slots, and ends before the last key
+    bufs = [torch.empty(n + ahead, dtype=torch.int32, device="cuda") for _ in range(2)]
+    for b, a in zip(bufs, (k, v)):
+        b[:n].copy_(torch.from_numpy(a))
+    runs = g.empty(1, np.uint32)
+    tmp = g.temp(DeviceReduce.GetReduceByKeyTempStorageBytes("int32", "int32", n))
+    log(f"reduce by key over its inputs n={n} ahead={ahead}")
+    DeviceReduce().ReduceByKey(tmp, bufs[0][:n], bufs[1][:n], bufs[0][ahead:], bufs[1][ahead:], runs, "sum", n)
+    assert g.to_host(runs)[0] == rk.size
+    assert (g.to_host(bufs[0])[ahead:ahead + rk.size] == rk).all()
+    assert (g.to_host(bufs[1])[ahead:ahead + rk.size] == rv).all()
