@@ -72,6 +72,15 @@ constexpr int scan_vecs_for(uint64_t n)
 {
     return n <= kScanMidBytes / sizeof(T) ? kScanMidVecs : scan_vecs<T, INCLUSIVE>();
 }
+// An output over the input, but not in its place, may be written before a later
+// tile has read what it replaces, so only calls of one tile are safe: these take
+// the largest tile there is.
+template <class T>
+bool scan_shifted(const T *in, const T *out, uint64_t n)
+{
+    const uintptr_t i = reinterpret_cast<uintptr_t>(in), o = reinterpret_cast<uintptr_t>(out);
+    return i != o && i < o + n * sizeof(T) && o < i + n * sizeof(T);
+}
 
 // Temp layout: the status header, then packed look-back words, 8 bytes per
 // tile (32-bit T) or 16 bytes per tile (64-bit T).  The query covers the
@@ -316,14 +325,14 @@ int scan_run_dir(uint64_t *head, const T *in, T *out, uint64_t n, uint64_t tiles
     const WaitCtl ctl = wait_ctl(status);
     const uintptr_t ia = reinterpret_cast<uintptr_t>(in), oa = reinterpret_cast<uintptr_t>(out);
     const int vec_ok = ((ia | oa) & 15) == 0;
-    const uint64_t bytes = n * sizeof(T);
+    const bool shifted = scan_shifted(in, out, n);
     auto launch = [&](const char *name, auto go) {
         if (instrument) LCPP_LAUNCH(name, s, go());
         else go();
         return hipGetLastError() == hipSuccess;
     };
     const char *name = INCLUSIVE ? "scan_inclusive" : "scan_exclusive";
-    if (n <= kScanAloneBytes / sizeof(T) && (ia + bytes <= oa || oa + bytes <= ia)) {
+    if (n <= kScanAloneBytes / sizeof(T) && ia != oa && !shifted) {
         const uint32_t lead = (uint32_t)((16 - (ia & 15)) & 15) / (uint32_t)sizeof(T);
         const uint32_t grid = (uint32_t)ceil_div(n, (uint64_t)kAloneBlock * kAloneVecs * (16 / sizeof(T)));
         return launch(name, [&] {
@@ -336,14 +345,16 @@ int scan_run_dir(uint64_t *head, const T *in, T *out, uint64_t n, uint64_t tiles
     const uint64_t g = ceil_div(nwords, 256);
     if (!launch("scan_init", [&] { lb_init_kernel<<<(uint32_t)(g < 1024 ? g : 1024), 256, 0, s>>>(head, nwords); }))
         return LCPP_ERR_HIP;
-    const bool mid = scan_vecs_for<T, INCLUSIVE>(n) == kScanMidVecs;
+    const bool mid = scan_vecs_for<T, INCLUSIVE>(n) == kScanMidVecs && !shifted;
+    // (the large tiles are fewer: the words cover them)
+    const uint32_t grid = (uint32_t)(shifted ? ceil_div(n, scan_tile<T, scan_vecs<T, INCLUSIVE>()>()) : tiles);
     return launch(name, [&] {
                if (mid)
                    scan_kernel<T, INCLUSIVE, Op, kScanMidVecs>
-                       <<<(uint32_t)tiles, kScanBlock, 0, s>>>(in, out, n, words, vec_ok, init, ctl);
+                       <<<grid, kScanBlock, 0, s>>>(in, out, n, words, vec_ok, init, ctl);
                else
                    scan_kernel<T, INCLUSIVE, Op, scan_vecs<T, INCLUSIVE>()>
-                       <<<(uint32_t)tiles, kScanBlock, 0, s>>>(in, out, n, words, vec_ok, init, ctl);
+                       <<<grid, kScanBlock, 0, s>>>(in, out, n, words, vec_ok, init, ctl);
            })
                ? LCPP_OK
                : LCPP_ERR_HIP;

@@ -284,3 +284,27 @@ def test_sizes_where_the_path_changes(gpu, dtype, kib, in_place):
         d, out = g.to_dev(a), g.empty(n, dtype)
         DeviceScan().ExclusiveScan(tmp, d, out, n, "max", init)
         assert (g.to_host(out) == o.scan_op(a, False, o.OP_MAX, init)).all()
+
+
+@pytest.mark.parametrize("dtype,largest", [(np.uint32, (20_480, 16_384)), (np.float32, (20_480, 24_576)),
+                                           (np.int64, (10_240, 8192))])
+@pytest.mark.parametrize("shift", [1, 4, 4096, -1, -4096])
+def test_output_shifted_over_the_input(gpu, dtype, largest, shift):
+    """Scans of up to one (large) tile may write over their input at any
+    distance (offsets[1:] = InclusiveSum(counts) in one buffer): the tile is
+    read before it is written."""
+    import gpu_util as g
+    from lc_parallel_primitive_amd import DeviceScan
+
+    for inclusive in (False, True):
+        for n in (5000, largest[inclusive] - 1, largest[inclusive]):
+            a = np.arange(n, dtype=dtype) % 7  # float sums of small integers are exact
+            t = g.empty(n + abs(shift), dtype)
+            d, out = (t[:n], t[shift:]) if shift > 0 else (t[-shift:], t[:n])
+            d.copy_(g.to_dev(a))
+            tmp = g.temp(DeviceScan.GetTempStorageBytes(np.dtype(dtype).name, n))
+            log(f"scan {np.dtype(dtype).name} n={n} shift={shift}")
+            s = DeviceScan()
+            (s.InclusiveSum if inclusive else s.ExclusiveSum)(tmp, d, out, n)
+            want = np.cumsum(a, dtype=dtype) - (0 if inclusive else a)
+            assert (g.to_host(out) == want).all()
