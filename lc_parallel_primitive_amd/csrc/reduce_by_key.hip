@@ -72,12 +72,17 @@ constexpr uint32_t kRbkGlobal = 0x80000000u;
 constexpr uint32_t kRbkBwStride = 16;
 
 // Up to this many tiles every tile waits for its place and there is no emit
-// launch: they are all resident (four workgroups per CU), and a wait costs less
-// than another launch that moves the staged runs.  Measured (us per call, C
-// calls back to back, staged -> direct): int32 keys, f32 values, runs of 128: 2^20
+// launch: a wait costs less than another launch that moves the staged runs.
+// Two to four tiles of the kernel fit a CU (two with 8-byte keys and 4-byte
+// values), so 1024 are one or two generations.  Measured (us per call, calls
+// back to back, staged -> direct): int32 keys, f32 values, runs of 128: 2^20
 // 18.5 -> 12.8, 5 * 10^6 23.5 -> 18.4, 2^23 (1024 tiles) 26.9 -> 22.3, 2^24 39.0 ->
-// 40.4; runs of 4: 5 * 10^6 27.5 -> 21.7; int64, f64, runs of 1000: 2^21 19.5 ->
-// 13.9, 5 * 10^6 (1221 tiles) 26.7 -> 25.9, 2^24 55.4 -> 66.7.
+// 40.4; runs of 4: 5 * 10^6 27.5 -> 21.7; one run: 8 * 10^6 22.5 -> 17.9; int64,
+// f64, runs of 1000: 2^21 19.5 -> 13.9, 5 * 10^6 (1221 tiles) 26.7 -> 25.9, 2^24
+// 55.4 -> 66.7; one run: 4 * 10^6 22.1 -> 17.5; int64 keys, f32 values, 8 * 10^6:
+// runs of 128 35.5 -> 34.9, of 4 47.8 -> 43.2, one run 30.3 -> 29.0.  (One run with
+// every tile waiting for a fold, 16 predecessors polled at once and no tile's
+// inclusive fold published: 33.1, 37.0 and 50.5.)
 constexpr uint64_t kRbkDirectTiles = 1024;
 
 template <class K, class V>
@@ -340,16 +345,26 @@ __global__ __launch_bounds__(kBkBlock) void rbk_tile_kernel(const K *__restrict_
     // for the run count before the tile (wave 0) and the fold entering it (wave 1), then write the runs directly
     const bool direct = all_direct || sm.tc > kRbkSlot;
     if (direct) {
+        // a tile inside one run closes none: its count and fold go unused
+        const bool used = sm.tc > 0 || tile == gridDim.x - 1;
         if (wave == 0) {
-            const uint32_t p = tile > 0 ? rbk_count_before(tcwords, bwords, tile, ctl) : 0u;
+            const bool closes_batch = tile % kRbkBatch == kRbkBatch - 1;
+            const uint32_t p = tile > 0 && (used || closes_batch) ? rbk_count_before(tcwords, bwords, tile, ctl) : 0u;
             // the batch's last tile closes the batch's walk for later tiles
-            if (lane == 0 && tile % kRbkBatch == kRbkBatch - 1 && tile != ctl.withhold)
+            if (lane == 0 && closes_batch && tile != ctl.withhold)
                 __hip_atomic_fetch_add(&bwords[(tile / kRbkBatch) * kRbkBwStride],
                                        ((uint64_t)(p + sm.tc) << 32) | kRbkGlobal, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
             if (lane == 0) s_cpre = p;
         } else if (wave == 1) {
-            const V p = tile > 0 ? lb_wait_prefix(tvwords, tile, op, ident, ctl) : ident;
+            // every 64th tile publishes the fold up to its end, so that a walk
+            // along a run of many tiles is short
+            const bool closes_walk = all_direct && tile % kWave == kWave - 1 && !sm.tf;
+            V p = ident;
+            if (tile > 0 && (used || closes_walk))
+                p = all_direct ? lb_wait_prefix<kWave>(tvwords, tile, op, ident, ctl)
+                               : lb_wait_prefix(tvwords, tile, op, ident, ctl);
+            if (lane == 0 && closes_walk) lb_publish(tvwords, tile, op(p, sm.ts), kStInclusive, ctl);
             if (lane == 0) s_vpre = p;
         }
         __syncthreads();

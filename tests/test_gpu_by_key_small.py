@@ -127,3 +127,30 @@ def test_reduce_by_key_outputs_over_the_inputs(gpu, n, ahead):
     assert g.to_host(runs)[0] == rk.size
     assert (g.to_host(bufs[0])[ahead:ahead + rk.size] == rk).all()
     assert (g.to_host(bufs[1])[ahead:ahead + rk.size] == rv).all()
+
+
+@pytest.mark.parametrize("kdt,vdt", [(np.int32, np.int32), (np.int64, np.uint64)])
+@pytest.mark.parametrize("tiles", [9, 63, 64, 65, 128, 200, 1024, 1025])
+def test_reduce_by_key_runs_of_many_tiles(gpu, kdt, vdt, tiles):
+    """Tiles inside one run wait for nothing, and every 64th publishes the
+    fold up to its end: runs that span from a few tiles to all of them, on
+    both sides of the line to staged runs (1024 tiles)."""
+    import gpu_util as g
+    from lc_parallel_primitive_amd import DeviceReduce
+
+    tile = 32_768 // np.dtype(vdt).itemsize
+    kn, vn = np.dtype(kdt).name, np.dtype(vdt).name
+    for n in (tiles * tile, tiles * tile - tile + 1):
+        v = g.random_array(vdt, n, seed=n)
+        dv = g.to_dev(v)
+        for heads in ([], [n - 1], [tile * 5], [1, tile * 7 - 1, n // 2, n // 2 + 1], [n // 3]):
+            k = np.zeros(n, kdt)
+            k[[h for h in heads if h < n]] = 1
+            k = np.cumsum(k).astype(kdt)
+            log(f"reduce by key {kn} {vn} tiles={tiles} n={n} heads={heads}")
+            rk, rv = o.reduce_by_key(k, v, o.OP_SUM)
+            tmp = g.temp(DeviceReduce.GetReduceByKeyTempStorageBytes(kn, vn, n))
+            uo, ao, runs = g.empty(n, kdt), g.empty(n, vdt), g.empty(1, np.uint32)
+            DeviceReduce().ReduceByKey(tmp, g.to_dev(k), dv, uo, ao, runs, "sum", n)
+            assert g.to_host(runs)[0] == rk.size
+            assert (g.to_host(uo)[:rk.size] == rk).all() and (g.to_host(ao)[:rk.size] == rv).all()
