@@ -284,6 +284,14 @@ int lcpp_radix_sort_rank_path(int *path);
  * ranking, 2 = force the ballot-match ranking.  Calls running concurrently see the same
  * setting. */
 int lcpp_test_set_sort_rank_path(int mode);
+/* Test hooks.  lcpp_test_set_sort_cut, process-wide: -1 = sorts of 8-byte keys decide by the
+ * keys how many low digits get no pass and are left to the repair of ties (default), 0..7 =
+ * this many, whatever the keys (only slower for keys with long ties).  Sorts of up to 8192
+ * keys, of more than 2^28, and those with an output over an input always sort every digit.
+ * lcpp_test_sort_cut: the number that the last such sort with this temp storage left out
+ * (copies from the device and waits). */
+int lcpp_test_set_sort_cut(int digits);
+int lcpp_test_sort_cut(const void *temp, size_t temp_bytes, int *digits);
 
 /* ---------------------------------------------------------------------
  * DeviceSegmentReduce — device/device_segment_reduce.h

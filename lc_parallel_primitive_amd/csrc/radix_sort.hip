@@ -255,12 +255,33 @@ constexpr int kPlanSrcShift = 2, kPlanDstShift = 4, kPlanRegionShift = 6;
 constexpr uint32_t kPlanClearPrev = 1u << 8;  // zero region (k - 1) % 4 for pass k + 3
 constexpr int kLbRegions = 4;
 enum PlanBuf : uint32_t { kBufIn = 0, kBufTmp = 1, kBufOut = 2 };
+// How many of the `low` digits that the sample offers to leave out may be: so
+// many that some digit above them is spread evenly over all keys (`most`: the
+// count of each digit's most frequent value).  Keys that tie in every upper
+// digit share its values in each of them, so a run of ties is no longer than the
+// least of those counts, and where the other keys are spread evenly, no longer
+// than what that count has beyond its 256th: at most n / 4096 and the scatter of
+// even counts (8 standard deviations) are taken.  This is exact where the sample
+// is not: half of 2 * 10^6 u64 keys equal and the others uniform, or ten distinct
+// ones, met nothing in the sample, and one workgroup of the repair had the run
+// (2920 and 591 us, 7230 with rare keys beside the frequent one, where passes for
+// every digit take 162, 195 and 163).
+__device__ __forceinline__ uint32_t rs_cut_digits(uint32_t low, const uint32_t *most, uint32_t passes, uint64_t n)
+{
+    const uint64_t even = n / kRadix + n / 4096 + (uint64_t)(sqrtf((float)n) * 0.5f);
+    for (; low >= 2; --low)
+        for (uint32_t p = low; p < passes; ++p)
+            if (most[p] <= even) return low;
+    return 0;
+}
 // Runs in the histogram's last workgroup (NT threads), after the acquire that
 // pairs with every workgroup's release of its bin adds.
-// The lowest `low` digits get no pass.
+// cut (8-byte keys): in, the digits that the sample offers, out, those that get
+// no pass, and in cut[1] their bits.  force: this many instead (kCutByRule: none).
+constexpr uint32_t kCutByRule = ~0u;
 template <int NT>
 __device__ void rs_make_plan(const uint32_t *bins, uint32_t passes, uint64_t n, uint32_t *__restrict__ hot,
-                             uint32_t *__restrict__ plan, uint32_t *s_trivial, uint32_t low)
+                             uint32_t *__restrict__ plan, uint32_t *s_most, uint32_t *cut, uint32_t force)
 {
     const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
     for (uint32_t p = wave; p < passes; p += NT / kWave) {
@@ -279,16 +300,23 @@ __device__ void rs_make_plan(const uint32_t *bins, uint32_t passes, uint64_t n, 
         }
         if (lane == 0) {
             hot[p] = (best >> 8) * 16 >= n ? 255u - (uint32_t)(best & 255u) : (uint32_t)kRadix;
-            s_trivial[p] = (best >> 8) == n || p < low;
+            s_most[p] = (uint32_t)(best >> 8);
         }
     }
     __syncthreads();
     if (threadIdx.x == 0) {
+        uint32_t low = 0;
+        if (cut) {
+            low = force != kCutByRule ? force : rs_cut_digits(ld_relaxed(cut), s_most, passes, n);
+            cut[0] = low;
+            cut[1] = low * kRadixBits;
+        }
+        auto trivial = [&](uint32_t p) { return p < low || s_most[p] == n; };
         uint32_t m = 0;
-        for (uint32_t p = 0; p < passes; ++p) m += s_trivial[p] ? 0u : 1u;
+        for (uint32_t p = 0; p < passes; ++p) m += trivial(p) ? 0u : 1u;
         uint32_t k = 0, cur = kBufIn;
         for (uint32_t p = 0; p < passes; ++p) {
-            if (s_trivial[p]) {
+            if (trivial(p)) {
                 plan[p] = kPlanSkip | (p + 1 == passes && m == 0 ? kPlanCopy : 0u);
             } else {
                 const uint32_t dst = (m - 1 - k) % 2 == 0 ? kBufOut : kBufTmp;  // the last one writes the output
@@ -354,16 +382,16 @@ constexpr uint64_t hist_round_steps(uint64_t step, uint32_t cols) { return 65535
 // many of kSamples^2 / 2 pairs say that a key has count * n / (kSamples^2 / 2)
 // such neighbours on average; a quarter of one is taken: a repair with 0.7 of
 // them moves as many bytes as a pass (12 * 10^6 u64 -> u32 pairs: 75 against 61
-// us; with 0.003: 37).  (At most 64 meetings in any case, so that no single
-// group of tying keys can be large in a small input; and no more keys than the
-// upper bits have values, since few meetings say little about a large one.  Above
+// us; with 0.003: 37).  (At most 64 meetings in any case, and no more keys than
+// the upper bits have values, since few meetings say little about a large one.
+// Keys that equal the one they meet are none to repair and don't count.  Above
 // kTieMaxItems keys no meeting still allows runs of 32, and every digit gets its
 // pass.)  At least two digits must
 // go, since the repair reads all keys once more.  The keys are taken four at a
 // time, from a pseudo-random place of each of 1024 equal parts of the input (at
 // 4096 places the histogram launch of 10^6 keys waited for it: 25.8 us, now
 // 20.0).  The workgroup runs beside those that count.
-// cut[0] = the number of digits, cut[1] = of bits; both are zeroed before.
+// cut[0] = the number of digits, zeroed before (rs_cut_digits has the last word).
 constexpr uint32_t kSamples = 4096, kPlaceKeys = 4, kTable = 8192, kMeetings = 64;
 constexpr uint64_t kMeetingKeys = (uint64_t)kSamples * kSamples / 2 / 4;  // most meetings * n
 constexpr uint64_t kTieMaxItems = 1u << 28;
@@ -426,10 +454,7 @@ __device__ void rs_sample(const UK *__restrict__ keys, uint64_t n, const Code &c
             __syncthreads();
             const uint32_t total = s_acc[2];
             if (total <= kMeetings && total * n <= kMeetingKeys && n >> (64 - sh) == 0) {
-                if (tid == 0) {
-                    cut[0] = low;
-                    cut[1] = sh;
-                }
+                if (tid == 0) cut[0] = low;
                 return;
             }
             __syncthreads();
@@ -445,19 +470,19 @@ template <class UK, class Code, uint32_t CO, int kVecs>
 __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
     const UK *__restrict__ keys, uint64_t n, uint64_t chunk, Code code, uint32_t *bins, u32x4 *__restrict__ clear,
     uint64_t clear_vecs, uint32_t *arrivals, uint32_t *__restrict__ hot, uint32_t *__restrict__ plan,
-    uint32_t *cut)
+    uint32_t *cut, uint32_t force_cut)
 {
     constexpr int P = sizeof(UK);
     constexpr uint32_t W = (uint32_t)hist_table_words<UK>(CO);
-    extern __shared__ uint32_t s_hist[];  // the counter table, then s_last, s_trivial[16]
+    extern __shared__ uint32_t s_hist[];  // the counter table, then s_last, s_plan[16]
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = lane_id();
-    uint32_t *s_last = s_hist + W, *s_trivial = s_last + 1;
+    uint32_t *s_last = s_hist + W, *s_plan = s_last + 1;
     // where low digits may be left out, the last workgroup samples the keys
     const uint32_t counters = gridDim.x - (cut ? 1u : 0u);
     const bool counts = blockIdx.x < counters;
     if constexpr (sizeof(UK) == 8) {
-        if (!counts) rs_sample<UK>(keys, n, code, s_hist, s_trivial, cut);
+        if (!counts) rs_sample<UK>(keys, n, code, s_hist, s_plan, cut);
     }
     if (counts)
         for (uint32_t i = tid; i < W; i += kHistBlock) s_hist[i] = 0;
@@ -549,7 +574,7 @@ __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
     __syncthreads();
     if (*s_last) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        rs_make_plan<kHistBlock>(bins, (uint32_t)P, n, hot, plan, s_trivial, cut ? ld_relaxed(cut) : 0u);
+        rs_make_plan<kHistBlock>(bins, (uint32_t)P, n, hot, plan, s_plan, cut, force_cut);
     }
 }
 
@@ -1056,6 +1081,7 @@ namespace lcpp {
 namespace {
 
 std::atomic<int> g_rank_force{0};  // lcpp_test_set_sort_rank_path
+std::atomic<uint32_t> g_cut_force{kCutByRule};  // lcpp_test_set_sort_cut
 std::mutex g_probe_mu;
 DeviceCache g_rank_cache;
 
@@ -1185,7 +1211,8 @@ int rs_pipeline(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, cons
         LCPP_LAUNCH("rs_histogram", s,
                     (rs_histogram_kernel<UK, Code, CO, kVecs><<<(uint32_t)grid, kHistBlock, lds, s>>>(
                         buf.kin, n, chunk, code, bins, reinterpret_cast<u32x4 *>(t + L.tc_off),
-                        (L.ktmp_off - L.tc_off) / 16, plan + P, hot, plan, cut)));
+                        (L.ktmp_off - L.tc_off) / 16, plan + P, hot, plan, cut,
+                        g_cut_force.load(std::memory_order_relaxed))));
         LCPP_CHECK_LAUNCH();
     }
     const int path = rs_rank_path(s);
@@ -1372,6 +1399,25 @@ extern "C" int lcpp_test_set_sort_rank_path(int mode)
 {
     if (mode < 0 || mode > 2) return LCPP_ERR_INVALID_ARG;
     g_rank_force.store(mode, std::memory_order_relaxed);
+    return LCPP_OK;
+}
+
+extern "C" int lcpp_test_set_sort_cut(int digits)
+{
+    if (digits < -1 || digits > 7) return LCPP_ERR_INVALID_ARG;
+    g_cut_force.store(digits < 0 ? kCutByRule : (uint32_t)digits, std::memory_order_relaxed);
+    return LCPP_OK;
+}
+
+extern "C" int lcpp_test_sort_cut(const void *temp, size_t temp_bytes, int *digits)
+{
+    // 8-byte keys: the words lie at the same place whatever n and the values are
+    const RsLayout L = rs_layout(1, 8, 0);
+    if (!temp || !digits || temp_bytes < L.tc_off) return LCPP_ERR_INVALID_ARG;
+    uint32_t word = 0;
+    const char *cut = static_cast<const char *>(temp) + L.hot_off + (2 * L.passes + 1) * 4;
+    if (hipMemcpy(&word, cut, sizeof(word), hipMemcpyDeviceToHost) != hipSuccess) return LCPP_ERR_HIP;
+    *digits = (int)word;
     return LCPP_OK;
 }
 

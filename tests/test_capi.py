@@ -194,6 +194,9 @@ def test_device_status_decode_and_hooks(L):
     # the sort's rank-path override: 0 (probe), 1 (LDS atomics), 2 (ballot match)
     assert L.lcpp_test_set_sort_rank_path(3) == -1 and L.lcpp_test_set_sort_rank_path(-1) == -1
     assert L.lcpp_test_set_sort_rank_path(2) == 0 and L.lcpp_test_set_sort_rank_path(0) == 0
+    assert L.lcpp_test_set_sort_cut(8) == -1 and L.lcpp_test_set_sort_cut(-2) == -1
+    assert L.lcpp_test_set_sort_cut(7) == 0 and L.lcpp_test_set_sort_cut(-1) == 0
+    assert L.lcpp_test_sort_cut(None, 1 << 20, ctypes.byref(ctypes.c_int())) == -1
     assert L.lcpp_radix_sort_rank_path(None) == -1
     assert L.lcpp_temp_status_record(None, 0, None, None) == -1  # no destination
     dummy = ctypes.c_void_p(0x1000)

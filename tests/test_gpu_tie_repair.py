@@ -12,6 +12,97 @@ from test_gpu_small_sort import rank_path  # noqa: F401  (both ranking paths)
 pytestmark = pytest.mark.gpu
 
 
+def check(k, vdt, descending=False):
+    """Sorts k (with values of vdt, None: alone), compares with the oracle; the digits left out."""
+    import ctypes
+
+    import gpu_util as g
+    from lc_parallel_primitive_amd import DeviceRadixSort, lib
+
+    n, name = k.size, k.dtype.name
+    dk, ko, s = g.to_dev(k), g.empty(k.size, k.dtype), DeviceRadixSort()
+    if vdt is None:
+        tmp = g.temp(s.GetSortKeysTempStorageBytes(name, n))
+        (s.SortKeysDescending if descending else s.SortKeys)(tmp, dk, ko, n)
+        assert same_bits(g.to_host(ko), o.radix_sort(k, descending=descending, nthreads=8))
+    else:
+        v = np.arange(n).astype(vdt)
+        tmp = g.temp(s.GetSortPairsTempStorageBytes(name, np.dtype(vdt).name, n))
+        vo = g.empty(n, vdt)
+        (s.SortPairsDescending if descending else s.SortPairs)(tmp, dk, ko, g.to_dev(v), vo, n)
+        rk, rv = o.radix_sort(k, v, descending=descending, nthreads=8)
+        assert same_bits(g.to_host(ko), rk) and same_bits(g.to_host(vo), rv)
+    digits = ctypes.c_int(-1)
+    assert lib().lcpp_test_sort_cut(tmp.data_ptr(), tmp.numel(), ctypes.byref(digits)) == 0
+    return digits.value
+
+
+@pytest.mark.parametrize("n", [8193, 100_003, 2_000_003])
+def test_frequent_keys_sort_every_digit(gpu, n):
+    """Long runs of ties (one frequent key, few distinct ones, equal keys with
+    others of the same upper bits) leave no digit to the repair, where one
+    workgroup would have them; keys spread evenly do."""
+    rng = np.random.default_rng(n)
+    full = rng.integers(0, 1 << 64, n, dtype=np.uint64)
+    u = rng.random(n)
+    zeros = np.where(u < 0.5, np.uint64(0), full)
+    sentinels = np.where(u < 0.3, np.uint64(0), np.where(u > 0.999, np.uint64(1), full))
+    few = full[:10][rng.integers(0, 10, n)]
+    for name, k in (("zeros", zeros), ("sentinels", sentinels), ("few", few), ("floats", np.where(u < 0.5, 0.0, rng.standard_normal(n)))):
+        log(f"tie repair frequent {name} n={n}")
+        assert check(k, np.uint32) == 0, name
+    assert check(full, np.uint32) >= 4
+    assert check(rng.standard_normal(n), None) >= 3
+
+
+@pytest.fixture
+def set_cut(gpu):
+    import lc_parallel_primitive_amd as lcpp
+
+    yield lcpp.lib().lcpp_test_set_sort_cut
+    assert lcpp.lib().lcpp_test_set_sort_cut(-1) == 0
+
+
+def runs(n, sizes, digits, rng):
+    """n uint64 keys in a random order, groups of these sizes equal in the bits above `digits` digits."""
+    k = rng.integers(0, 1 << 64, n, dtype=np.uint64)
+    low = np.uint64((1 << 8 * digits) - 1)
+    at = 0
+    while True:
+        for size in sizes:
+            if at + size > n:
+                rng.shuffle(k)
+                return k
+            k[at:at + size] = (k[at] & ~low) | (k[at:at + size] & low)
+            at += size
+
+
+RUNS = {"pairs": [2, 1, 3], "short": [31, 32, 33, 34, 1], "in LDS": [64, 65, 1, 900, 2], "LDS edge": [2111, 2112, 2113],
+        "chunks": [1023, 4096, 1, 4097], "long": [20_001, 7]}
+
+
+@pytest.mark.parametrize("layout", RUNS)
+@pytest.mark.parametrize("vdt", [None, np.uint32, np.int64])
+def test_runs_of_every_length(set_cut, layout, vdt):
+    """Runs of ties at the lengths that the repair treats differently, differing
+    in two, three and five digits, whatever the rule would say to them."""
+    for digits in (2, 3, 5):
+        assert set_cut(digits) == 0
+        rng = np.random.default_rng(digits)
+        for n in (40_000, 100_003):
+            k = runs(n, RUNS[layout], digits, rng)
+            for descending in (False, True):
+                log(f"tie repair runs {layout} n={n} values={vdt} digits={digits} desc={descending}")
+                assert check(k, vdt, descending) == digits
+            kk = k.view(np.int64) if digits == 3 else np.where(np.isnan(k.view(np.float64)), 0.5, k.view(np.float64))
+            assert check(kk, vdt, digits == 5) == digits
+    # equal keys: runs in order already, and one key out of order in the longest
+    k = np.repeat(rng.integers(0, 1 << 64, 1 + 40_000 // 500, dtype=np.uint64), 500)[:40_000]
+    k[:20_000] = k[0] | np.uint64(1)
+    k[19_000] ^= np.uint64(1)
+    assert check(k, vdt) == 5
+
+
 def layouts(n, rng):
     """name -> n uint64 sort keys"""
     full = rng.integers(0, 1 << 64, n, dtype=np.uint64)
