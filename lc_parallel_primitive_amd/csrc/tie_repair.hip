@@ -8,22 +8,33 @@
 // upper digits, those that tie are few and lie side by side wherever the keys
 // are spread out (2^23.5 uniform keys: after the top 24 bits every second key
 // has a neighbour of equal upper bits, after the top 32 bits one in 360).  So
-// the sort stops after the digits that a sample of the keys asks for
-// (rs_sample_kernel, radix_sort.hip) and this kernel orders what
-// ties: one read of the keys, and writes where something moves.
+// the sort stops after the digits that a sample of the keys and the counts of
+// their digits ask for (rs_sample and rs_cut_digits in the histogram launch,
+// radix_sort.hip) and this kernel orders what ties: one read of the keys, and
+// writes where something moves.
 //  * A 256-thread workgroup owns the runs that begin in its 2048 keys; 64 more
-//    keys cover the runs that begin last.  Keys that tie with a neighbour are
-//    listed; each counts its place among its run in LDS (runs of up to 32 keys),
-//    and those that move are written with their values.
-//  * Longer runs are found to the end by the whole workgroup, skipped if in
-//    order already (equal keys are), ranked against each other in LDS up to
-//    2112 keys, and else sorted digit by digit between the output and the
-//    scratch, by the one workgroup, at a cost linear in their length.
+//    keys cover the runs that begin last.  One bit per key says whether a run
+//    begins there and one whether the key ranks below the one before it; with
+//    none of the latter every run is in order (equal keys are) and nothing is
+//    left to do.  Else the keys that tie with a neighbour are listed; those of a
+//    run of up to 32 keys that is not in order count their places in LDS, and
+//    those that move are written with their values.
+//  * The keys of longer runs that are not in order are ranked against each other
+//    by the whole workgroup.
+//  * A run that goes on past the 64 keys is followed to its end by the one
+//    workgroup, and if it is not in order ranked in LDS (up to 2112 keys) or
+//    sorted digit by digit between the output and the scratch, at a cost linear
+//    in its length: such a run of 30000 among 2^27 keys adds 390 us to a sort of
+//    3540.  rs_cut_digits bounds it: n / 256 keys at the most, and
+//    n / 4096 and the scatter of even counts where the other keys are spread
+//    evenly.
 // What bounds it is the read of the keys, and the writes of those that move: 12 *
 // 10^6 u64 keys with u32 values, us, after 32 / 24 upper bits: 37 / 75 (one
 // thread per run, by insertion in LDS: - / 93; every key looking for its place,
-// unlisted: - / 80).  The whole sort: 540 -> 315 us, of u64 keys alone 10^6:
-// 125 -> 78.
+// unlisted: - / 80).  The whole sort: 540 -> 305 us, of u64 keys alone 10^6:
+// 125 -> 78; keys that come ten times each 559 -> 330, 60 times 653 -> 304 (with
+// every key walking along its run, and the workgroup along each of more than 32:
+// 440 and 1135).
 // A neighbouring workgroup may read keys of a run while its owner moves them;
 // it looks at the upper bits alone, and those are the same wherever they go.
 #include "tie_repair.hpp"
@@ -34,21 +45,31 @@ namespace {
 constexpr int kTrBlock = 256;
 constexpr int kTrWaves = kTrBlock / kWave;
 constexpr uint32_t kTrTile = 2048, kTrHalo = 64, kTrCap = kTrTile + kTrHalo;
-constexpr uint32_t kTrShort = 32;  // longest run for one thread
+constexpr uint32_t kTrShort = 32;  // longest run whose keys find their places by themselves
 constexpr int kTrItems = (int)ceil_div(kTrCap, kTrBlock);
+constexpr int kTrWords = kTrItems * kTrWaves;  // bit words, of the 64 keys that a wave holds in one register
 constexpr int kTrRadixItems = 4;  // per thread and step of a run longer than kTrCap
-static_assert(kTrHalo > kTrShort, "a run that begins in the tile is known to its first 33 keys");
+constexpr int kTrFarLoads = 4;    // per thread and step along a run past the halo
+static_assert(kTrHalo > kTrShort, "a run that leaves the halo is longer than kTrShort");
 
 template <class UV, bool PAIRS, bool ZEROS>
 __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV *vals, uint64_t *ktmp, UV *vtmp,
                                                               uint32_t n, KeyCode<uint64_t, ZEROS> code,
                                                               const uint32_t *__restrict__ cut_word)
 {
-    __shared__ uint64_t sk[kTrCap];
+    // (the counters of a run sorted digit by digit lie where the keys were: 22
+    // KiB, seven workgroups per CU)
+    __shared__ union {
+        uint64_t key[kTrCap];
+        struct {
+            uint32_t wcnt[kTrWaves][256], dbase[256], wsum[kTrWaves];
+        } digit;
+    } sm;
     __shared__ uint16_t place[kTrCap];
-    __shared__ uint32_t longs[kTrTile / kTrShort];
-    __shared__ uint32_t nlong, nties, s_end, s_flag;
-    __shared__ uint32_t wcnt[kTrWaves][256], dbase[256], wsum[kTrWaves];
+    __shared__ uint64_t heads[kTrWords], downs[kTrWords];
+    __shared__ uint32_t longs[kTrTile / kTrShort];  // begin | end << 16
+    __shared__ uint32_t nlong, any_down, s_end, s_flag;
+    uint64_t *sk = sm.key;
 
     const uint32_t cut = __builtin_amdgcn_readfirstlane(*cut_word);
     if (cut == 0) return;
@@ -58,7 +79,7 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
     const uint32_t own = n - base < kTrTile ? n - base : kTrTile;  // those whose runs are this workgroup's
     auto top = [&](uint64_t t) { return code.ranked(t) >> cut; };
 
-    if (tid == 0) nlong = nties = 0;
+    if (tid == 0) nlong = any_down = 0;
     uint64_t k[kTrItems];
 #pragma unroll
     for (int u = 0; u < kTrItems; ++u) {
@@ -73,24 +94,50 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
     }
     __syncthreads();
 
-    // the keys that tie with a neighbour, listed
+    // bit i of heads: a run begins at key i (or i is past the last key); of
+    // downs: key i ties with the one before it and ranks below it.  (What key 0
+    // is to the one before it matters to that one's workgroup alone.)
 #pragma unroll
     for (int u = 0; u < kTrItems; ++u) {
-        const uint32_t i = tid + u * kTrBlock;
-        const uint64_t t = top(k[u]);
-        const uint64_t l = top(sk[i > 0 && i < m ? i - 1 : 0]), r = top(sk[i + 1 < m ? i + 1 : 0]);
-        const bool tie = i < m && ((i > 0 && l == t) || (i + 1 < m && r == t));
-        const uint64_t who = ballot(tie);
-        if (who == 0) continue;
-        uint32_t at = 0;
-        if (lane == 0) at = atomicAdd(&nties, (uint32_t)__builtin_popcountll(who));
-        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + mask_rank(who);
-        if (tie) place[at] = (uint16_t)i;
+        const uint32_t w = u * kTrWaves + wave, i = w * kWave + lane;
+        const uint64_t l = wave_shr1(k[u], sk[w > 0 && w * kWave < m ? w * kWave - 1 : 0]);
+        const bool head = i >= m || (i > 0 ? top(l) != top(k[u]) : base == 0 || before != top(k[u]));
+        const uint64_t hw = ballot(head);
+        const uint64_t dw = ballot(!head && i > 0 && code.ranked(l) > code.ranked(k[u]));
+        if (lane == 0) {
+            heads[w] = hw;
+            downs[w] = dw;
+            if (dw) any_down = 1;
+        }
     }
     __syncthreads();
-    // each finds its place in its run by itself: the keys to its left that do
-    // not rank above it and those to its right that rank below it
-    const uint32_t ties = nties;
+    // where the run of key i begins (~0u: before the tile)
+    auto begin_of = [&](uint32_t i) {
+        uint32_t w = i / kWave;
+        uint64_t x = heads[w] & (~0ull >> (kWave - 1 - i % kWave));
+        while (x == 0 && w > 0) x = heads[--w];
+        return x ? w * kWave + (uint32_t)(kWave - 1 - __builtin_clzll(x)) : ~0u;
+    };
+    // the run that holds the last key in LDS may go on
+    const uint32_t last = begin_of(m - 1);
+    const bool open = last < own && base + m < n;
+    if (!any_down && !open) return;  // every run is in order (the same for the whole workgroup)
+
+    // the keys that tie with a neighbour, listed: lane w counts those of word w
+    uint64_t tied = 0;
+    if (lane < (uint32_t)kTrWords)
+        tied = ~heads[lane] | ~heads[lane] >> 1 | (lane + 1 < (uint32_t)kTrWords ? ~heads[lane + 1] << (kWave - 1) : 0ull);
+    const uint32_t upto = wave_inclusive_scan((uint32_t)__builtin_popcountll(tied), SumOp());
+    const uint32_t ties = read_lane(upto, kWave - 1);
+#pragma unroll
+    for (int u = 0; u < kTrItems; ++u) {
+        const int w = __builtin_amdgcn_readfirstlane((int)(u * kTrWaves + wave));
+        const uint64_t who = read_lane(tied, w);
+        const uint32_t at = read_lane(upto, w) - (uint32_t)__builtin_popcountll(who) + mask_rank(who);
+        if (who >> lane & 1u) place[at] = (uint16_t)(w * kWave + lane);
+    }
+    __syncthreads();
+    // each key of a run that is not in order finds its place in it
     uint32_t to[kTrItems];
     UV v[PAIRS ? kTrItems : 1];
 #pragma unroll
@@ -99,30 +146,28 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
         const uint32_t q = tid + u * kTrBlock;
         if (q >= ties) continue;
         const uint32_t i = place[q];
-        k[u] = sk[i];
-        const uint64_t x = code.ranked(k[u]), t = x >> cut;
-        uint32_t left = 0, right = 0, r = 0;
-        while (left <= kTrShort && left < i) {
-            const uint64_t y = code.ranked(sk[i - 1 - left]);
-            if (y >> cut != t) break;
-            r += y <= x ? 1u : 0u;
-            ++left;
-        }
-        while (left + right <= kTrShort && i + 1 + right < m) {
-            const uint64_t y = code.ranked(sk[i + 1 + right]);
-            if (y >> cut != t) break;
-            r += y < x ? 1u : 0u;
-            ++right;
-        }
-        const uint32_t first = i - left;
-        // the run is another workgroup's, or goes to the whole workgroup
-        if (first >= own || (first == 0 && base && before == t)) continue;
-        if (left + 1 + right > kTrShort) {
-            if (left == 0) longs[atomicAdd(&nlong, 1u)] = base + i;
+        const uint32_t first = begin_of(i);
+        // the run is another workgroup's, or goes on past the halo
+        if (first >= own || (open && first == last)) continue;
+        uint32_t w = first / kWave;
+        uint64_t x = heads[w] & (~1ull << first % kWave), d = downs[w] & (~1ull << first % kWave), down = 0;
+        for (; x == 0; x = heads[++w], d = downs[w]) down |= d;
+        const uint32_t end = w * kWave + (uint32_t)__builtin_ctzll(x);  // (key m counts as a head)
+        down |= d & ~(~0ull << end % kWave);
+        if (down == 0) continue;
+        if (end - first > kTrShort) {
+            if (i == first) longs[atomicAdd(&nlong, 1u)] = first | end << 16;
             continue;
         }
-        if (r == left) continue;  // in its place
-        to[u] = first + r;
+        k[u] = sk[i];
+        const uint64_t rank = code.ranked(k[u]);
+        uint32_t r = first;
+        for (uint32_t j = first; j < end; ++j) {
+            const uint64_t y = code.ranked(sk[j]);
+            r += y < rank || (y == rank && j < i) ? 1u : 0u;
+        }
+        if (r == i) continue;  // in its place
+        to[u] = r;
         if constexpr (PAIRS) v[u] = vals[base + i];
     }
     __syncthreads();  // every key and value that moves has been read
@@ -133,69 +178,80 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
             if constexpr (PAIRS) vals[base + to[u]] = v[u];
         }
     }
-    __syncthreads();
 
+    // keys [b, b + L) of LDS, L <= kTrCap, which lie at keys[g], ranked against
+    // each other
+    auto rank_in_lds = [&](uint32_t b, uint32_t L, uint32_t g) {
+        if constexpr (PAIRS) {
+#pragma unroll
+            for (int u = 0; u < kTrItems; ++u) {
+                const uint32_t i = tid + u * kTrBlock;
+                if (i < L) v[u] = vals[g + i];
+            }
+            __syncthreads();  // every value has been read
+        }
+#pragma unroll
+        for (int u = 0; u < kTrItems; ++u) {
+            const uint32_t i = tid + u * kTrBlock;
+            if (i >= L) break;
+            const uint64_t t = sk[b + i], x = code.ranked(t);
+            uint32_t r = 0;
+            for (uint32_t j = 0; j < L; ++j) {
+                const uint64_t y = code.ranked(sk[b + j]);
+                r += y < x || (y == x && j < i) ? 1u : 0u;
+            }
+            keys[g + r] = code.out(t);
+            if constexpr (PAIRS) vals[g + r] = v[u];
+        }
+    };
     const uint32_t runs = nlong;
 #pragma unroll 1
     for (uint32_t q = 0; q < runs; ++q) {
-        const uint32_t g0 = longs[q];
-        const uint64_t t = top(code.in(keys[g0]));
+        const uint32_t b = longs[q] & 0xFFFFu;
+        rank_in_lds(b, (longs[q] >> 16) - b, base + b);
+    }
+
+    if (open) {
+        const uint32_t g0 = base + last;
+        const uint64_t t = top(sk[last]);
         // the first position past the run
-        uint32_t end = g0 + kTrShort + 1;
-        for (;; end += kTrBlock) {
+        uint32_t end = base + m;
+        for (;; end += kTrBlock * kTrFarLoads) {
             __syncthreads();
             if (tid == 0) s_end = ~0u;
             __syncthreads();
-            const uint64_t i = (uint64_t)end + tid;
-            if (i >= n || top(code.in(keys[i])) != t) atomicMin(&s_end, tid);
+            uint32_t past = ~0u;
+#pragma unroll
+            for (int u = kTrFarLoads - 1; u >= 0; --u) {
+                const uint32_t i = end + u * kTrBlock + tid;
+                if (i >= n || top(code.in(keys[i])) != t) past = u * kTrBlock + tid;
+            }
+            if (past != ~0u) atomicMin(&s_end, past);
             __syncthreads();
             if (s_end != ~0u) break;
         }
-        end = end + s_end < n ? end + s_end : n;
+        end += s_end;
         const uint32_t L = end - g0;
         __syncthreads();
         if (tid == 0) s_flag = 0;
         __syncthreads();
         bool down = false;
+#pragma unroll 4
         for (uint32_t i = tid; i + 1 < L; i += kTrBlock)
             down |= code.ranked(code.in(keys[g0 + i])) > code.ranked(code.in(keys[g0 + i + 1]));
         if (down) s_flag = 1;
         __syncthreads();
-        if (!s_flag) continue;  // the same for the whole workgroup
+        if (!s_flag) return;  // the same for the whole workgroup
         if (L <= kTrCap) {
             for (uint32_t i = tid; i < L; i += kTrBlock) sk[i] = code.in(keys[g0 + i]);
-            if constexpr (PAIRS) {
-#pragma unroll
-                for (int u = 0; u < kTrItems; ++u) {
-                    const uint32_t i = tid + u * kTrBlock;
-                    if (i < L) v[u] = vals[g0 + i];
-                }
-            }
             __syncthreads();
-            for (int u = 0; u < kTrItems; ++u) {
-                const uint32_t i = tid + u * kTrBlock;
-                if (i >= L) break;
-                const uint64_t x = code.ranked(sk[i]);
-                uint32_t r = 0;
-                for (uint32_t j = 0; j < L; ++j) {
-                    const uint64_t y = code.ranked(sk[j]);
-                    r += y < x || (y == x && j < i) ? 1u : 0u;
-                }
-                place[i] = (uint16_t)r;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < kTrItems; ++u) {
-                const uint32_t i = tid + u * kTrBlock;
-                if (i < L) {
-                    keys[g0 + place[i]] = code.out(sk[i]);
-                    if constexpr (PAIRS) vals[g0 + place[i]] = v[u];
-                }
-            }
-            continue;
+            rank_in_lds(0, L, g0);
+            return;
         }
         // digit by digit, kTrBlock * kTrRadixItems keys at a time (items of a
         // wave are consecutive: ranked by ballot match, stable)
+        auto &wcnt = sm.digit.wcnt;
+        uint32_t *dbase = sm.digit.dbase, *wsum = sm.digit.wsum;
         uint64_t *ka = keys + g0, *kb = ktmp + g0;
         UV *va = PAIRS ? vals + g0 : nullptr, *vb = PAIRS ? vtmp + g0 : nullptr;
 #pragma unroll 1
@@ -269,7 +325,6 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
                 if constexpr (PAIRS) vals[g0 + i] = va[i];
             }
         }
-        __syncthreads();
     }
 }
 
