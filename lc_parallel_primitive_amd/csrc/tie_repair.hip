@@ -24,8 +24,8 @@
 //  * A run that goes on past the 64 keys is followed to its end by the one
 //    workgroup, and if it is not in order ranked in LDS (up to 2112 keys) or
 //    sorted digit by digit between the output and the scratch, at a cost linear
-//    in its length: such a run of 30000 among 2^27 keys adds 390 us to a sort of
-//    3540.  rs_cut_digits bounds it: n / 256 keys at the most, and
+//    in its length: such a run of 30000 among 2^27 keys adds 420 us to a sort of
+//    3560.  rs_cut_digits bounds it: n / 256 keys at the most, and
 //    n / 4096 and the scatter of even counts where the other keys are spread
 //    evenly.
 // What bounds it is the read of the keys, and the writes of those that move: 12 *
@@ -50,36 +50,46 @@ constexpr int kTrItems = (int)ceil_div(kTrCap, kTrBlock);
 constexpr int kTrWords = kTrItems * kTrWaves;  // bit words, of the 64 keys that a wave holds in one register
 constexpr int kTrRadixItems = 4;  // per thread and step of a run longer than kTrCap
 constexpr int kTrFarLoads = 4;    // per thread and step along a run past the halo
+// Most workgroups launched per CU; beyond them each takes several tiles.  A sort
+// whose digits all have passes pays for this launch's empty workgroups (2^27 u64
+// keys of 16 low bits, u32 values: 1673 us with one per tile, 65536 of them, 1661
+// with 16384, 1659 with 8192), one that has ties to repair for tiles that
+// wait for each other (uniform keys: 3580 / 3578 / 3600; 7 per CU: 3874).
+constexpr uint32_t kTrPerCu = 64;
 static_assert(kTrHalo > kTrShort, "a run that leaves the halo is longer than kTrShort");
 
-template <class UV, bool PAIRS, bool ZEROS>
-__global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV *vals, uint64_t *ktmp, UV *vtmp,
-                                                              uint32_t n, KeyCode<uint64_t, ZEROS> code,
-                                                              const uint32_t *__restrict__ cut_word)
-{
-    // (the counters of a run sorted digit by digit lie where the keys were: 22
-    // KiB, seven workgroups per CU)
-    __shared__ union {
+// The LDS of a workgroup.  (The counters of a run sorted digit by digit lie where
+// the keys were: 22 KiB, seven workgroups per CU.)
+struct TrSmem {
+    union {
         uint64_t key[kTrCap];
         struct {
             uint32_t wcnt[kTrWaves][256], dbase[256], wsum[kTrWaves];
         } digit;
-    } sm;
-    __shared__ uint16_t place[kTrCap];
-    __shared__ uint64_t heads[kTrWords], downs[kTrWords];
-    __shared__ uint32_t longs[kTrTile / kTrShort];  // begin | end << 16
-    __shared__ uint32_t nlong, any_down, s_end, s_flag;
-    uint64_t *sk = sm.key;
+    };
+    uint16_t place[kTrCap];
+    uint64_t heads[kTrWords], downs[kTrWords];
+    uint32_t longs[kTrTile / kTrShort];  // begin | end << 16
+    uint32_t nlong, any_down, end, flag;
+};
 
-    const uint32_t cut = __builtin_amdgcn_readfirstlane(*cut_word);
-    if (cut == 0) return;
-    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
-    const uint32_t base = blockIdx.x * kTrTile;
+// The runs that begin in keys [base, base + kTrTile).  Every thread of the
+// workgroup calls it.
+template <class UV, bool PAIRS, bool ZEROS>
+__device__ __forceinline__ void tr_tile(uint64_t *keys, UV *vals, uint64_t *ktmp, UV *vtmp, uint32_t n,
+                                        const KeyCode<uint64_t, ZEROS> &code, uint32_t cut, uint32_t base, TrSmem &sm)
+{
+    uint64_t *sk = sm.key, *heads = sm.heads, *downs = sm.downs;
+    uint16_t *place = sm.place;
+    uint32_t tid = threadIdx.x;
+    // (opaque: what is computed from it is not kept in registers from tile to tile)
+    asm volatile("" : "+v"(tid));
+    const uint32_t lane = tid % kWave, wave = tid / kWave;
     const uint32_t m = n - base < kTrCap ? n - base : kTrCap;     // keys in LDS
     const uint32_t own = n - base < kTrTile ? n - base : kTrTile;  // those whose runs are this workgroup's
     auto top = [&](uint64_t t) { return code.ranked(t) >> cut; };
 
-    if (tid == 0) nlong = any_down = 0;
+    if (tid == 0) sm.nlong = sm.any_down = 0;
     uint64_t k[kTrItems];
 #pragma unroll
     for (int u = 0; u < kTrItems; ++u) {
@@ -107,7 +117,7 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
         if (lane == 0) {
             heads[w] = hw;
             downs[w] = dw;
-            if (dw) any_down = 1;
+            if (dw) sm.any_down = 1;
         }
     }
     __syncthreads();
@@ -121,7 +131,7 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
     // the run that holds the last key in LDS may go on
     const uint32_t last = begin_of(m - 1);
     const bool open = last < own && base + m < n;
-    if (!any_down && !open) return;  // every run is in order (the same for the whole workgroup)
+    if (!sm.any_down && !open) return;  // every run is in order (the same for the whole workgroup)
 
     // the keys that tie with a neighbour, listed: lane w counts those of word w
     uint64_t tied = 0;
@@ -156,7 +166,7 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
         down |= d & ~(~0ull << end % kWave);
         if (down == 0) continue;
         if (end - first > kTrShort) {
-            if (i == first) longs[atomicAdd(&nlong, 1u)] = first | end << 16;
+            if (i == first) sm.longs[atomicAdd(&sm.nlong, 1u)] = first | end << 16;
             continue;
         }
         k[u] = sk[i];
@@ -204,11 +214,11 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
             if constexpr (PAIRS) vals[g + r] = v[u];
         }
     };
-    const uint32_t runs = nlong;
+    const uint32_t runs = sm.nlong;
 #pragma unroll 1
     for (uint32_t q = 0; q < runs; ++q) {
-        const uint32_t b = longs[q] & 0xFFFFu;
-        rank_in_lds(b, (longs[q] >> 16) - b, base + b);
+        const uint32_t b = sm.longs[q] & 0xFFFFu;
+        rank_in_lds(b, (sm.longs[q] >> 16) - b, base + b);
     }
 
     if (open) {
@@ -218,7 +228,7 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
         uint32_t end = base + m;
         for (;; end += kTrBlock * kTrFarLoads) {
             __syncthreads();
-            if (tid == 0) s_end = ~0u;
+            if (tid == 0) sm.end = ~0u;
             __syncthreads();
             uint32_t past = ~0u;
 #pragma unroll
@@ -226,22 +236,22 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
                 const uint32_t i = end + u * kTrBlock + tid;
                 if (i >= n || top(code.in(keys[i])) != t) past = u * kTrBlock + tid;
             }
-            if (past != ~0u) atomicMin(&s_end, past);
+            if (past != ~0u) atomicMin(&sm.end, past);
             __syncthreads();
-            if (s_end != ~0u) break;
+            if (sm.end != ~0u) break;
         }
-        end += s_end;
+        end += sm.end;
         const uint32_t L = end - g0;
         __syncthreads();
-        if (tid == 0) s_flag = 0;
+        if (tid == 0) sm.flag = 0;
         __syncthreads();
         bool down = false;
 #pragma unroll 4
         for (uint32_t i = tid; i + 1 < L; i += kTrBlock)
             down |= code.ranked(code.in(keys[g0 + i])) > code.ranked(code.in(keys[g0 + i + 1]));
-        if (down) s_flag = 1;
+        if (down) sm.flag = 1;
         __syncthreads();
-        if (!s_flag) return;  // the same for the whole workgroup
+        if (!sm.flag) return;  // the same for the whole workgroup
         if (L <= kTrCap) {
             for (uint32_t i = tid; i < L; i += kTrBlock) sk[i] = code.in(keys[g0 + i]);
             __syncthreads();
@@ -258,18 +268,18 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
         for (uint32_t shift = 0; shift < cut; shift += 8) {
             __syncthreads();
             dbase[tid] = 0;
-            if (tid == 0) s_flag = 0;
+            if (tid == 0) sm.flag = 0;
             __syncthreads();
             for (uint32_t i = tid; i < L; i += kTrBlock) atomicAdd(&dbase[code.digit(code.in(ka[i]), shift)], 1u);
             __syncthreads();
             const uint32_t c = dbase[tid];
-            if (c == L) s_flag = 1;
+            if (c == L) sm.flag = 1;
             uint32_t ex = wave_inclusive_scan(c, SumOp());
             if (lane == kWave - 1) wsum[wave] = ex;
             ex -= c;
             __syncthreads();
             for (uint32_t w = 0; w < wave; ++w) ex += wsum[w];
-            const bool same = s_flag != 0;
+            const bool same = sm.flag != 0;
             dbase[tid] = ex;
             if (same) continue;  // one digit for all: nothing moves
             for (uint32_t s0 = 0; s0 < L; s0 += kTrBlock * kTrRadixItems) {
@@ -328,11 +338,26 @@ __global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV
     }
 }
 
+template <class UV, bool PAIRS, bool ZEROS>
+__global__ __launch_bounds__(kTrBlock) void tie_repair_kernel(uint64_t *keys, UV *vals, uint64_t *ktmp, UV *vtmp,
+                                                              uint32_t n, KeyCode<uint64_t, ZEROS> code,
+                                                              const uint32_t *__restrict__ cut_word)
+{
+    __shared__ TrSmem sm;
+    const uint32_t cut = __builtin_amdgcn_readfirstlane(*cut_word);
+    if (cut == 0) return;
+    for (uint64_t base = (uint64_t)blockIdx.x * kTrTile; base < n; base += (uint64_t)gridDim.x * kTrTile) {
+        tr_tile<UV, PAIRS>(keys, vals, ktmp, vtmp, n, code, cut, (uint32_t)base, sm);
+        __syncthreads();  // the LDS is free
+    }
+}
+
 template <class UV, bool PAIRS>
 int tr_run(int kind, bool desc, void *keys, void *vals, void *ktmp, void *vtmp, uint32_t n, const uint32_t *cut,
            hipStream_t s)
 {
-    const uint32_t grid = (uint32_t)ceil_div(n, kTrTile);
+    const uint32_t tiles = (uint32_t)ceil_div(n, kTrTile), most = kTrPerCu * (uint32_t)device_cus();
+    const uint32_t grid = (uint32_t)ceil_div(tiles, ceil_div(tiles, most));  // as many tiles for each
     auto go = [&](auto zeros) {
         constexpr bool Z = decltype(zeros)::value;
         LCPP_LAUNCH("rs_tie_repair", s,

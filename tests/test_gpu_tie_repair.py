@@ -221,3 +221,17 @@ def test_graph_replays(gpu):
         dk.copy_(torch.from_numpy(k))
         graph.replay()
         assert same_bits(g.to_host(ko), o.radix_sort(k)), name
+
+
+def test_several_tiles_per_workgroup(set_cut):
+    """More tiles than the repair launches workgroups (64 per CU): each takes
+    two, with runs at the tiles' edges."""
+    n = 64 * 256 * 2048 + 4097
+    rng = np.random.default_rng(5)
+    k = rng.integers(0, 1 << 64, n, dtype=np.uint64)
+    a, b = k[0:n - 2:3], k[1:n - 1:3]  # pairs
+    a[:] = (b & ~np.uint64(0xFFFFFFFF)) | (a & np.uint64(0xFFFFFFFF))
+    k[5_000_000:5_003_000] = (k[0] & ~np.uint64(0xFFFFFF)) | (k[5_000_000:5_003_000] & np.uint64(0xFFFFFF))
+    assert set_cut(4) == 0
+    log(f"tie repair several tiles n={n}")
+    assert check(k, np.uint32) == 4
