@@ -390,7 +390,10 @@ constexpr uint64_t hist_round_steps(uint64_t step, uint32_t cols) { return 65535
 // go, since the repair reads all keys once more.  The keys are taken four at a
 // time, from a pseudo-random place of each of 1024 equal parts of the input (at
 // 4096 places the histogram launch of 10^6 keys waited for it: 25.8 us, now
-// 20.0).  The workgroup runs beside those that count.
+// 20.0).  The workgroup runs beside those that count: it is the first, and where
+// each takes a whole CU they are one fewer than the CUs (with 256 of them the last
+// workgroup, whichever, began when another had ended: u64 keys alone, 2^24: 344
+// us, now 329; u64 -> u32 pairs, 2^22 139 and 131, 2^24 463 and 452).
 // cut[0] = the number of digits, zeroed before (rs_cut_digits has the last word).
 constexpr uint32_t kSamples = 4096, kPlaceKeys = 4, kTable = 8192, kMeetings = 64;
 constexpr uint64_t kMeetingKeys = (uint64_t)kSamples * kSamples / 2 / 4;  // most meetings * n
@@ -478,9 +481,10 @@ __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = lane_id();
     uint32_t *s_last = s_hist + W, *s_plan = s_last + 1;
-    // where low digits may be left out, the last workgroup samples the keys
-    const uint32_t counters = gridDim.x - (cut ? 1u : 0u);
-    const bool counts = blockIdx.x < counters;
+    // where low digits may be left out, the first workgroup samples the keys
+    const uint32_t samplers = cut ? 1u : 0u;
+    const uint32_t counters = gridDim.x - samplers, counter = blockIdx.x - samplers;
+    const bool counts = counter < counters;
     if constexpr (sizeof(UK) == 8) {
         if (!counts) rs_sample<UK>(keys, n, code, s_hist, s_plan, cut);
     }
@@ -492,7 +496,7 @@ __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
     // the stores go out beside the key stream instead of before it (2^28 u32
     // keys: 48 MiB of state).  The arrival's release below covers them.
     const uint64_t cshare = ceil_div(clear_vecs, (uint64_t)counters);
-    const uint64_t c0 = counts ? (uint64_t)blockIdx.x * cshare : clear_vecs;
+    const uint64_t c0 = counts ? (uint64_t)counter * cshare : clear_vecs;
     const uint64_t c1 = c0 + cshare < clear_vecs ? c0 + cshare : clear_vecs;
     uint64_t cnext = c0 + tid;
     auto clear_step = [&]() {
@@ -500,7 +504,7 @@ __global__ __launch_bounds__(kHistBlock) void rs_histogram_kernel(
         cnext += kHistBlock;
     };
 
-    const uint64_t b0 = counts ? (uint64_t)blockIdx.x * chunk : n;
+    const uint64_t b0 = counts ? (uint64_t)counter * chunk : n;
     const uint64_t b1 = b0 + chunk < n ? b0 + chunk : n;
     auto count = [&](UK raw) {
         const UK tk = code.in(raw);
@@ -1204,7 +1208,8 @@ int rs_pipeline(const RsBuffers<UK, UV> &buf, const Code &code, uint64_t n, cons
             return LCPP_ERR_HIP;
         const uint64_t htile = (uint64_t)kHistBlock * kVecs * (16 / sizeof(UK));
         const uint64_t htiles = ceil_div(n, htile);
-        const uint64_t cus = (uint64_t)device_cus() / (MID ? 2 : 1);
+        // (the sampling workgroup takes a CU of its own)
+        const uint64_t cus = (uint64_t)std::max(device_cus() / (MID ? 2 : 1) - (cut && !MID ? 1 : 0), 1);
         uint64_t grid = htiles < cus ? htiles : cus;
         const uint64_t chunk = ceil_div(htiles, grid) * htile;
         grid = ceil_div(n, chunk) + (cut ? 1 : 0);
