@@ -55,6 +55,15 @@ def test_frequent_keys_sort_every_digit(gpu, n):
     assert check(rng.standard_normal(n), None) >= 3
 
 
+def test_more_keys_than_upper_values_sort_every_digit(gpu):
+    """40-bit keys have 2^24 values above 16 bits: two digits are left out of a
+    tenth as many keys, none of half as many again, which nearly all tie."""
+    rng = np.random.default_rng(4)
+    for n, digits in ((1_600_000, 2), (25_000_000, 0)):
+        log(f"tie repair 40-bit keys n={n}")
+        assert check(rng.integers(0, 1 << 40, n, dtype=np.uint64), None) == digits
+
+
 @pytest.fixture
 def set_cut(gpu):
     import lc_parallel_primitive_amd as lcpp
