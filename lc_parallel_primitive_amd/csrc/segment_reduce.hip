@@ -72,6 +72,7 @@ constexpr int kSegPerWave = 64;  // at most (seg_split)
 constexpr uint32_t kSegLong = 8192;
 constexpr uint32_t kSegLongAlone = 2048;  // with one segment per workgroup
 constexpr uint32_t kNoIndex = 0xFFFFFFFFu;
+constexpr uint64_t kSegResident = 6;  // workgroups of segment_reduce_kernel that a CU holds (seg_split)
 
 enum SegOpKind { kSegSum = 0, kSegMin = 1, kSegMax = 2, kSegArgMin = 3, kSegArgMax = 4 };
 
@@ -714,30 +715,35 @@ int resident_blocks(K kernel, DeviceCache &cache)
 // How S segments are dealt out: segments per workgroup and per wave, and the
 // length from which the whole workgroup takes a segment.  A wave reads its
 // segments one 4 KiB chunk after the other, so what bounds a call with few
-// segments is how many waves they are spread over, whatever their lengths
-// (64 per wave at every S: 4096 segments of 1000 f32, ArgMax, kept 64 waves
-// busy for 73 us; 1024 segments of mean 16000 took 1340 us, one workgroup
-// reading up to 256 long ones in turn).  Measured, us per call (f32 Sum unless
-// named; lines in S, 256 CUs):
-//  * S < 4096, one segment per workgroup, the workgroup taking those over
-//    2048 elements: mean 16000, S = 1048: 20 (one per wave: 36); size 5000
-//    ArgMax, S = 3355: 17 (one per wave: 24).
-//  * from there one segment per wave for every 8192 segments, up to 8: mean
-//    1024, S = 16384: 15 (4 per wave: 29); size 1000 ArgMax, S = 67108: 45
-//    (64 per wave: 94); skewed, mean 4096, S = 16384: 56 (4 per wave: 90).
-//  * from 131072 on 32, from 262144 on 64: mean 128, S = 131072: 13.2 with
-//    32, 14.6 with 16; mean 37, S = 453438: 12.9 with 64, 14.4 with 32.
+// segments is how many waves they are spread over (64 per wave at every S: 4096
+// segments of 1000 f32, ArgMax, kept 64 waves busy for 73 us), but workgroups
+// beyond those that are resident at once wait for the first ones to end, 3 us
+// however short their segments are.  So the segments are spread over what is
+// resident and no more.  Fixed-size segments shorter than a chunk fill one first;
+// the lengths behind offsets are not known here.  Measured (us per call, device
+// time, f32 Sum; 64 per wave / this rule / up to three times as many workgroups):
+//  * mean 8: S = 1000 3.0 / 3.3 / 3.3, 4000 3.0 / 4.1 / 6.6, 30000 3.1 / 4.9 / 9.2,
+//    100000 3.4 / 5.2 / 8.3; of fixed size 8, 3.0 to 3.4 at any S here
+//  * mean 256: S = 4000 13.6 / 4.2 / 6.6, 30000 14.1 / 7.2 / 9.3, 100000 20 / 19 / 17
+//  * mean 1024: S = 4000 49 / 4.2 / 6.9, 30000 52 / 20 / 19, 65536 54 / 42 / 43
+//  * mean 4096: S = 4000 164 / 10 / 13, 30000 178 / 75 / 76; 16000, S = 1048: 1325 /
+//    12 / 12.
+// With one segment per workgroup, the workgroup takes those over 2048 elements
+// (mean 16000, S = 1048: 12; one per wave: 22).
 struct SegSplit {
     uint32_t per_wg, per_wave, long_len;
 };
-SegSplit seg_split(uint64_t S)
+// size: of every segment, 0 if not known; chunk: elements that a wave reads at a
+// time.
+SegSplit seg_split(uint64_t S, uint32_t size, uint32_t chunk)
 {
-    const uint64_t cus = (uint64_t)device_cus();
-    if (S < 16 * cus) return {1, 1, kSegLongAlone};
-    uint32_t per_wave = 1;
-    while (per_wave < 8 && S >= 2 * per_wave * cus * 32) per_wave *= 2;
-    if (S >= 512 * cus) per_wave = S >= 1024 * cus ? kSegPerWave : kSegPerWave / 2;
-    return {kSegWaves * per_wave, per_wave, kSegLong};
+    const uint64_t resident = kSegResident * (uint64_t)device_cus();
+    const uint64_t fill = size && size < chunk ? chunk / size : 1;
+    if (S <= resident && fill == 1) return {1, 1, kSegLongAlone};
+    const uint64_t even = ceil_div(S, resident * kSegWaves);
+    const uint64_t per_wave = even > fill ? even : fill;
+    if (per_wave > kSegPerWave / 2) return {kSegWaves * kSegPerWave, kSegPerWave, kSegLong};
+    return {(uint32_t)(kSegWaves * per_wave), (uint32_t)per_wave, kSegLong};
 }
 
 template <class T, int OP, bool FIXED>
@@ -765,7 +771,7 @@ int segment_launch(const void *in_, void *out_, uint32_t *index_out, uint64_t S,
         LCPP_CHECK_LAUNCH();
         return LCPP_OK;
     }
-    const SegSplit split = seg_split(S);
+    const SegSplit split = seg_split(S, FIXED ? sb.size : 0, kWave * flat_epl<T>());
     const uint32_t grid = (uint32_t)ceil_div(S, (uint64_t)split.per_wg);
     const int vec_ok = (reinterpret_cast<uintptr_t>(in) & 15) == 0;
     LCPP_LAUNCH("segment_reduce", s,

@@ -729,3 +729,35 @@ def test_long_segment_sums_keep_four_partial_sums(gpu, size, S):
     model = np.sqrt(np.mean((_four_chain_sums(rows).astype(np.float64) - exact) ** 2))
     log(f"segment long sums size={size}: rms error {rms:.3g}, four chains {model:.3g}")
     assert rms <= 1.15 * model
+
+
+@pytest.mark.parametrize("S", [1535, 1536, 1537, 6144, 6145, 12_289, 60_001, 196_609, 300_000])
+@pytest.mark.parametrize("dtype", [np.int32, np.float64])
+def test_segment_counts_where_the_split_changes(gpu, S, dtype):
+    """One segment per workgroup, one and more per wave: offsets of any order
+    with empty and long segments, and short fixed sizes, which fill a chunk."""
+    import gpu_util as g
+
+    rng = np.random.default_rng(S)
+    L = rng.geometric(1 / 20, S) - 1
+    L[::97] = rng.integers(0, 3000, L[::97].size)
+    L[S // 3] = 9000
+    n = int(L.sum()) + 5
+    e = np.cumsum(L)
+    p = rng.permutation(S) if S % 2 else np.arange(S)
+    b, e = (e - L)[p].astype(np.uint32), e[p].astype(np.uint32)
+    a = rng.integers(-40, 40, n).astype(dtype)  # float sums of small integers are exact
+    log(f"segment split S={S} {np.dtype(dtype).name}")
+    d = g.to_dev(a)
+    assert same(seg_call("Sum", d, S, (b, e), dtype), o.segment_reduce(o.OP_SUM, a, b, e))
+    v, i = seg_call("ArgMax", d, S, (b, e), dtype, arg=True)
+    ev, ei = o.segment_reduce_arg(True, a, b, e)
+    assert same(v, ev) and (i == ei).all()
+    for size in (1, 3, 16, 100, 513):
+        if size * S > 4_000_000:
+            continue
+        a = rng.integers(-40, 40, size * S).astype(dtype)
+        d, rows = g.to_dev(a), a.reshape(S, size)
+        assert same(seg_call("Sum", d, S, (size,), dtype), rows.sum(axis=1).astype(dtype)), size
+        v, i = seg_call("ArgMin", d, S, (size,), dtype, arg=True)
+        assert same(v, rows.min(axis=1)) and (i == rows.argmin(axis=1)).all(), size
