@@ -210,9 +210,10 @@ def test_reduce_by_key_sizes_ops_guard(gpu, n, op):
 @pytest.mark.parametrize("vdt", [np.int32, np.float64])
 @pytest.mark.parametrize("op", ["sum", "min", "max"])
 def test_reduce_by_key_across_emit_groups(gpu, vdt, op):
-    """Run counts and folds carried across the emit launch's groups of 64
-    tiles: dense runs (every tile's staging area nearly full), runs longer
-    than a group (whole groups without a head), and one run over everything."""
+    """Run counts and folds carried across 193 tiles, which all write their
+    runs directly (test_reduce_by_key_across_emit_groups_staged: with the
+    emit launch): dense runs, runs longer than 64 tiles, and one run over
+    everything."""
     tile = 8192 if np.dtype(vdt).itemsize == 4 else 4096
     n = 3 * 64 * tile + 4097
     for mean in (1.5, 1.5 * 64 * tile, float(n) * 10):
@@ -233,14 +234,14 @@ def test_reduce_by_key_across_emit_groups(gpu, vdt, op):
 
 @pytest.mark.parametrize("op", ["sum", "max"])
 def test_reduce_by_key_dense_and_sparse_tiles_mixed(gpu, op):
-    """Tiles with more than 128 runs (processed again from the input with
-    their prefixes) next to tiles that stage their runs: alternating regions
-    of runs of mean 2 and mean 500, a single dense tile, and a tile with
-    exactly 128 and 129 runs."""
+    """Dense tiles next to sparse ones: alternating regions of runs of mean 2
+    and mean 500, a single dense tile, and a tile with exactly 128 and 129
+    runs.  All write their runs directly at this size
+    (test_reduce_by_key_dense_and_sparse_tiles_staged: with staging)."""
     n = 40 * 8192 + 77
     rng = np.random.default_rng(11)
     mean = np.full(n, 500.0)
-    mean[3 * 8192:9 * 8192] = 2.0        # dense tiles, crossing emit groups? (64-tile groups: no)
+    mean[3 * 8192:9 * 8192] = 2.0        # dense tiles
     mean[20 * 8192:21 * 8192] = 1.0      # one all-distinct tile
     mean[30 * 8192 + 100:31 * 8192] = 3.0
     heads = rng.random(n) < 1.0 / mean
@@ -389,3 +390,52 @@ def test_at_the_32_bit_limit(gpu):
     assert bool((out[full:] == step[:127]).all())
     del dk, dv, out, tmp
     torch.cuda.empty_cache()
+
+
+# ReduceByKey stages runs and moves them with the emit launch (groups of 64
+# tiles) from 1025 tiles on
+@pytest.mark.parametrize("vdt,op", [(np.int32, "sum"), (np.int32, "min"), (np.float32, "sum"), (np.float32, "max"),
+                                    (np.float64, "sum"), (np.int64, "max")])
+def test_reduce_by_key_across_emit_groups_staged(gpu, vdt, op):
+    tile = 8192 if np.dtype(vdt).itemsize == 4 else 4096
+    n = (1024 + 2 * 64) * tile + 4097
+    for mean in (1.5, 300, 1.5 * 64 * tile, float(n) * 10):
+        keys = run_keys(n, mean, 8, np.int64)
+        v = values(vdt, n, 9)
+        log(f"ReduceByKey staged groups n={n} mean={mean:.0f} {np.dtype(vdt).name} {op}")
+        uk, ag, r = reduce_by_key(keys, v, op, guard=8)
+        ek, ea = o.reduce_by_key(keys, v, OPS[op])
+        assert r == ek.size
+        assert (uk[:r] == ek).all()
+        if np.dtype(vdt).kind == "f" and op == "sum":
+            s_, ab = o.reduce_by_key_f64(keys, v)
+            assert (np.abs(ag[:r] - s_) <= RTOL * ab + 1e-30).all()
+        else:
+            assert (ag[:r] == ea).all()
+        assert (uk[r:] == 0).all() and (ag[r:] == 0).all(), "write past the last run"
+
+
+@pytest.mark.parametrize("op", ["sum", "max"])
+def test_reduce_by_key_dense_and_sparse_tiles_staged(gpu, op):
+    """Tiles with more than 128 runs write them directly, the others stage
+    them: dense regions across and within groups, all-distinct tiles, tiles
+    with exactly 128 and 129 runs."""
+    n = 1100 * 8192 + 77
+    rng = np.random.default_rng(11)
+    mean = np.full(n, 500.0)
+    mean[60 * 8192:70 * 8192] = 2.0
+    mean[200 * 8192:201 * 8192] = 1.0
+    mean[1000 * 8192 + 100:1090 * 8192] = 3.0
+    heads = rng.random(n) < 1.0 / mean
+    heads[0] = True
+    for t, h in ((12, 128), (13, 129), (128, 128), (1099, 129)):
+        heads[t * 8192:(t + 1) * 8192] = False
+        heads[t * 8192 + rng.choice(8192, h, replace=False)] = True
+    keys = (np.cumsum(heads) * 3 % 65_521).astype(np.int32)
+    v = values(np.int32, n, 12)
+    log(f"ReduceByKey staged dense/sparse tiles {op}")
+    uk, ag, r = reduce_by_key(keys, v, op, guard=8)
+    ek, ea = o.reduce_by_key(keys, v, OPS[op])
+    assert r == ek.size
+    assert (uk[:r] == ek).all() and (ag[:r] == ea).all()
+    assert (uk[r:] == 0).all() and (ag[r:] == 0).all()

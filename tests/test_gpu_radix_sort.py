@@ -117,11 +117,10 @@ def test_pairs_stable_vs_oracle(gpu, kdt, vdt, n):
     assert same_bits(g.to_host(ko), rk) and same_bits(g.to_host(vo), rv)
 
 
-# Tiles hold 16384 keys (8192 when keys or values are 8 bytes) and the look-back
-# groups them in batches of 8: sizes around 1, 2, 3, 5, 8, 9 and 25 batches,
-# ragged and exact (a walk reads up to 8 batch words per poll in the kernels
-# at four waves per SIMD, so the walks from batch 8 on take the unguarded
-# window).
+# The look-back groups tiles in batches of 8: sizes around 1, 2, 3, 5, 8, 9 and 25
+# batches of the largest tiles (16384 keys, 8192 when keys or values are 8 bytes
+# or values ride along), ragged and exact.  Sorts of these sizes take smaller tiles
+# in part: test_lookback_batch_boundaries_by_tile has the batches of every tile.
 @pytest.mark.parametrize("kdt,vdt", [(np.uint32, None), (np.uint64, None), (np.uint32, np.uint32),
                                      (np.uint64, np.uint32)])
 @pytest.mark.parametrize("tiles,delta", [(7, 0), (8, -1), (8, 0), (8, 1), (9, 0), (16, 0), (17, 5),
@@ -142,6 +141,34 @@ def test_lookback_batch_boundaries(gpu, kdt, vdt, tiles, delta):
         ko, vo = sort_pairs(g.to_dev(k), g.to_dev(v), n, kdt, vdt)
         rk, rv = o.radix_sort(k, v)
         assert same_bits(g.to_host(ko), rk) and same_bits(g.to_host(vo), rv)
+
+
+# Tiles of 2048 keys up to 2^19, of 4096 up to 2^22 (4-byte keys alone) or 2^21 (with
+# 4-byte values), then the largest.  (A walk reads up to 8 batch words per poll, so
+# that from batch 8 on it takes the unguarded window.)
+@pytest.mark.parametrize("kdt,vdt,tile,counts", [
+    (np.uint32, None, 2048, (9, 64, 65, 72, 200, 256)), (np.uint32, None, 4096, (129, 136, 200, 513, 1024)),
+    (np.uint32, None, 16_384, (257, 264, 265, 328)), (np.uint32, np.uint32, 2048, (9, 16, 17, 72, 256)),
+    (np.uint32, np.uint32, 4096, (129, 136, 512)), (np.uint32, np.uint32, 8192, (257, 264, 328)),
+    (np.uint32, np.int64, 8192, (193, 200, 264)), (np.uint64, None, 2048, (5, 64, 65, 72, 256)),
+    (np.uint64, np.uint32, 2048, (5, 72, 256)), (np.uint64, np.uint32, 8192, (65, 72, 136)),
+])
+def test_lookback_batch_boundaries_by_tile(gpu, kdt, vdt, tile, counts):
+    import gpu_util as g
+
+    for tiles in counts:
+        for delta in (-3, 0, 1) if tiles * tile & (tiles * tile - 1) else (-3, 0):  # (a power of two: the line)
+            n = tiles * tile + delta
+            k = g.random_array(kdt, n, seed=tiles * 7 + delta)
+            log(f"sort batches of {tile} {np.dtype(kdt).name}/{vdt and np.dtype(vdt).name} n={n}")
+            if vdt is None:
+                assert same_bits(g.to_host(sort_keys(g.to_dev(k), n, kdt)), o.radix_sort(k, nthreads=8))
+            else:
+                k = k & np.array(0xFFF, dtype=kdt)  # duplicates: stability across tiles and batches
+                v = np.arange(n, dtype=vdt)
+                ko, vo = sort_pairs(g.to_dev(k), g.to_dev(v), n, kdt, vdt)
+                rk, rv = o.radix_sort(k, v, nthreads=8)
+                assert same_bits(g.to_host(ko), rk) and same_bits(g.to_host(vo), rv)
 
 
 @pytest.mark.parametrize("dtype", KEY_DTYPES)
@@ -232,17 +259,24 @@ def test_full_size_pairs_u64_index(gpu):
     assert o.check_stable_pairs_u64_u32(g.to_host(k), g.to_host(ko), g.to_host(vo))
 
 
-def test_full_size_pairs_u64_full_range_8_passes(gpu):
+@pytest.mark.parametrize("digits", [0, -1])
+def test_full_size_pairs_u64_full_range_8_passes(gpu, digits):
     # C4's shape with keys over the full 64-bit range: no digit pass is
-    # trivial, so all 8 onesweep passes move keys and values
+    # trivial, so all 8 onesweep passes move keys and values (and clear
+    # look-back regions inside them); -1: as it comes, with low digits left to
+    # the repair of ties
     import gpu_util as g
-    from lc_parallel_primitive_amd import datagen
+    from lc_parallel_primitive_amd import datagen, lib
 
     n = 1 << 27
-    log("sort pairs u64 (full range)/u32 2^27, 8 passes")
+    log(f"sort pairs u64 (full range)/u32 2^27, {8 if digits == 0 else 'fewer'} passes")
     k = datagen.keys_u64(n)
     v = datagen.iota_u32(n)
-    ko, vo = sort_pairs(k, v, n, np.uint64, np.uint32)
+    assert lib().lcpp_test_set_sort_cut(digits) == 0
+    try:
+        ko, vo = sort_pairs(k, v, n, np.uint64, np.uint32)
+    finally:
+        assert lib().lcpp_test_set_sort_cut(-1) == 0
     assert o.check_stable_pairs_u64_u32(g.to_host(k), g.to_host(ko), g.to_host(vo))
 
 

@@ -41,8 +41,10 @@ def test_kat_ones_reused_temp(gpu):
 
 
 @pytest.mark.parametrize("dtype", INT_DTYPES)
-# exclusive tiles hold 20480 32-bit / 10240 64-bit elements, inclusive ones 16384 /
-# 8192 (24576 for float): cover every boundary
+# the boundaries of the large tiles (exclusive 20480 32-bit / 10240 64-bit elements,
+# inclusive 16384 / 8192, 24576 for float), most of which the one-launch scan and
+# the 8192-element tiles take over at these sizes (test_large_tiles has the tiles
+# themselves)
 @pytest.mark.parametrize("n", [1, 2, 4097, 8191, 8192, 8193, 10239, 10240, 10241, 16383, 16384, 16385,
                                20479, 20480, 20481, 24575, 24576, 24577, 3 * 16384 + 5,
                                3 * 20480 + 5, 3 * 24576 + 5, 100_003, 1 << 20])
@@ -207,6 +209,38 @@ def test_scan_op_init_vs_oracle(gpu, dtype, op, n, pad):
             assert np.array_equal(got, o.scan_op(a, incl, SCAN_OPS[op], init)), kind
         else:
             assert got.tobytes() == o.scan_op(a, incl, SCAN_OPS[op], init).tobytes(), kind
+
+
+@pytest.mark.parametrize("dtype", ALL_DTYPES)
+@pytest.mark.parametrize("op", ["sum", "min", "max"])
+@pytest.mark.parametrize("extra", [1, 3 * 20_480 + 5])
+def test_large_tiles(gpu, dtype, op, extra):
+    """Inputs of more than 16 MiB: tiles of 16 to 24 vectors per thread, the
+    last one ragged, aligned and not; nothing is stored past the end."""
+    import gpu_util as g
+
+    n = (1 << 24) // np.dtype(dtype).itemsize + extra
+    a = g.random_array(dtype, n, seed=n + len(op))
+    init = op_init(dtype, op)
+    for pad in (0, 1):
+        log(f"scan large tiles op={op} {np.dtype(dtype).name} n={n} pad={pad}")
+        d = g.to_dev(a, pad=pad)
+        for kind, incl in (("ExclusiveScan", False), ("InclusiveScan", True)):
+            from lc_parallel_primitive_amd import DeviceScan
+
+            out = g.empty(n + 4096, dtype, pad=pad)
+            out[n:].fill_(77)
+            tmp = g.temp(DeviceScan.GetTempStorageBytes(np.dtype(dtype).name, n))
+            getattr(DeviceScan(), kind)(tmp, d, out, n, op, init)
+            got = g.to_host(out)
+            assert (got[n:] == 77).all(), "store past the end of the output"
+            got = got[:n]
+            if np.dtype(dtype).kind == "f" and op == "sum":
+                ref, ab = o.scan_f64(a, incl)
+                err = np.abs(got.astype(np.float64) - (ref + init))
+                assert (err <= RTOL_SCAN * (ab + abs(init)) + 1e-30).all(), kind
+            else:
+                assert np.array_equal(got, o.scan_op(a, incl, SCAN_OPS[op], init)), kind
 
 
 @pytest.mark.parametrize("kind", ["ExclusiveScan", "InclusiveScan"])

@@ -159,15 +159,14 @@ def test_by_key_withheld_tile_reports_timeout(gpu):
     assert status(t) == OK
     assert (g.to_host(out) == o.scan_by_key(keys, vals, inclusive=True)).all()
 
-    # ReduceByKey's look-back runs over groups of 64 tiles (its emit launch):
-    # withhold group 4 of 7
+    # 448 tiles that write their runs directly: withhold tile 4
     n = 7 * 64 * 8192 - 1000
     keys = (np.arange(n) // 97).astype(np.int32)
     vals = g.random_array(np.int32, n, seed=5)
     dk, dv = g.to_dev(keys), g.to_dev(vals)
     uk, agg, runs = g.empty(n, np.int32), g.empty(n, np.int32), g.empty(1, np.uint32)
     t = _temp(L.lcpp_reduce_by_key_temp_bytes, 0, 0, n)
-    log("status: reduce by key group 4 withheld")
+    log("status: reduce by key tile 4 withheld")
     with withheld(4):
         assert L.lcpp_reduce_by_key(0, 0, 0, _p(t), t.numel(), _p(dk), _p(dv), _p(uk), _p(agg), _p(runs), n,
                                     _sp()) == 0
@@ -201,6 +200,33 @@ def test_by_key_withheld_tile_reports_timeout(gpu):
         assert status(t) == OK
         r = int(g.to_host(runs)[0])
         assert r == n and (g.to_host(uk) == keys).all() and (g.to_host(agg) == vals).all()
+
+
+@pytest.mark.parametrize("tiles,run,tile", [(17 * 64, 97, 4), (17 * 64, 97, 15), (200, 1 << 30, 63), (200, 1 << 30, 150)])
+def test_reduce_by_key_withheld_group_or_fold(gpu, tiles, run, tile):
+    """Staged runs (more than 1024 tiles): the emit launch's look-back over
+    groups of 64 tiles, with group 4 or the last but one of 17 withheld.  One
+    run over tiles that write directly: the fold up to every 64th tile, with such
+    a tile or another withheld (the last tile waits for it)."""
+    import gpu_util as g
+
+    L = _L()
+    n = tiles * 8192 - 1000
+    keys = (np.arange(n) // run).astype(np.int32)
+    vals = g.random_array(np.int32, n, seed=5)
+    dk, dv = g.to_dev(keys), g.to_dev(vals)
+    uk, agg, runs = g.empty(n, np.int32), g.empty(n, np.int32), g.empty(1, np.uint32)
+    t = _temp(L.lcpp_reduce_by_key_temp_bytes, 0, 0, n)
+    log(f"status: reduce by key, {tiles} tiles, {tile} withheld")
+    args = (0, 0, 0, _p(t), t.numel(), _p(dk), _p(dv), _p(uk), _p(agg), _p(runs), n, _sp())
+    with withheld(tile):
+        assert L.lcpp_reduce_by_key(*args) == 0
+        assert status(t) == TIMEOUT
+    assert L.lcpp_reduce_by_key(*args) == 0
+    assert status(t) == OK
+    ek, ev = o.reduce_by_key(keys, vals)
+    r = int(g.to_host(runs)[0])
+    assert r == ek.size and (g.to_host(uk)[:r] == ek).all() and (g.to_host(agg)[:r] == ev).all()
 
 
 def test_status_cleared_by_every_primitive(gpu):

@@ -1,6 +1,6 @@
-"""Sorts of 8-byte keys that leave low digits to the repair of ties: keys whose
-upper bits tie in runs of every length that the repair treats differently, and
-keys that must be sorted digit by digit."""
+"""Sorts of 8-byte keys that leave low digits to the repair of ties: keys as they
+come, for which the sort decides how many digits that is, and, with the number
+forced, runs of ties of every length that the repair treats differently."""
 import numpy as np
 import pytest
 
@@ -116,7 +116,7 @@ def layouts(n, rng):
     """name -> n uint64 sort keys"""
     full = rng.integers(0, 1 << 64, n, dtype=np.uint64)
     out = {"uniform": full}
-    # groups of equal upper 40 bits: pairs, short runs, runs ranked in LDS (33..2112), longer ones
+    # groups of equal upper 40 bits, of every length: too many for a digit to be left out
     k = full.copy()
     at = 0
     for size in (2, 2, 3, 31, 32, 33, 34, 64, 65, 100, 257, 900, 2111, 2112, 2113, 4097, 6000):
