@@ -256,8 +256,8 @@ constexpr uint32_t kPlanClearPrev = 1u << 8;  // zero region (k - 1) % 4 for pas
 constexpr int kLbRegions = 4;
 enum PlanBuf : uint32_t { kBufIn = 0, kBufTmp = 1, kBufOut = 2 };
 // How many of the `low` digits that the sample offers to leave out may be: so
-// many that some digit above them is spread evenly over all keys (`most`: the
-// count of each digit's most frequent value).  Keys that tie in every upper
+// many that some digit above them is spread evenly over all keys (most[p]: the
+// count of digit p's most frequent value).  Keys that tie in every upper
 // digit share its values in each of them, so a run of ties is no longer than the
 // least of those counts, and where the other keys are spread evenly, no longer
 // than what that count has beyond its 256th: at most n / 4096 and the scatter of
@@ -266,13 +266,14 @@ enum PlanBuf : uint32_t { kBufIn = 0, kBufTmp = 1, kBufOut = 2 };
 // ones, met nothing in the sample, and one workgroup of the repair had the run
 // (2920 and 591 us, 7230 with rare keys beside the frequent one, where passes for
 // every digit take 162, 195 and 163).
-__device__ __forceinline__ uint32_t rs_cut_digits(uint32_t low, const uint32_t *most, uint32_t passes, uint64_t n)
+// (Lane p of a wave holds most[p], lanes past the digits anything; uniform.)
+__device__ __forceinline__ uint32_t rs_cut_digits(uint32_t low, uint32_t most, uint32_t passes, uint64_t n)
 {
     const uint64_t even = n / kRadix + n / 4096 + (uint64_t)(sqrtf((float)n) * 0.5f);
-    for (; low >= 2; --low)
-        for (uint32_t p = low; p < passes; ++p)
-            if (most[p] <= even) return low;
-    return 0;
+    const uint64_t spread = ballot(lane_id() < passes && most <= even);
+    const uint32_t top = spread ? (uint32_t)(kWave - 1 - __builtin_clzll(spread)) : 0u;  // the highest such digit
+    low = low < top ? low : top;
+    return low >= 2 ? low : 0u;
 }
 // Runs in the histogram's last workgroup (NT threads), after the acquire that
 // pairs with every workgroup's release of its bin adds.
@@ -284,6 +285,7 @@ __device__ void rs_make_plan(const uint32_t *bins, uint32_t passes, uint64_t n, 
                              uint32_t *__restrict__ plan, uint32_t *s_most, uint32_t *cut, uint32_t force)
 {
     const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
+    const uint32_t offer = cut ? ld_relaxed(cut) : 0u;
     for (uint32_t p = wave; p < passes; p += NT / kWave) {
         // lane l looks at digits l, l + 64, l + 128, l + 192
         uint64_t best = 0;  // (count << 8) | (255 - digit): max picks the larger count, then the smaller digit
@@ -304,27 +306,24 @@ __device__ void rs_make_plan(const uint32_t *bins, uint32_t passes, uint64_t n, 
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (wave == 0) {  // lane p: pass p
+        const bool pass = lane < passes;
+        const uint32_t most = pass ? s_most[lane] : 0u;
         uint32_t low = 0;
         if (cut) {
-            low = force != kCutByRule ? force : rs_cut_digits(ld_relaxed(cut), s_most, passes, n);
-            cut[0] = low;
-            cut[1] = low * kRadixBits;
+            low = force != kCutByRule ? force : rs_cut_digits(offer, most, passes, n);
+            if (lane < 2) cut[lane] = lane == 0 ? low : low * kRadixBits;
         }
-        auto trivial = [&](uint32_t p) { return p < low || s_most[p] == n; };
-        uint32_t m = 0;
-        for (uint32_t p = 0; p < passes; ++p) m += trivial(p) ? 0u : 1u;
-        uint32_t k = 0, cur = kBufIn;
-        for (uint32_t p = 0; p < passes; ++p) {
-            if (trivial(p)) {
-                plan[p] = kPlanSkip | (p + 1 == passes && m == 0 ? kPlanCopy : 0u);
-            } else {
-                const uint32_t dst = (m - 1 - k) % 2 == 0 ? kBufOut : kBufTmp;  // the last one writes the output
-                plan[p] = (cur << kPlanSrcShift) | (dst << kPlanDstShift) | ((k % kLbRegions) << kPlanRegionShift) |
-                          (k >= 1 && k + kLbRegions - 1 < m ? kPlanClearPrev : 0u);
-                cur = dst;
-                ++k;
-            }
+        const uint64_t moving = ballot(pass && lane >= low && most != n);
+        const uint32_t m = (uint32_t)__builtin_popcountll(moving), k = mask_rank(moving);
+        // the last one writes the output
+        auto written_by = [&](uint32_t j) { return (m - 1 - j) % 2 == 0 ? (uint32_t)kBufOut : (uint32_t)kBufTmp; };
+        if (pass) {
+            const bool moves = (moving >> lane & 1u) != 0;
+            plan[lane] = !moves ? kPlanSkip | (lane + 1 == passes && m == 0 ? kPlanCopy : 0u)
+                                : ((k ? written_by(k - 1) : (uint32_t)kBufIn) << kPlanSrcShift) |
+                                      (written_by(k) << kPlanDstShift) | ((k % kLbRegions) << kPlanRegionShift) |
+                                      (k >= 1 && k + kLbRegions - 1 < m ? kPlanClearPrev : 0u);
         }
     }
 }
