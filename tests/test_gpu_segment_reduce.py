@@ -713,10 +713,10 @@ def _four_chain_sums(rows):
 
 
 @pytest.mark.parametrize("size,S", [(100_000, 512), (200_000, 512)])
-def test_long_segment_sums_keep_four_partial_sums(gpu, size, S):
+def test_long_segment_sums_are_as_exact_as_four_partial_sums(gpu, size, S):
     """The error of a long float32 segment's sum grows with the length of a
-    thread's chain of additions: it is that of four partial sums per thread
-    (chains of half that number are 1.3-1.4 times as far off).  The bound is
+    thread's chain of additions: it is no more than that of four partial sums
+    per thread (two are 1.3-1.4 times as far off).  The bound is
     that of the model, with 15 % for the spread of an rms over S sums
     (1 / sqrt(2 S), 3 %) on either side."""
     import gpu_util as g
