@@ -649,7 +649,7 @@ __global__ __launch_bounds__(kSegBlock) __attribute__((amdgpu_waves_per_eu(6))) 
     const uint64_t wg_seg0 = (uint64_t)blockIdx.x * per_wg;
     const uint64_t wseg0 = wg_seg0 + (uint64_t)wave * spw;
     // lanes 0..spw-1 hold the bounds of the wave's segments (one coalesced
-    // load); with one segment per workgroup it is wave 0's
+    // load); with fewer segments than waves the first waves have one each
     const bool owner = wave * spw < per_wg;
     uint32_t b = 0, len = 0;
     if (owner && lane < spw) seg_bounds<FIXED>(sb, wseg0 + lane, S, b, len);
@@ -732,8 +732,9 @@ int resident_blocks(K kernel, DeviceCache &cache)
 //  * mean 1024: S = 4000 49 / 4.2 / 6.9, 30000 52 / 20 / 19, 65536 54 / 42 / 43
 //  * mean 4096: S = 4000 164 / 10 / 13, 30000 178 / 75 / 76; 16000, S = 1048: 1325 /
 //    12 / 12.
-// With one segment per workgroup, the workgroup takes those over 2048 elements
-// (mean 16000, S = 1048: 12; one per wave: 22).
+// One or two segments per workgroup: it takes those over 2048 elements itself
+// (mean 16000, S = 1048: 12; one per wave: 22; 30000, S = 2236: 42, four per
+// workgroup 45; three, size 5000, ArgMax, S = 3355: 18, four 13).
 struct SegSplit {
     uint32_t per_wg, per_wave, long_len;
 };
@@ -743,8 +744,11 @@ SegSplit seg_split(uint64_t S, uint32_t size, uint32_t chunk)
 {
     const uint64_t resident = kSegResident * (uint64_t)device_cus();
     const uint64_t fill = size && size < chunk ? chunk / size : 1;
-    if (S <= resident && fill == 1) return {1, 1, kSegLongAlone};
-    const uint64_t even = ceil_div(S, resident * kSegWaves);
+    const uint64_t per_wg = ceil_div(S, resident);
+    if (per_wg <= kSegWaves / 2 && fill == 1) return {(uint32_t)per_wg, 1, kSegLongAlone};
+    // two rounds of workgroups where each is known to last (size 1207, S = 39828,
+    // ArgMax: 33.4; one round 36.9)
+    const uint64_t even = ceil_div(S, resident * kSegWaves * (size >= chunk / 2 ? 2 : 1));
     const uint64_t per_wave = even > fill ? even : fill;
     if (per_wave > kSegPerWave / 2) return {kSegWaves * kSegPerWave, kSegPerWave, kSegLong};
     return {(uint32_t)(kSegWaves * per_wave), (uint32_t)per_wave, kSegLong};
