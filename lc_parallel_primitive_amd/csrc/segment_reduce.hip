@@ -43,6 +43,7 @@
 //    value max() (ArgMin) / lowest() (ArgMax).  The fold starts from the
 //    segment's own elements (no sentinel value takes part), so +-inf
 //    elements are found like any other.
+#include <algorithm>
 #include <cstring>
 
 #include "common.hpp"
@@ -70,9 +71,10 @@ constexpr int kSegWaves = kSegBlock / kWave;
 // (gathering the tiling layout: 104; with no segment lookup at all 96).
 constexpr int kSegPerWave = 64;  // at most (seg_split)
 constexpr uint32_t kSegLong = 8192;
-constexpr uint32_t kSegLongAlone = 2048;  // with one segment per workgroup
+constexpr uint32_t kSegLongAlone = 2048;  // with one or two segments per workgroup
 constexpr uint32_t kNoIndex = 0xFFFFFFFFu;
-constexpr uint64_t kSegResident = 6;  // workgroups of segment_reduce_kernel that a CU holds (seg_split)
+constexpr uint64_t kSegResident = 6;  // workgroups of segment_reduce_kernel that a CU holds
+constexpr uint64_t kSegMost = 13;     // and that are launched for it, at most (seg_split)
 
 enum SegOpKind { kSegSum = 0, kSegMin = 1, kSegMax = 2, kSegArgMin = 3, kSegArgMax = 4 };
 
@@ -720,21 +722,26 @@ int resident_blocks(K kernel, DeviceCache &cache)
 // length from which the whole workgroup takes a segment.  A wave reads its
 // segments one 4 KiB chunk after the other, so what bounds a call with few
 // segments is how many waves they are spread over (64 per wave at every S: 4096
-// segments of 1000 f32, ArgMax, kept 64 waves busy for 73 us), but workgroups
-// beyond those that are resident at once wait for the first ones to end, 3 us
-// however short their segments are.  So the segments are spread over what is
-// resident and no more.  Fixed-size segments shorter than a chunk fill one first;
-// the lengths behind offsets are not known here.  Measured (us per call, device
-// time, f32 Sum; 64 per wave / this rule / up to three times as many workgroups):
-//  * mean 8: S = 1000 3.0 / 3.3 / 3.3, 4000 3.0 / 4.1 / 6.6, 30000 3.1 / 4.9 / 9.2,
-//    100000 3.4 / 5.2 / 8.3; of fixed size 8, 3.0 to 3.4 at any S here
-//  * mean 256: S = 4000 13.6 / 4.2 / 6.6, 30000 14.1 / 7.2 / 9.3, 100000 20 / 19 / 17
-//  * mean 1024: S = 4000 49 / 4.2 / 6.9, 30000 52 / 20 / 19, 65536 54 / 42 / 43
-//  * mean 4096: S = 4000 164 / 10 / 13, 30000 178 / 75 / 76; 16000, S = 1048: 1325 /
-//    12 / 12.
+// segments of 1000 f32, ArgMax, kept 64 waves busy for 73 us), and how evenly
+// their lengths are; but workgroups beyond those that are resident at once wait
+// for the first ones to end, 3 us however short their segments are.  So there
+// are little more than two rounds of workgroups at most, one where the segments
+// are known to be short, and those of a fixed size fill a chunk first; the lengths
+// behind offsets are not known here.  With many segments lengths even out, and a
+// wave takes more of them.
+// Measured (us per call, device time, f32 Sum; 64 per wave / this rule / one round
+// / one segment per workgroup below S = 4096, up to 4096 workgroups above):
+//  * mean 8: S = 1000 3.0 / 3.3 / 3.3 / 3.3, 4000 3.0 / 5.2 / 4.1 / 6.6, 30000 3.1 / 6.9 /
+//    4.9 / 9.2, 100000 3.4 / 8.0 / 5.2 / 8.3; of fixed size 16, 2.9 to 3.3 at any S
+//  * mean 256: S = 4000 13.6 / 5.2 / 4.2 / 6.6, 30000 14.1 / 7.7 / 7.2 / 9.3
+//  * mean 1024: S = 30000 52 / 20 / 20 / 19, 65536 54 / 43 / 42 / 43
+//  * mean 4096: S = 4000 164 / 12 / 10 / 13, 30000 178 / 75 / 75 / 76
+//  * mean 2000, lengths over several powers of ten: S = 8810 350 / 21 / 27 / 22, 40000
+//    525 / 68 / 83 / 70, 120000 686 / 182 / 230 / 178.
 // One or two segments per workgroup: it takes those over 2048 elements itself
 // (mean 16000, S = 1048: 12; one per wave: 22; 30000, S = 2236: 42, four per
-// workgroup 45; three, size 5000, ArgMax, S = 3355: 18, four 13).
+// workgroup 45).  Above 1536 of a fixed size four are the better (size 5000,
+// ArgMax, S = 3355: 12.5, three 18).
 struct SegSplit {
     uint32_t per_wg, per_wave, long_len;
 };
@@ -742,14 +749,17 @@ struct SegSplit {
 // time.
 SegSplit seg_split(uint64_t S, uint32_t size, uint32_t chunk)
 {
-    const uint64_t resident = kSegResident * (uint64_t)device_cus();
+    const uint64_t cus = (uint64_t)device_cus(), resident = kSegResident * cus;
     const uint64_t fill = size && size < chunk ? chunk / size : 1;
-    const uint64_t per_wg = ceil_div(S, resident);
-    if (per_wg <= kSegWaves / 2 && fill == 1) return {(uint32_t)per_wg, 1, kSegLongAlone};
-    // two rounds of workgroups where each is known to last (size 1207, S = 39828,
-    // ArgMax: 33.4; one round 36.9)
-    const uint64_t even = ceil_div(S, resident * kSegWaves * (size >= chunk / 2 ? 2 : 1));
-    const uint64_t per_wave = even > fill ? even : fill;
+    if (fill == 1 && S <= resident) return {1, 1, kSegLongAlone};
+    if (!size && S < 16 * cus) return {2, 1, kSegLongAlone};
+    const bool small = size && size < chunk / 2;
+    uint64_t per_wave = 1;
+    if (!small) {
+        while (per_wave < 8 && S >= 2 * per_wave * cus * 32) per_wave *= 2;
+        if (S >= 512 * cus) per_wave = S >= 1024 * cus ? kSegPerWave : kSegPerWave / 2;
+    }
+    per_wave = std::max({per_wave, fill, ceil_div(S, (small ? resident : kSegMost * cus) * kSegWaves)});
     if (per_wave > kSegPerWave / 2) return {kSegWaves * kSegPerWave, kSegPerWave, kSegLong};
     return {(uint32_t)(kSegWaves * per_wave), (uint32_t)per_wave, kSegLong};
 }

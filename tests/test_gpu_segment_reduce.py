@@ -731,9 +731,9 @@ def test_long_segment_sums_are_as_exact_as_four_partial_sums(gpu, size, S):
     assert rms <= 1.15 * model
 
 
-@pytest.mark.parametrize("S", [1535, 1536, 1537, 6144, 6145, 12_289, 60_001, 196_609, 300_000])
+@pytest.mark.parametrize("S", [1535, 1536, 1537, 6144, 6145, 13_313, 60_001, 196_609, 300_000])
 @pytest.mark.parametrize("dtype", [np.int32, np.float64])
-def test_segment_counts_where_the_split_changes(gpu, S, dtype):
+def test_segment_counts_at_the_rounds_of_workgroups(gpu, S, dtype):
     """One segment per workgroup, one and more per wave: offsets of any order
     with empty and long segments, and short fixed sizes, which fill a chunk."""
     import gpu_util as g
