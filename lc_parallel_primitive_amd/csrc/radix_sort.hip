@@ -437,7 +437,7 @@ __device__ void rs_sample(const UK *__restrict__ keys, uint64_t n, const Code &c
     for (uint32_t p = 0; p < 5; ++p) vary += (diff >> (p * kRadixBits) & 255u) != 0;
     for (uint32_t low = 5; vary >= 2; --low) {
         const uint32_t sh = low * kRadixBits;
-        if (diff >> sh != 0) {  // else all of them tie
+        if (n >> __builtin_popcountll(diff >> sh) == 0) {  // else too many tie
             uint32_t met = 0;
 #pragma unroll
             for (uint32_t q = 0; q < kEach; ++q) {
@@ -458,7 +458,7 @@ __device__ void rs_sample(const UK *__restrict__ keys, uint64_t n, const Code &c
             if (lane_id() == 0 && met) atomicAdd(&s_acc[2], met);
             __syncthreads();
             const uint32_t total = s_acc[2];
-            if (total <= kMeetings && total * n <= kMeetingKeys && n >> __builtin_popcountll(diff >> sh) == 0) {
+            if (total <= kMeetings && total * n <= kMeetingKeys) {
                 if (tid == 0) cut[0] = low;
                 return;
             }
