@@ -67,7 +67,7 @@ struct TrSmem {
             uint32_t wcnt[kTrWaves][256], dbase[256], wsum[kTrWaves];
         } digit;
     };
-    uint16_t place[kTrCap];
+    uint16_t place[kTrWaves][kTrItems * kWave];
     uint64_t heads[kTrWords], downs[kTrWords];
     uint32_t longs[kTrTile / kTrShort];  // begin | end << 16
     uint32_t nlong, any_down, end, flag;
@@ -80,11 +80,11 @@ __device__ __forceinline__ void tr_tile(uint64_t *keys, UV *vals, uint64_t *ktmp
                                         const KeyCode<uint64_t, ZEROS> &code, uint32_t cut, uint32_t base, TrSmem &sm)
 {
     uint64_t *sk = sm.key, *heads = sm.heads, *downs = sm.downs;
-    uint16_t *place = sm.place;
     uint32_t tid = threadIdx.x;
     // (opaque: what is computed from it is not kept in registers from tile to tile)
     asm volatile("" : "+v"(tid));
     const uint32_t lane = tid % kWave, wave = tid / kWave;
+    uint16_t *place = sm.place[wave];
     const uint32_t m = n - base < kTrCap ? n - base : kTrCap;     // keys in LDS
     const uint32_t own = n - base < kTrTile ? n - base : kTrTile;  // those whose runs are this workgroup's
     auto top = [&](uint64_t t) { return code.ranked(t) >> cut; };
@@ -133,27 +133,29 @@ __device__ __forceinline__ void tr_tile(uint64_t *keys, UV *vals, uint64_t *ktmp
     const bool open = last < own && base + m < n;
     if (!sm.any_down && !open) return;  // every run is in order (the same for the whole workgroup)
 
-    // the keys that tie with a neighbour, listed: lane w counts those of word w
+    // the wave's keys that tie with a neighbour, listed: lane u counts those of its
+    // u-th word
     uint64_t tied = 0;
-    if (lane < (uint32_t)kTrWords)
-        tied = ~heads[lane] | ~heads[lane] >> 1 | (lane + 1 < (uint32_t)kTrWords ? ~heads[lane + 1] << (kWave - 1) : 0ull);
+    if (lane < (uint32_t)kTrItems) {
+        const uint32_t w = lane * kTrWaves + wave;
+        tied = ~heads[w] | ~heads[w] >> 1 | (w + 1 < (uint32_t)kTrWords ? ~heads[w + 1] << (kWave - 1) : 0ull);
+    }
     const uint32_t upto = wave_inclusive_scan((uint32_t)__builtin_popcountll(tied), SumOp());
     const uint32_t ties = read_lane(upto, kWave - 1);
 #pragma unroll
     for (int u = 0; u < kTrItems; ++u) {
-        const int w = __builtin_amdgcn_readfirstlane((int)(u * kTrWaves + wave));
-        const uint64_t who = read_lane(tied, w);
-        const uint32_t at = read_lane(upto, w) - (uint32_t)__builtin_popcountll(who) + mask_rank(who);
-        if (who >> lane & 1u) place[at] = (uint16_t)(w * kWave + lane);
+        const uint64_t who = read_lane(tied, u);
+        const uint32_t at = read_lane(upto, u) - (uint32_t)__builtin_popcountll(who) + mask_rank(who);
+        if (who >> lane & 1u) place[at] = (uint16_t)((u * kTrWaves + wave) * kWave + lane);
     }
-    __syncthreads();
+    wave_lds_sync();
     // each key of a run that is not in order finds its place in it
     uint32_t to[kTrItems];
     UV v[PAIRS ? kTrItems : 1];
 #pragma unroll
     for (int u = 0; u < kTrItems; ++u) {
         to[u] = ~0u;
-        const uint32_t q = tid + u * kTrBlock;
+        const uint32_t q = lane + u * kWave;
         if (q >= ties) continue;
         const uint32_t i = place[q];
         const uint32_t first = begin_of(i);
