@@ -70,8 +70,8 @@
 //    every key (from the histogram) is skipped, and the others ping-pong so
 //    that the last one writes the output.
 //  * 8-byte keys: digits that are not needed to tell nearly all keys apart (a
-//    sample says so) get no pass; a last launch orders the keys that tie in the
-//    others (tie_repair.hip).  Small sorts take one workgroup (small_sort.hip),
+//    sample offers them, the counts of all digits decide) get no pass; a last
+//    launch orders the keys that tie in the others (tie_repair.hip).  Small sorts take one workgroup (small_sort.hip),
 //    medium ones smaller tiles (os_ipt_for).
 //  * Descending order sorts the bit-inverted sort keys (one XOR in, one out,
 //    compiled only into the descending kernels), as RadixSortTwiddle<true>
