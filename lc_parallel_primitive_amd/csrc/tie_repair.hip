@@ -20,14 +20,14 @@
 //    run of up to 32 keys that is not in order count their places in LDS, and
 //    those that move are written with their values.
 //  * The keys of longer runs that are not in order are ranked against each other
-//    by the whole workgroup.
-//  * A run that goes on past the 64 keys is followed to its end by the one
-//    workgroup, and if it is not in order ranked in LDS (up to 2112 keys) or
-//    sorted digit by digit between the output and the scratch, at a cost linear
-//    in its length: such a run of 30000 among 2^27 keys adds 420 us to a sort of
-//    3560.  rs_cut_digits bounds it: n / 256 keys at the most, and
-//    n / 4096 and the scatter of even counts where the other keys are spread
-//    evenly.
+//    by the whole workgroup, up to 256 of them; more are sorted digit by digit
+//    between the output and the scratch, by the one workgroup, at a cost linear in
+//    their number.
+//  * A run that goes on past the 64 keys is followed to its end, and sorted by
+//    digits if it is not in order.  Such a run of 60000 among 2^27 keys, u32 values,
+//    adds 1270 us to a sort of 3530, one of 5000 among 12 * 10^6 170 to 300.
+//    rs_cut_digits bounds it: 1 / 227 of the keys at the most, and n / 2048 and the
+//    scatter of even counts where the other keys are spread evenly.
 // What bounds it is the read of the keys, and the writes of those that move: 12 *
 // 10^6 u64 keys with u32 values, us, after 32 / 24 upper bits: 37 / 75 (one
 // thread per run, by insertion in LDS: - / 93; every key looking for its place,
@@ -48,7 +48,14 @@ constexpr uint32_t kTrTile = 2048, kTrHalo = 64, kTrCap = kTrTile + kTrHalo;
 constexpr uint32_t kTrShort = 32;  // longest run whose keys find their places by themselves
 constexpr int kTrItems = (int)ceil_div(kTrCap, kTrBlock);
 constexpr int kTrWords = kTrItems * kTrWaves;  // bit words, of the 64 keys that a wave holds in one register
-constexpr int kTrRadixItems = 4;  // per thread and step of a run longer than kTrCap
+// Longest run that the workgroup ranks (L * L / 256 steps of 35 ns); longer ones, and
+// those that go on past the halo, are sorted digit by digit (some 40 us, mostly
+// beside other workgroups' tiles).  A sort with one run of L among uniform keys, us,
+// ranked / by digits: 10^6 u64, L = 300 100 / 90, 600 140 / 92 (79 without); 12 * 10^6
+// u64 -> u32 pairs, L = 600 382 / 334, 2100 947 / 340 (300 without).
+constexpr uint32_t kTrRanked = 256;
+constexpr int kTrRankedItems = kTrRanked / kTrBlock;
+constexpr int kTrRadixItems = 4;  // per thread and step of a run sorted by digits
 constexpr int kTrFarLoads = 4;    // per thread and step along a run past the halo
 // Most workgroups launched per CU; beyond them each takes several tiles.  A sort
 // whose digits all have passes pays for this launch's empty workgroups (2^27 u64
@@ -72,6 +79,94 @@ struct TrSmem {
     uint32_t longs[kTrTile / kTrShort];  // begin | end << 16
     uint32_t nlong, any_down, end, flag;
 };
+
+// Keys [0, L), which tie from bit `cut` on, sorted by the bits below, stably,
+// between `keys` and `ktmp`; vals move along.  Every thread of the workgroup calls
+// it.
+template <class UV, bool PAIRS, bool ZEROS>
+__device__ __forceinline__ void tr_by_digits(uint64_t *keys, UV *vals, uint64_t *ktmp, UV *vtmp, uint32_t L,
+                                             const KeyCode<uint64_t, ZEROS> &code, uint32_t cut, uint32_t tid,
+                                             TrSmem &sm)
+{
+    const uint32_t lane = tid % kWave, wave = tid / kWave;
+    // kTrBlock * kTrRadixItems keys at a time (items of a wave are consecutive:
+    // ranked by ballot match, stable)
+    auto &wcnt = sm.digit.wcnt;
+    uint32_t *dbase = sm.digit.dbase, *wsum = sm.digit.wsum;
+    uint64_t *ka = keys, *kb = ktmp;
+    UV *va = vals, *vb = vtmp;
+#pragma unroll 1
+    for (uint32_t shift = 0; shift < cut; shift += 8) {
+        __syncthreads();
+        dbase[tid] = 0;
+        if (tid == 0) sm.flag = 0;
+        __syncthreads();
+        for (uint32_t i = tid; i < L; i += kTrBlock) atomicAdd(&dbase[code.digit(code.in(ka[i]), shift)], 1u);
+        __syncthreads();
+        const uint32_t c = dbase[tid];
+        if (c == L) sm.flag = 1;
+        uint32_t ex = wave_inclusive_scan(c, SumOp());
+        if (lane == kWave - 1) wsum[wave] = ex;
+        ex -= c;
+        __syncthreads();
+        for (uint32_t w = 0; w < wave; ++w) ex += wsum[w];
+        const bool same = sm.flag != 0;
+        dbase[tid] = ex;
+        if (same) continue;  // one digit for all: nothing moves
+        for (uint32_t s0 = 0; s0 < L; s0 += kTrBlock * kTrRadixItems) {
+            for (uint32_t i = tid; i < kTrWaves * 256u; i += kTrBlock) (&wcnt[0][0])[i] = 0;
+            __syncthreads();
+            uint64_t kk[kTrRadixItems];
+            UV w[kTrRadixItems];
+            uint32_t r[kTrRadixItems], d[kTrRadixItems];
+            const uint32_t p = s0 + wave * (kWave * kTrRadixItems) + lane;
+#pragma unroll
+            for (int u = 0; u < kTrRadixItems; ++u) {
+                const bool ok = p + u * kWave < L;
+                kk[u] = ok ? ka[p + u * kWave] : 0;
+                if constexpr (PAIRS) w[u] = ok ? va[p + u * kWave] : UV(0);
+                d[u] = code.digit(code.in(kk[u]), shift);
+                const uint64_t peers = match_any8(d[u]) & ballot(ok);
+                const uint32_t below = mask_rank(peers);
+                uint32_t b = 0;
+                if (ok && below == 0) b = atomicAdd(&wcnt[wave][d[u]], (uint32_t)__builtin_popcountll(peers));
+                r[u] = (uint32_t)__shfl((int)b, ok ? (int)__builtin_ctzll(peers) : 0) + below;
+            }
+            __syncthreads();
+            uint32_t at = dbase[tid];
+#pragma unroll
+            for (int x = 0; x < kTrWaves; ++x) {
+                const uint32_t cc = wcnt[x][tid];
+                wcnt[x][tid] = at;
+                at += cc;
+            }
+            dbase[tid] = at;
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < kTrRadixItems; ++u) {
+                if (p + u * kWave < L) {
+                    const uint32_t at = wcnt[wave][d[u]] + r[u];
+                    kb[at] = kk[u];
+                    if constexpr (PAIRS) vb[at] = w[u];
+                }
+            }
+            __syncthreads();
+        }
+        uint64_t *kx = ka;
+        ka = kb;
+        kb = kx;
+        UV *vx = va;
+        va = vb;
+        vb = vx;
+    }
+    __syncthreads();
+    if (ka != keys) {
+        for (uint32_t i = tid; i < L; i += kTrBlock) {
+            keys[i] = ka[i];
+            if constexpr (PAIRS) vals[i] = va[i];
+        }
+    }
+}
 
 // The runs that begin in keys [base, base + kTrTile).  Every thread of the
 // workgroup calls it.
@@ -191,152 +286,84 @@ __device__ __forceinline__ void tr_tile(uint64_t *keys, UV *vals, uint64_t *ktmp
         }
     }
 
-    // keys [b, b + L) of LDS, L <= kTrCap, which lie at keys[g], ranked against
-    // each other
-    auto rank_in_lds = [&](uint32_t b, uint32_t L, uint32_t g) {
+    // the longer ones, one after the other
+    const uint32_t runs = sm.nlong;
+    const uint64_t open_top = top(sk[last < m ? last : 0]);
+    uint16_t *rank = &sm.place[0][0];
+#pragma unroll 1
+    for (uint32_t q = 0; q < runs; ++q) {
+        const uint32_t b = sm.longs[q] & 0xFFFFu, L = (sm.longs[q] >> 16) - b, g = base + b;
+        if (L > kTrRanked) continue;
+        __syncthreads();  // `rank` is free
+        // each key counts those that go before it
+#pragma unroll 1
+        for (uint32_t i = tid; i < L; i += kTrBlock) {
+            const uint64_t x = code.ranked(sk[b + i]);
+            uint32_t r = 0;
+#pragma unroll 4
+            for (uint32_t j = 0; j < L; ++j) {
+                const uint64_t y = code.ranked(sk[b + j]);
+                r += y < x || (y == x && j < i) ? 1u : 0u;
+            }
+            rank[i] = (uint16_t)r;
+        }
         if constexpr (PAIRS) {
 #pragma unroll
-            for (int u = 0; u < kTrItems; ++u) {
+            for (int u = 0; u < kTrRankedItems; ++u) {
                 const uint32_t i = tid + u * kTrBlock;
                 if (i < L) v[u] = vals[g + i];
             }
             __syncthreads();  // every value has been read
         }
 #pragma unroll
-        for (int u = 0; u < kTrItems; ++u) {
+        for (int u = 0; u < kTrRankedItems; ++u) {
             const uint32_t i = tid + u * kTrBlock;
-            if (i >= L) break;
-            const uint64_t t = sk[b + i], x = code.ranked(t);
-            uint32_t r = 0;
-            for (uint32_t j = 0; j < L; ++j) {
-                const uint64_t y = code.ranked(sk[b + j]);
-                r += y < x || (y == x && j < i) ? 1u : 0u;
+            if (i < L) {  // (a thread reads the ranks that it wrote)
+                keys[g + rank[i]] = code.out(sk[b + i]);
+                if constexpr (PAIRS) vals[g + rank[i]] = v[u];
             }
-            keys[g + r] = code.out(t);
-            if constexpr (PAIRS) vals[g + r] = v[u];
         }
-    };
-    const uint32_t runs = sm.nlong;
-#pragma unroll 1
-    for (uint32_t q = 0; q < runs; ++q) {
-        const uint32_t b = sm.longs[q] & 0xFFFFu;
-        rank_in_lds(b, (sm.longs[q] >> 16) - b, base + b);
     }
-
-    if (open) {
-        const uint32_t g0 = base + last;
-        const uint64_t t = top(sk[last]);
-        // the first position past the run
-        uint32_t end = base + m;
-        for (;; end += kTrBlock * kTrFarLoads) {
-            __syncthreads();
-            if (tid == 0) sm.end = ~0u;
-            __syncthreads();
-            uint32_t past = ~0u;
-#pragma unroll
-            for (int u = kTrFarLoads - 1; u >= 0; --u) {
-                const uint32_t i = end + u * kTrBlock + tid;
-                if (i >= n || top(code.in(keys[i])) != t) past = u * kTrBlock + tid;
-            }
-            if (past != ~0u) atomicMin(&sm.end, past);
-            __syncthreads();
-            if (sm.end != ~0u) break;
-        }
-        end += sm.end;
-        const uint32_t L = end - g0;
-        __syncthreads();
-        if (tid == 0) sm.flag = 0;
-        __syncthreads();
-        bool down = false;
-#pragma unroll 4
-        for (uint32_t i = tid; i + 1 < L; i += kTrBlock)
-            down |= code.ranked(code.in(keys[g0 + i])) > code.ranked(code.in(keys[g0 + i + 1]));
-        if (down) sm.flag = 1;
-        __syncthreads();
-        if (!sm.flag) return;  // the same for the whole workgroup
-        if (L <= kTrCap) {
-            for (uint32_t i = tid; i < L; i += kTrBlock) sk[i] = code.in(keys[g0 + i]);
-            __syncthreads();
-            rank_in_lds(0, L, g0);
-            return;
-        }
-        // digit by digit, kTrBlock * kTrRadixItems keys at a time (items of a
-        // wave are consecutive: ranked by ballot match, stable)
-        auto &wcnt = sm.digit.wcnt;
-        uint32_t *dbase = sm.digit.dbase, *wsum = sm.digit.wsum;
-        uint64_t *ka = keys + g0, *kb = ktmp + g0;
-        UV *va = PAIRS ? vals + g0 : nullptr, *vb = PAIRS ? vtmp + g0 : nullptr;
 #pragma unroll 1
-        for (uint32_t shift = 0; shift < cut; shift += 8) {
+    for (uint32_t q = 0; q < runs + (open ? 1u : 0u); ++q) {
+        uint32_t L, g;
+        if (q < runs) {
+            g = base + (sm.longs[q] & 0xFFFFu);
+            L = base + (sm.longs[q] >> 16) - g;
+            if (L <= kTrRanked) continue;
+        } else {
+            g = base + last;
+            // the first position past the run
+            uint32_t end = base + m;
+            for (;; end += kTrBlock * kTrFarLoads) {
+                __syncthreads();
+                if (tid == 0) sm.end = ~0u;
+                __syncthreads();
+                uint32_t past = ~0u;
+#pragma unroll
+                for (int u = kTrFarLoads - 1; u >= 0; --u) {
+                    const uint32_t i = end + u * kTrBlock + tid;
+                    if (i >= n || top(code.in(keys[i])) != open_top) past = u * kTrBlock + tid;
+                }
+                if (past != ~0u) atomicMin(&sm.end, past);
+                __syncthreads();
+                if (sm.end != ~0u) break;
+            }
+            end += sm.end;
+            L = end - g;
             __syncthreads();
-            dbase[tid] = 0;
             if (tid == 0) sm.flag = 0;
             __syncthreads();
-            for (uint32_t i = tid; i < L; i += kTrBlock) atomicAdd(&dbase[code.digit(code.in(ka[i]), shift)], 1u);
+            bool down = false;
+#pragma unroll 4
+            for (uint32_t i = tid; i + 1 < L; i += kTrBlock)
+                down |= code.ranked(code.in(keys[g + i])) > code.ranked(code.in(keys[g + i + 1]));
+            if (down) sm.flag = 1;
             __syncthreads();
-            const uint32_t c = dbase[tid];
-            if (c == L) sm.flag = 1;
-            uint32_t ex = wave_inclusive_scan(c, SumOp());
-            if (lane == kWave - 1) wsum[wave] = ex;
-            ex -= c;
-            __syncthreads();
-            for (uint32_t w = 0; w < wave; ++w) ex += wsum[w];
-            const bool same = sm.flag != 0;
-            dbase[tid] = ex;
-            if (same) continue;  // one digit for all: nothing moves
-            for (uint32_t s0 = 0; s0 < L; s0 += kTrBlock * kTrRadixItems) {
-                for (uint32_t i = tid; i < kTrWaves * 256u; i += kTrBlock) (&wcnt[0][0])[i] = 0;
-                __syncthreads();
-                uint64_t kk[kTrRadixItems];
-                UV w[kTrRadixItems];
-                uint32_t r[kTrRadixItems], d[kTrRadixItems];
-                const uint32_t p = s0 + wave * (kWave * kTrRadixItems) + lane;
-#pragma unroll
-                for (int u = 0; u < kTrRadixItems; ++u) {
-                    const bool ok = p + u * kWave < L;
-                    kk[u] = ok ? ka[p + u * kWave] : 0;
-                    if constexpr (PAIRS) w[u] = ok ? va[p + u * kWave] : UV(0);
-                    d[u] = code.digit(code.in(kk[u]), shift);
-                    const uint64_t peers = match_any8(d[u]) & ballot(ok);
-                    const uint32_t below = mask_rank(peers);
-                    uint32_t b = 0;
-                    if (ok && below == 0) b = atomicAdd(&wcnt[wave][d[u]], (uint32_t)__builtin_popcountll(peers));
-                    r[u] = (uint32_t)__shfl((int)b, ok ? (int)__builtin_ctzll(peers) : 0) + below;
-                }
-                __syncthreads();
-                uint32_t at = dbase[tid];
-#pragma unroll
-                for (int x = 0; x < kTrWaves; ++x) {
-                    const uint32_t cc = wcnt[x][tid];
-                    wcnt[x][tid] = at;
-                    at += cc;
-                }
-                dbase[tid] = at;
-                __syncthreads();
-#pragma unroll
-                for (int u = 0; u < kTrRadixItems; ++u) {
-                    if (p + u * kWave < L) {
-                        const uint32_t at = wcnt[wave][d[u]] + r[u];
-                        kb[at] = kk[u];
-                        if constexpr (PAIRS) vb[at] = w[u];
-                    }
-                }
-                __syncthreads();
-            }
-            uint64_t *kx = ka;
-            ka = kb;
-            kb = kx;
-            UV *vx = va;
-            va = vb;
-            vb = vx;
+            if (!sm.flag) return;  // the same for the whole workgroup
         }
-        __syncthreads();
-        if (ka != keys + g0) {
-            for (uint32_t i = tid; i < L; i += kTrBlock) {
-                keys[g0 + i] = ka[i];
-                if constexpr (PAIRS) vals[g0 + i] = va[i];
-            }
-        }
+        tr_by_digits<UV, PAIRS>(keys + g, PAIRS ? vals + g : nullptr, ktmp + g, PAIRS ? vtmp + g : nullptr, L, code, cut,
+                                tid, sm);
     }
 }
 

@@ -86,8 +86,9 @@ def runs(n, sizes, digits, rng):
             at += size
 
 
-RUNS = {"pairs": [2, 1, 3], "short": [31, 32, 33, 34, 1], "in LDS": [64, 65, 1, 900, 2], "LDS edge": [2111, 2112, 2113],
-        "chunks": [1023, 4096, 1, 4097], "long": [20_001, 7]}
+RUNS = {"pairs": [2, 1, 3], "short": [31, 32, 33, 34, 1], "ranked": [64, 65, 1, 255, 256, 257, 2],
+        "digits": [256, 257, 300, 900, 1], "LDS edge": [2111, 2112, 2113], "chunks": [1023, 4096, 1, 4097],
+        "long": [20_001, 7]}
 
 
 @pytest.mark.parametrize("layout", RUNS)
