@@ -260,8 +260,11 @@ enum PlanBuf : uint32_t { kBufIn = 0, kBufTmp = 1, kBufOut = 2 };
 // count of digit p's most frequent value).  Keys that tie in every upper
 // digit share its values in each of them, so a run of ties is no longer than the
 // least of those counts, and where the other keys are spread evenly, no longer
-// than what that count has beyond its 256th: at most n / 4096 and the scatter of
-// even counts (8 standard deviations) are taken.  This is exact where the sample
+// than what that count has beyond its 256th: at most n / 2048 and the scatter of
+// even counts (4 standard deviations) are taken, from where on one workgroup may
+// take longer with a run than the passes saved take (u64 -> u32 pairs, one run of
+// n / 1200 keys out of order: 12 * 10^6 545 us, 526 with every digit; of n / 2400 469;
+// of n / 2240, 2^27, 4800 and 5786).  This is exact where the sample
 // is not: half of 2 * 10^6 u64 keys equal and the others uniform, or ten distinct
 // ones, met nothing in the sample, and one workgroup of the repair had the run
 // (2920 and 591 us, 7230 with rare keys beside the frequent one, where passes for
@@ -269,7 +272,7 @@ enum PlanBuf : uint32_t { kBufIn = 0, kBufTmp = 1, kBufOut = 2 };
 // (Lane p of a wave holds most[p], lanes past the digits anything; uniform.)
 __device__ __forceinline__ uint32_t rs_cut_digits(uint32_t low, uint32_t most, uint32_t passes, uint64_t n)
 {
-    const uint64_t even = n / kRadix + n / 4096 + (uint64_t)(sqrtf((float)n) * 0.5f);
+    const uint64_t even = n / kRadix + n / 2048 + (uint64_t)(sqrtf((float)n) * 0.25f);
     const uint64_t spread = ballot(lane_id() < passes && most <= even);
     const uint32_t top = spread ? (uint32_t)(kWave - 1 - __builtin_clzll(spread)) : 0u;  // the highest such digit
     low = low < top ? low : top;
